@@ -115,8 +115,10 @@ struct Level {
   double *dtim = nullptr;
   double *rtrms = nullptr;
   double *force = nullptr;
-  int kc = 0;                   // autotuned k planes per stage workgroup (0: fill rule)
-  int tj = 0;                   // autotuned tile rows of the stage kernels (0: the precision's default)
+  int kc = 0;                   // tuned or forced k planes per stage workgroup (0: tile_pick's)
+  int tj = 0;                   // tuned or forced tile rows of the stage kernels (0: tile_pick's)
+  bool tuned = false;           // kc and tj come from the autotuner (a batch picks its own)
+  int btj = 0, bkc = 0;         // the batch's common choice while the case is recorded into it (0: none)
   void *vprim = nullptr;        // Navier-Stokes: velocity and temperature per cell (4E)
   int nvcell = 0;               // cut cells with wall records (viscous wall terms)
   long *vcell = nullptr;
@@ -642,24 +644,62 @@ StageArgs<T> stage_args(mge_case *h, Level &L, int m, int src, int dst, int w0, 
   return A;
 }
 
-// tile rows of the LDS-tiled stage kernels: the level's autotuned value
-// when set, else the precision's default
-template <class T>
-int stage_tj(const Level &L, int distype) {
-  if (L.tj > 0) return L.tj;
-  return distype != 0 ? RoeTile<T>::TJ : Stage2Tile<T>::TJ;
+// ---- launch shape of the LDS-tiled stage kernels --------------------------
+//
+// A launch of W workgroups of tj x TI threads, kc planes each, runs in about
+//   c0 + (a + b kc) max(1, ceil(W / 256) / s)   microseconds:
+// one workgroup's own time is a chunk start (column loads, first k face) and
+// kc planes, one after another and latency-bound; the fullest of the 256 CUs
+// runs ceil(W / 256) of them, s at the cost of one.  Fitted to timed launches
+// of 30 block shapes from 8 x 8 x 4 to 192^3, every kc = 1, 2, 4, ... nk
+// (residual 7-12%; s < 1 where a second workgroup cannot be resident).  The
+// pick is within 2% of the fastest timed shape on the mean of those blocks
+// and 18% on the worst.  Examples (FP64 JST; before: 8 rows and chunks of at
+// least 4 to 8 planes): 24^3 41 -> 13 us, 48^3 42 -> 22 us, 128 x 128 x 4
+// 31 -> 14 us, 96^3 85 -> 81 us.
+struct TileModel {
+  double c0, a, b, s;
+};
+const TileModel kTileModel[2][2][2] = {  // [FP32][Roe][8 rows]
+    {{{4.8, 3.1, 5.5, 1.46}, {5.0, 4.1, 6.0, 0.89}}, {{5.3, 2.2, 5.9, 1.46}, {4.8, 3.5, 7.3, 0.97}}},
+    {{{6.3, 2.8, 6.5, 2.37}, {5.1, 4.1, 6.2, 1.35}}, {{5.7, 0.9, 5.7, 2.46}, {4.3, 2.2, 5.3, 0.92}}}};
+
+struct TileShape {
+  int tj, kc;
+};
+
+// the cheapest shape by that model for one launch over the blocks ds (one
+// case, or the same level of every case of a batch); tj, kc > 0 are kept
+TileShape tile_pick(const std::vector<const Dims *> &ds, bool fp32, bool roe, int tj, int kc) {
+  int nk = 1;
+  for (const Dims *d : ds) nk = std::max(nk, d->nk);
+  TileShape best{0, 0};
+  double best_us = 0.0;
+  for (int t : {4, 8}) {
+    if (tj > 0 && t != tj) continue;
+    const TileModel &M = kTileModel[fp32 ? 1 : 0][roe ? 1 : 0][t == 8 ? 1 : 0];
+    for (int c = kc > 0 ? std::min(kc, nk) : 1;; c = std::min(2 * c, nk)) {
+      long W = 0;
+      for (const Dims *d : ds)
+        W += (long)((d->ni + TI - 1) / TI) * ((d->nj + t - 1) / t) * ((d->nk + c - 1) / c);
+      const double us = M.c0 + (M.a + M.b * c) * std::max(1.0, (double)((W + 255) / 256) / M.s);
+      if (best.tj == 0 || us < best_us) {
+        best = TileShape{t, c};
+        best_us = us;
+      }
+      if (kc > 0 || c == nk) break;
+    }
+  }
+  return best;
 }
 
-// k planes per workgroup of the LDS-tiled stage kernels: the level's
-// autotuned value when set, else halve from nk while the launch has fewer
-// than 2048 workgroups (enough to fill 256 CUs)
-int stage_kc(const Level &L) {
-  const Dims &d = L.d;
-  if (L.kc > 0) return std::min(L.kc, d.nk);
-  int kc = d.nk;
-  long tiles = (long)((d.ni + TI - 1) / TI) * ((d.nj + TJ - 1) / TJ);
-  while (kc > 8 && tiles * ((d.nk + kc - 1) / kc) < 2048) kc = (kc + 1) / 2;
-  return kc;
+// the stage launch shape of a level: the batch's choice while it is recorded
+// into one (unless the caller forced a shape), else the tuned or forced
+// values, the rest by tile_pick
+TileShape stage_shape(const mge_case *h, const Level &L) {
+  if (h->rec && L.btj > 0) return TileShape{L.btj, std::min(L.bkc, L.d.nk)};
+  if (L.tj > 0 && L.kc > 0) return TileShape{L.tj, std::min(L.kc, L.d.nk)};
+  return tile_pick({&L.d}, h->fp32, h->prm.distype != 0, L.tj, L.kc);
 }
 
 // single-case and batch entry points of the LDS-tiled stage kernel of a
@@ -750,8 +790,8 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       h->next_bytes = per * (double)d.ni * d.nj * d.nk;
     }
     {
-      const int kc = stage_kc(L);
-      const int tj = stage_tj<T>(L, P.distype);  // tile rows of the LDS-tiled kernel
+      const TileShape sh = stage_shape(h, L);
+      const int kc = sh.kc, tj = sh.tj;
       dim3 g((d.ni + TI - 1) / TI, (d.nj + tj - 1) / tj, (d.nk + kc - 1) / kc);
       A.kc = kc;
       if (P.distype != 0 || P.dissip == 0) {
@@ -1192,6 +1232,7 @@ int do_autotune(mge_case *h, Level &L, int *kc_out, double *us_out) {
     if (it != g_tune.end()) {
       L.kc = it->second.kc;
       L.tj = it->second.tj;
+      L.tuned = true;
       if (kc_out) *kc_out = L.kc;
       if (us_out) *us_out = it->second.us;
       return MGE_OK;
@@ -1211,8 +1252,7 @@ int do_autotune(mge_case *h, Level &L, int *kc_out, double *us_out) {
   // timing's spread between runs (isolated repeats of a launch rank the two
   // within a few percent either way)
   constexpr double kOtherMargin = 0.98;
-  L.tj = 0;
-  const int tj_def = stage_tj<T>(L, P.distype);
+  const int tj_def = P.distype != 0 ? RoeTile<T>::TJ : Stage2Tile<T>::TJ;
   int best = 0, best_tj = 0, best_o = 0;
   double best_us = 1e300, best_o_us = 1e300;
   hipError_t err = hipSuccess;
@@ -1256,6 +1296,7 @@ int do_autotune(mge_case *h, Level &L, int *kc_out, double *us_out) {
   CHKRC(check_err(h));
   L.kc = best;
   L.tj = best_tj;
+  L.tuned = true;
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune[key] = {best_tj, best, best_us};
@@ -1656,6 +1697,29 @@ int batch_build(mge_batch *b) {
   if (nc == 0) return MGE_OK;
   std::vector<std::vector<Rec>> R(nc);
   b->cur1.resize(nc);
+  // one stage launch shape per level for all cases: they run in one launch,
+  // whose workgroups fill the chip together, so the shape that is fastest for
+  // each case alone (many small chunks, and other tile rows for some, hence a
+  // second launch) is not the batch's
+  struct ShapeTag {
+    mge_batch *b;
+    ~ShapeTag() {
+      for (int s : b->prog_slots)
+        for (Level &L : b->cs[s]->lv) L.btj = L.bkc = 0;
+    }
+  } stag{b};
+  for (int l = 1; l <= b->nlevel; l++) {
+    std::vector<const Dims *> ds;
+    for (int s : b->prog_slots) ds.push_back(&b->cs[s]->lv[l].d);
+    const TileShape sh = tile_pick(ds, b->fp32 == 1, b->distype != 0, 0, 0);
+    for (int s : b->prog_slots) {
+      Level &L = b->cs[s]->lv[l];
+      if (L.tuned || (L.tj == 0 && L.kc == 0)) {
+        L.btj = sh.tj;
+        L.bkc = sh.kc;
+      }
+    }
+  }
   for (int i = 0; i < nc; i++) {
     mge_case *h = b->cs[b->prog_slots[i]];
     h->rec = &R[i];
@@ -2706,6 +2770,7 @@ int mge_set_kc(mge_case *h, int lvl, int kc) {
   Level *L = get_level(h, lvl);
   if (!L || kc < 0) return set_err(MGE_ERR_ARG, "bad level or kc");
   L->kc = kc;
+  L->tuned = false;
   return MGE_OK;
 }
 
@@ -2719,9 +2784,9 @@ int mge_set_freeze(mge_case *h, int far, int lim) {
 int mge_stage_tile(mge_case *h, int lvl, int *tj, int *kc) {
   Level *L = get_level(h, lvl);
   if (!L || !tj || !kc) return set_err(MGE_ERR_ARG, "bad level or output pointer");
-  const int distype = h->prm.distype;
-  *tj = h->fp32 ? stage_tj<float>(*L, distype) : stage_tj<double>(*L, distype);
-  *kc = stage_kc(*L);
+  const TileShape sh = stage_shape(h, *L);
+  *tj = sh.tj;
+  *kc = sh.kc;
   return MGE_OK;
 }
 
@@ -2730,6 +2795,7 @@ int mge_set_tile(mge_case *h, int lvl, int tj, int kc) {
   if (!L || !(tj == 0 || tj == 4 || tj == 8) || kc < 0) return set_err(MGE_ERR_ARG, "bad level, tile rows or kc");
   L->tj = tj;
   L->kc = kc;
+  L->tuned = false;
   return MGE_OK;
 }
 

@@ -338,12 +338,13 @@ __device__ __attribute__((always_inline)) inline void roe_wall_rec(const FluxCtx
 // converted to primitive variables in LDS; every i and j face of the tile
 // is evaluated once (each cell its low face, plus the faces at the tile's
 // high edges) into LDS; k faces are carried from plane to plane in
-// registers with the primitives of the cell column k-1..k+2.  By default
-// FP64 uses an 8-row tile (512 threads, 121 KB LDS, one workgroup per CU:
+// registers with the primitives of the cell column k-1..k+2.  On large levels
+// FP64 runs fastest with an 8-row tile (512 threads, 121 KB LDS, one workgroup per CU:
 // the two waves per SIMD its registers allow anyway, with half the halo per
 // cell) and FP32 4 rows (four waves per SIMD fit its registers only at 256
-// threads per workgroup); both row counts are built for both precisions and
-// the autotuner may pick the other one per level shape.
+// threads per workgroup); small levels take 4 rows, whose workgroup is done
+// sooner.  Both row counts are built for both precisions and picked per level
+// shape (tile_pick, or the autotuner).
 template <typename T>
 struct RoeTile {
   static constexpr int TJ = kDelta<T> ? 4 : 8;

@@ -282,11 +282,11 @@ MGE_ENTRY_T(k_stage, StageArgs, 256, 1)
 // reference, so results equal k_stage's bit for bit.
 constexpr int TI = 64, TJ = 4;
 
-// rows of the JST tile by default: FP64 uses 8 (512 threads, about 100 KB
+// rows of the JST tile on large levels: FP64 uses 8 (512 threads, about 100 KB
 // LDS, one workgroup per CU -- the two waves per SIMD its registers allow
 // anyway, with half the y-halo work per cell); FP32 keeps 4 rows.  Both row
-// counts (4 and 8) are built for both precisions; the autotuner may pick the
-// other one per level shape.
+// counts (4 and 8) are built for both precisions and picked per level shape
+// (tile_pick, or the autotuner).
 template <typename T>
 struct Stage2Tile {
   static constexpr int TJ = kDelta<T> ? 4 : 8;

@@ -216,8 +216,8 @@ class Case:
         return tj.value, kc.value
 
     def set_tile(self, lvl, tj, kc=0):
-        """force the stage kernel's tile rows (4 or 8; 0: the precision's
-        default) and k-chunk length (0: the fill rule) of level lvl"""
+        """force the stage kernel's tile rows (4 or 8; 0: the library's pick)
+        and k-chunk length (0: the library's pick) of level lvl"""
         _ffi.check(self.lib.mge_set_tile(self.h, lvl, tj, kc), "mge_set_tile")
 
     def sync(self):

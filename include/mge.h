@@ -306,13 +306,15 @@ int mge_kernel_timing(mge_case *h, int enable, const char *name, double *ms, lon
  * (256 or 512 threads per workgroup) and every k-chunk length kc = 1, 2,
  * 4, ... nk, and keeps the fastest pair for the level; results are cached
  * per (shape, precision, scheme) for the process.  The launch shape changes
- * no arithmetic.  Overwrites only scratch state (a non-current state
+ * no arithmetic.  An untuned level takes the shape a cost model picks, and a
+ * batch picks one shape per level for all its cases whether tuned or not
+ * (a shape forced with mge_set_tile or mge_set_kc stays).  Overwrites only scratch state (a non-current state
  * buffer, dw, fw, the time-step arrays); call it between solves, not while
  * a batch is recording.  *kc (0 for the matrix-dissipation kernel, which has
  * no chunks) and *us (best launch time, microseconds) may be NULL; the
  * chosen tile rows are read with mge_stage_tile. */
 int mge_autotune(mge_case *h, int lvl, int *kc, double *us);
-/* force the k-chunk length of level lvl (0: the built-in fill rule) */
+/* force the k-chunk length of level lvl (0: the library's pick) */
 int mge_set_kc(mge_case *h, int lvl, int kc);
 /* set the case's freeze flags directly: far-field branches (ffreeze) and
  * limiter choices (lfreeze); each flag is otherwise set by the case's own
@@ -322,8 +324,8 @@ int mge_set_freeze(mge_case *h, int far, int lim);
 /* the tile rows and k-chunk length the stage kernel of level lvl launches
  * with (no counterpart in the reference) */
 int mge_stage_tile(mge_case *h, int lvl, int *tj, int *kc);
-/* force the tile rows (4 or 8; 0: the precision's default) and k-chunk
- * length (0: the fill rule) of level lvl (no counterpart in the reference) */
+/* force the tile rows (4 or 8; 0: the library's pick) and k-chunk length
+ * (0: the library's pick) of level lvl (no counterpart in the reference) */
 int mge_set_tile(mge_case *h, int lvl, int tj, int kc);
 /* ---- embedded multi-block hierarchies (composite grids) ----------------
  * Several blocks per multigrid level, each finer level covering part of the
