@@ -1136,7 +1136,7 @@ __global__ void k_wall_terms(FluxCtx<T> fc, const DevRec *recs, const double *ws
   if (roe) {
     double ws5[5], ve[5], vd[5];
     for (int n = 0; n < 5; n++) ws5[n] = wsol[n * nmir + m];
-    roe_wall_rec(fc, r, ws5, psol[m], gamma, eps, 1.0, ve, vd, err);
+    roe_wall_rec(fc, r, r.faceid >= 4, ws5, psol[m], gamma, eps, 1.0, ve, vd, err);
     for (int dd = 0; dd < 3; dd++) terms[3 * m + dd] = ve[1 + dd] + vd[1 + dd];
     return;
   }

@@ -102,11 +102,10 @@ struct Level {
   DevRec *recs = nullptr;
   double *wsol = nullptr, *psol = nullptr;
   std::vector<mge_cutrec> hrecs;
-  int ntouch = 0, nops = 0;
   long *tcell = nullptr;
   int *beg = nullptr;
-  int2 *ops = nullptr;
-  int2 *chunks = nullptr;  // k_rec's workgroups (touched-cell ranges)
+  RecOp *ops = nullptr;
+  int4 *chunks = nullptr;  // k_rec's workgroups (touched cells and ops)
   int nchunk = 0;
   double *opval = nullptr;
   double *partial = nullptr;
@@ -806,7 +805,6 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       RecArgs<T> R;
       R.st = A;
       R.st.store_fw = 1;
-      R.recs = L.recs;
       R.wsol = L.wsol;
       R.psol = L.psol;
       R.nmir = L.nmir;
@@ -814,8 +812,6 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       R.beg = L.beg;
       R.ops = L.ops;
       R.chunks = L.chunks;
-      R.ntouch = L.ntouch;
-      R.nops = L.nops;
       R.err = h->err;
       LAUNCHT(h, "k_rec", k_rec, T, dim3((unsigned)L.nchunk), dim3(kRecOps), R);
     }
@@ -1407,24 +1403,38 @@ int build_records(mge_case *h, Level &L, int nmir, const mge_cutrec *recs) {
   }
   std::vector<long> tcell;
   std::vector<int> begv(1, 0);
-  std::vector<int2> opv;
+  std::vector<RecOp> opv;
+  auto add_op = [&](const int2 &o) {
+    const DevRec &r = dr[o.x];
+    RecOp p{};
+    p.rec = o.x;
+    p.kind = (uint8_t)o.y;
+    p.zz = (uint8_t)r.zz;
+    p.hi = r.faceid >= 4;
+    for (int a = 0; a < 3; a++) {
+      p.c[a] = r.c[a];
+      p.s[a] = r.s[a];
+    }
+    p.qc = ix(d, r.c[0], r.c[1], r.c[2]);
+    opv.push_back(p);
+  };
   for (auto &kv : per) {
     tcell.push_back(kv.first);
-    for (auto &o : kv.second.first) opv.push_back(o);
-    for (auto &o : kv.second.second) opv.push_back(o);
+    for (auto &o : kv.second.first) add_op(o);
+    for (auto &o : kv.second.second) add_op(o);
     begv.push_back((int)opv.size());
   }
-  L.ntouch = (int)tcell.size();
-  L.nops = (int)opv.size();
+  const int ntouch = (int)tcell.size();
   // workgroups of k_rec: consecutive touched cells with at most kRecOps ops
-  std::vector<int2> chunks;
-  for (int t = 0, t0 = 0; t < L.ntouch; t++) {
+  std::vector<int4> chunks;
+  auto add_chunk = [&](int t0, int t1) { chunks.push_back(make_int4(t0, t1, begv[t0], begv[t1])); };
+  for (int t = 0, t0 = 0; t < ntouch; t++) {
     if (begv[t + 1] - begv[t] > kRecOps) return set_err(MGE_ERR_ARG, "too many wall ops on one cell");
     if (begv[t + 1] - begv[t0] > kRecOps) {
-      chunks.push_back(make_int2(t0, t));
+      add_chunk(t0, t);
       t0 = t;
     }
-    if (t == L.ntouch - 1) chunks.push_back(make_int2(t0, L.ntouch));
+    if (t == ntouch - 1) add_chunk(t0, ntouch);
   }
   L.nchunk = (int)chunks.size();
   CHKRC(dalloc(L, &L.recs, nmir));
@@ -1471,8 +1481,8 @@ int build_records(mge_case *h, Level &L, int nmir, const mge_cutrec *recs) {
   }
   HIPCHK(h2d_sync(L.tcell, tcell.data(), sizeof(long) * tcell.size(), h->stream));
   HIPCHK(h2d_sync(L.beg, begv.data(), sizeof(int) * begv.size()));
-  if (!opv.empty()) HIPCHK(h2d_sync(L.ops, opv.data(), sizeof(int2) * opv.size()));
-  if (!chunks.empty()) HIPCHK(h2d_sync(L.chunks, chunks.data(), sizeof(int2) * chunks.size()));
+  if (!opv.empty()) HIPCHK(h2d_sync(L.ops, opv.data(), sizeof(RecOp) * opv.size()));
+  if (!chunks.empty()) HIPCHK(h2d_sync(L.chunks, chunks.data(), sizeof(int4) * chunks.size()));
   std::vector<uint8_t> fl(d.E);
   HIPCHK(d2h_sync(fl.data(), L.flags, d.E, h->stream));
   for (long q : tcell) fl[q] |= F_TOUCHED;

@@ -292,14 +292,14 @@ __device__ inline void roe_face_vec(double gamma, double eps, double cdis, const
   for (int n = 0; n < 5; n++) d[n] = cdis * (0.5 * dd[n]);
 }
 
-// wall face of record r: the signed contributions (ve, vd) to the cut cell,
-// in FP64 from the bulk state and the mirror state
-template <typename T>
-__device__ __attribute__((always_inline)) inline void roe_wall_rec(const FluxCtx<T> &c, const DevRec &r, const double *wsol, double psol, double gamma,
+// wall face of record r (a DevRec or RecOp; hi: its cut cell's high face):
+// the signed contributions (ve, vd) to the cut cell, in FP64 from the bulk
+// state and the mirror state
+template <typename T, class R>
+__device__ __attribute__((always_inline)) inline void roe_wall_rec(const FluxCtx<T> &c, const R &r, bool hi, const double *wsol, double psol, double gamma,
                              double eps, double cdis, double *ve, double *vd, int *err) {
   const Dims &d = c.d;
   int zz = r.zz;
-  bool hi = r.faceid >= 4;
   long qc = ix(d, r.c[0], r.c[1], r.c[2]);
   if (fabs(full(c.inf, 0, c.s.w[qc])) < (double)1.0e-8f) raise_err(err, MGE_ERR_WALL_RHO);
   int fi = r.c[0], fj = r.c[1], fk = r.c[2];

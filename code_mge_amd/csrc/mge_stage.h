@@ -84,18 +84,26 @@ struct StageArgs {
 };
 
 
+// one op of a touched cell: the record's fields that its value needs, copied
+// by the host so that one load, not a chain through the record, precedes the
+// op's stencil loads
+struct alignas(16) RecOp {
+  int rec;                  // record (mirror state)
+  uint8_t kind, zz, hi, pad;
+  int c[3], s[3];           // cut cell, solid cell
+  long qc;                  // cell index of the cut cell
+};
+
 template <typename T>
 struct RecArgs {
   StageArgs<T> st;
-  const DevRec *recs;
   const double *wsol;       // 5*nmir, component-major
   const double *psol;
   int nmir;
   const long *tcell;        // touched cells
   const int *beg;           // op range of each touched cell (ntouch+1)
-  const int2 *ops;          // (record, kind), fw ops then dw ops per cell
-  const int2 *chunks;       // touched cells [x, y) of each workgroup, at most kRecOps ops
-  int ntouch, nops;
+  const RecOp *ops;         // fw ops then dw ops per cell
+  const int4 *chunks;       // touched cells [x, y) of each workgroup and their ops [z, w), at most kRecOps
   int *err;
 };
 
@@ -104,8 +112,8 @@ struct RecArgs {
 constexpr int kRecOps = 64;
 
 // the Roe wall-face term of a record (defined with the Roe scheme)
-template <typename T>
-__device__ __attribute__((always_inline)) inline void roe_wall_rec(const FluxCtx<T> &c, const DevRec &r, const double *wsol, double psol, double gamma,
+template <typename T, class R>
+__device__ __attribute__((always_inline)) inline void roe_wall_rec(const FluxCtx<T> &c, const R &r, bool hi, const double *wsol, double psol, double gamma,
                              double eps, double cdis, double *ve, double *vd, int *err);
 
 // ------------------------------------------------------------------ finish of a cell
@@ -113,14 +121,15 @@ __device__ __attribute__((always_inline)) inline void roe_wall_rec(const FluxCtx
 // dw = dw + fw, forcing, blanking, time-step scaling and (unsmoothed) the
 // update with the EOS (euler.f90:217-223, 294-342, 363-399).  With PRE the
 // caller has already loaded the cell's W(0) (wnp), local time step (vdt) and
-// flags (fl), so that their latency overlapped its face evaluation.  GEN
+// flags (fl), so that their latency overlapped its face evaluation (and with
+// qfp the forcing of a coarse level).  GEN
 // false is the form for a launch that is not on a coarse level, not
 // unsteady, not on a stretched level and uses the local time step (the
 // host picks it only then): those branches and their pointers drop out, which
 // frees the scalar registers they held in the stage kernels' plane loops.
 template <typename T, bool PRE = false, bool GEN = true>
 __device__ inline void finish_cell(const StageArgs<T> &A, long q, const T *f, const T *e, const T *wnp = nullptr,
-                                   T vdt = T(0), uint8_t fl = 0) {
+                                   T vdt = T(0), uint8_t fl = 0, const T *qfp = nullptr) {
   const long E = A.fx.d.E;
   T r[5];
 #pragma unroll
@@ -147,7 +156,7 @@ __device__ inline void finish_cell(const StageArgs<T> &A, long q, const T *f, co
         if (A.marker[q] == 1) qv = T(1) * A.wr[n * E + q] - r[n];
         A.qf[n * E + q] = qv;
       } else {
-        qv = A.qf[n * E + q];
+        qv = qfp ? qfp[n] : A.qf[n * E + q];
       }
       r[n] = r[n] + qv;
     }
@@ -779,29 +788,6 @@ __global__ void __launch_bounds__(TI * TJ_, Stage2Tile<T>::MINW)
 
 // ------------------------------------------------------------------ wall records
 
-template <int DIR, typename T>
-__device__ inline void rec_dfs(const FluxCtx<T> &c, int i, int j, int k, int a, T *o) {
-  long base = DIR == 0 ? ix(c.d, 0, j, k) : (DIR == 1 ? ix(c.d, i, 0, k) : ix(c.d, i, j, 0));
-  dface<DIR>(c, base, a, i, j, k, o);
-}
-template <typename T>
-__device__ inline void rec_dfs_any(const FluxCtx<T> &c, int zz, int i, int j, int k, int a, T *o) {
-  if (zz == 1) rec_dfs<0>(c, i, j, k, a, o);
-  else if (zz == 2) rec_dfs<1>(c, i, j, k, a, o);
-  else rec_dfs<2>(c, i, j, k, a, o);
-}
-template <int DIR, typename T>
-__device__ inline void rec_efs(const FluxCtx<T> &c, int i, int j, int k, int a, T *o) {
-  long base = DIR == 0 ? ix(c.d, 0, j, k) : (DIR == 1 ? ix(c.d, i, 0, k) : ix(c.d, i, j, 0));
-  eface<DIR>(c, base, a, i, j, k, o);
-}
-template <typename T>
-__device__ inline void rec_efs_any(const FluxCtx<T> &c, int zz, int i, int j, int k, int a, T *o) {
-  if (zz == 1) rec_efs<0>(c, i, j, k, a, o);
-  else if (zz == 2) rec_efs<1>(c, i, j, k, a, o);
-  else rec_efs<2>(c, i, j, k, a, o);
-}
-
 // face_s<zz-1> for a runtime zz: the three vertex differences are loaded
 // and the product selected (branches on zz that each load through a
 // different pointer of g are merged into one load through a selected field
@@ -822,281 +808,298 @@ __device__ inline void axis_vec(double *v, int zz, double s) {
   v[2] = zz == 3 ? s : 0.0;
 }
 
-// the two recomputed faces of dfluxb.f90 for record r: fs1 (inner face of
-// the pair) and fs2 (the wall face or the face behind it).  They involve the
-// FP64 mirror state, so they are evaluated in FP64 from the bulk values.
+// The line of cells along zz that a JST wall op reads, around a centre s0 + off:
+// p at -3..3 (index 3 is the centre), w at -2..2 (index 2), radius sums at
+// -1..1.  Every value is loaded before any is used, so an op waits for one
+// round trip; the ops of a wave differ only in arithmetic.
 template <typename T>
-__device__ __attribute__((always_inline)) inline void dfluxb_rec(const FluxCtx<T> &c, const DevRec &r, const double *wsolv, double psol, double *fs1,
-                           double *fs2) {
+struct RecLine {
+  T p[7], w[5][5], rd[3];
+  int a, ne;   // line index of the centre, last face of the line
+};
+template <typename T>
+__device__ inline RecLine<T> rec_line(const FluxCtx<T> &c, const RecOp &r, int off) {
   const Dims &d = c.d;
-  const long E = d.E;
-  int zz = r.zz, id = r.faceid;
-  int i = r.c[0], j = r.c[1], k = r.c[2];
-  int s0 = zz == 1 ? i : (zz == 2 ? j : k);
-  long st = zz == 1 ? 1L : (zz == 2 ? d.sy : d.sz);
-  long base = ix(d, i, j, k) - (long)s0 * st;
-  // a sum of the three values rather than a select between the fields (see
-  // face_s_any)
-  const int nbmax = (zz == 1) * d.ib + (zz == 2) * d.jb + (zz == 3) * d.kb;
-  const double vis2 = c.vis2, vis4 = c.vis4, cdis = c.cdis;
-  double wsol[5];
-  for (int n = 0; n < 5; n++) wsol[n] = wsolv[n];
-  wsol[4] = wsol[4] + psol;
-  auto P = [&](int s) { return full(c.inf, 5, c.s.p[base + (long)s * st]); };
-  auto H = [&](int s, int n) {
-    long q = base + (long)s * st;
-    return n < 4 ? full(c.inf, n, c.s.w[n * E + q]) : full(c.inf, 4, c.s.w[4 * E + q]) + full(c.inf, 5, c.s.p[q]);
-  };
-  auto RS = [&](int s) { return (double)c.radsum[base + (long)s * st]; };
-  auto SS = [&](int s, double *ss) {
-    int fi = zz == 1 ? s : i, fj = zz == 2 ? s : j, fk = zz == 3 ? s : k;
-    axis_vec(ss, zz, (double)face_s_any(c.g, zz, fi, fj, fk));
-  };
-  double fp[3], ep, lm, lp, lam, dis2, dis4, diw[3][5];
-  int hi = (id >= 4);
-  int s = s0;
-  if (hi) {
-    if (zz == 1) {
-      fp[0] = fabs(P(s - 2) - 2.0 * P(s - 1) + P(s)) / fabs(P(s - 2) + 2.0 * P(s - 1) + P(s));
-      fp[1] = fabs(P(s - 1) - 2.0 * P(s) + psol) / fabs(P(s - 1) + 2.0 * P(s) + psol);
-    } else {
-      fp[0] = fabs(P(s) - 2.0 * P(s - 1) + P(s - 2)) / fabs(P(s) + 2.0 * P(s - 1) + P(s - 2));
-      fp[1] = fabs(psol - 2.0 * P(s) + P(s - 1)) / fabs(psol + 2.0 * P(s) + P(s - 1));
+  RecLine<T> L;
+  const long st = r.zz == 1 ? 1L : (r.zz == 2 ? d.sy : d.sz);
+  // sums of products rather than selects between fields (see face_s_any)
+  const int nl = (r.zz == 1) * d.il + (r.zz == 2) * d.jl + (r.zz == 3) * d.kl;
+  const int a = (r.zz == 1 ? r.c[0] : (r.zz == 2 ? r.c[1] : r.c[2])) + off;
+  const long q = r.qc + (long)off * st;
+  L.a = a;
+  L.ne = nl + 1;
+#pragma unroll
+  for (int t = -3; t <= 3; t++) {
+    const int s = min(max(a + t, 0), nl + 2);   // the outermost, past the array, enter only a switch that is 0
+    L.p[t + 3] = c.s.p[q + (long)(s - a) * st];
+  }
+#pragma unroll
+  for (int t = -2; t <= 2; t++)
+#pragma unroll
+    for (int n = 0; n < 5; n++) L.w[t + 2][n] = c.s.w[n * d.E + q + (long)t * st];
+#pragma unroll
+  for (int t = -1; t <= 1; t++) {
+    const int s = min(max(a + t, 2), nl);   // rad_at's line-end copies
+    L.rd[t + 1] = c.radsum[q + (long)(s - a) * st];
+  }
+  return L;
+}
+
+// dface's value at the line's face a + F (F = 0, 1), the bulk kernel's
+// expressions on the loaded line (S the face's vector component)
+template <int F, typename T>
+__device__ inline void rec_face(const FluxCtx<T> &c, const RecLine<T> &L, int zz, T S, T *out) {
+  const int a = L.a + F, nb = L.ne + 1;
+  T f[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {   // switch at a - 2 + t from p at its own place and its neighbours'
+    const T lo = L.p[F + t], up = L.p[F + t + 2];
+    const T v = fp_val<0>(c.inf, zz == 2 ? up : lo, L.p[F + t + 1], zz == 2 ? lo : up);
+    const int s = a - 2 + t;
+    f[t] = (s <= 0 || s >= nb) ? T(0) : v;
+  }
+  const T ep = maxd(maxd(maxd(f[0], f[1]), f[2]), f[3]);
+  const T lam = T(0.5) * (L.rd[F] + L.rd[F + 1]);
+  T dis2 = c.vis2 * ep, dis4 = dimd(c.vis4, dis2);
+  dis2 = dis2 * c.cdis;
+  dis4 = dis4 * c.cdis;
+  T dd[5];
+#pragma unroll
+  for (int n = 0; n < 5; n++) {
+    T q[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {   // a-2 .. a+1
+      q[t] = L.w[min(F + t, 4)][n];
+      if (n == 4) q[t] = q[t] + L.p[min(F + t, 4) + 1];
     }
-    ep = maxd(fp[0], fp[1]);
-    lm = RS(s);
-    lam = lm;
-    dis2 = vis2 * ep; dis4 = vis4; dis4 = dimd(dis4, dis2);
-    dis2 = dis2 * cdis; dis4 = dis4 * cdis;
-    for (int n = 0; n < 5; n++) {
-      diw[0][n] = H(s, n) - H(s - 1, n);
-      diw[1][n] = wsol[n] - H(s, n);
-      diw[2][n] = diw[1][n];
-      fs2[n] = diw[2][n] - 2.0 * diw[1][n] + diw[0][n];
-      fs2[n] = dis2 * diw[1][n] - dis4 * fs2[n];
-    }
-    if (c.dissip == 0) {
-      for (int n = 0; n < 5; n++) fs2[n] = fs2[n] * lam;
-    } else {
-      double uc[5], ss[3], o[5];
-      for (int n = 0; n < 5; n++) uc[n] = H(s, n);
-      SS(s + 1, ss);
-      dmatrix((double)c.gamma, uc, wsol, fs2, ss, o);
-      for (int n = 0; n < 5; n++) fs2[n] = o[n];
-    }
-    if ((s - 3) >= 0)
-      fp[2] = fabs(P(s - 1) - 2.0 * P(s - 2) + P(s - 3)) / fabs(P(s - 1) + 2.0 * P(s - 2) + P(s - 3));
-    else
-      fp[2] = 0.0;
-    ep = maxd(maxd(fp[0], fp[1]), fp[2]);
-    lm = RS(s - 1);
-    lp = RS(s);
-    lam = 0.5 * (lm + lp);
-    dis2 = vis2 * ep; dis4 = vis4; dis4 = dimd(dis4, dis2);
-    dis2 = dis2 * cdis; dis4 = dis4 * cdis;
-    for (int n = 0; n < 5; n++) {
-      diw[0][n] = H(s - 1, n) - H(s - 2, n);
-      diw[1][n] = H(s, n) - H(s - 1, n);
-      diw[2][n] = wsol[n] - H(s, n);
-      fs1[n] = diw[2][n] - 2.0 * diw[1][n] + diw[0][n];
-      fs1[n] = dis2 * diw[1][n] - dis4 * fs1[n];
-    }
-    if (c.dissip == 0) {
-      for (int n = 0; n < 5; n++) fs1[n] = fs1[n] * lam;
-    } else {
-      double um[5], uc[5], ss[3], o[5];
-      for (int n = 0; n < 5; n++) { um[n] = H(s - 1, n); uc[n] = H(s, n); }
-      SS(s, ss);
-      dmatrix((double)c.gamma, um, uc, fs1, ss, o);
-      for (int n = 0; n < 5; n++) fs1[n] = o[n];
-    }
+    const T da = q[2] - q[1];
+    const T dm = a == 2 ? da : q[1] - q[0], dp = a == L.ne ? da : q[3] - q[2];
+    dd[n] = dis2 * da - dis4 * (dp - T(2) * da + dm);
+  }
+  if (c.dissip == 0) {
+#pragma unroll
+    for (int n = 0; n < 5; n++) out[n] = dd[n] * lam;
   } else {
-    fp[0] = fabs(P(s + 1) - 2.0 * P(s) + psol) / fabs(P(s + 1) + 2.0 * P(s) + psol);
-    fp[1] = fabs(P(s + 2) - 2.0 * P(s + 1) + P(s)) / fabs(P(s + 2) + 2.0 * P(s + 1) + P(s));
-    if ((s + 3) <= nbmax)
-      fp[2] = fabs(P(s + 3) - 2.0 * P(s + 2) + P(s + 1)) / fabs(P(s + 3) + 2.0 * P(s + 2) + P(s + 1));
-    else
-      fp[2] = 0.0;
-    ep = maxd(maxd(fp[0], fp[1]), fp[2]);
-    lm = RS(s);
-    lp = RS(s + 1);
-    lam = 0.5 * (lm + lp);
-    dis2 = vis2 * ep; dis4 = vis4; dis4 = dimd(dis4, dis2);
-    dis2 = dis2 * cdis; dis4 = dis4 * cdis;
+    T um[5], ua[5];
+#pragma unroll
     for (int n = 0; n < 5; n++) {
-      diw[0][n] = H(s, n) - wsol[n];
-      diw[1][n] = H(s + 1, n) - H(s, n);
-      diw[2][n] = H(s + 2, n) - H(s + 1, n);
-      fs2[n] = diw[2][n] - 2.0 * diw[1][n] + diw[0][n];
-      fs2[n] = dis2 * diw[1][n] - dis4 * fs2[n];
+      um[n] = L.w[F + 1][n];
+      ua[n] = L.w[F + 2][n];
+      if constexpr (kDelta<T>) {
+        um[n] = um[n] + c.inf.w[n];
+        ua[n] = ua[n] + c.inf.w[n];
+      }
     }
-    if (c.dissip == 0) {
-      for (int n = 0; n < 5; n++) fs2[n] = fs2[n] * lam;
-    } else {
-      double uc[5], up[5], ss[3], o[5];
-      for (int n = 0; n < 5; n++) { uc[n] = H(s, n); up[n] = H(s + 1, n); }
-      SS(s + 1, ss);
-      dmatrix((double)c.gamma, uc, up, fs2, ss, o);
-      for (int n = 0; n < 5; n++) fs2[n] = o[n];
+    T pm = L.p[F + 2], pa = L.p[F + 3];
+    if constexpr (kDelta<T>) {
+      pm = pm + c.inf.p;
+      pa = pa + c.inf.p;
     }
-    ep = maxd(fp[0], fp[1]);
-    lp = RS(s);
-    lam = lp;
-    dis2 = vis2 * ep; dis4 = vis4; dis4 = dimd(dis4, dis2);
-    dis2 = dis2 * cdis; dis4 = dis4 * cdis;
-    for (int n = 0; n < 5; n++) {
-      diw[1][n] = H(s, n) - wsol[n];
-      diw[0][n] = diw[1][n];
-      diw[2][n] = H(s + 1, n) - H(s, n);
-      fs1[n] = diw[2][n] - 2.0 * diw[1][n] + diw[0][n];
-      fs1[n] = dis2 * diw[1][n] - dis4 * fs1[n];
-    }
-    if (c.dissip == 0) {
-      for (int n = 0; n < 5; n++) fs1[n] = fs1[n] * lam;
-    } else {
-      double uc[5], ss[3], o[5];
-      for (int n = 0; n < 5; n++) uc[n] = H(s, n);
-      SS(s, ss);
-      dmatrix((double)c.gamma, wsol, uc, fs1, ss, o);
-      for (int n = 0; n < 5; n++) fs1[n] = o[n];
-    }
+    um[4] = um[4] + pm;
+    ua[4] = ua[4] + pa;
+    const T ss[3] = {zz == 1 ? S : T(0), zz == 2 ? S : T(0), zz == 3 ? S : T(0)};
+    dmatrix(c.gamma, um, ua, dd, ss, out);
   }
 }
 
-// the wall flux fs and the opposite-face flux fa of efluxb.f90:50-80,
-// in FP64 like dfluxb_rec
+// the two recomputed faces of dfluxb.f90 for a record: `inner`, the face
+// between the cut cell and its inner neighbour, and `wall`, the one to the
+// mirror state.  They involve the FP64 mirror state, so they are evaluated
+// in FP64 from the bulk values.  x0, x1, x2 are the cut cell and the two
+// cells inside it (the line's centre is x1); a high and a low record use the
+// same expressions with the differences' sign turned (the reference's two
+// branches, :41-105 and :106-171).  A record's cut cell lies in 3 .. nl-1, so
+// the three cells inside it exist.
 template <typename T>
-__device__ __attribute__((always_inline)) inline void efluxb_rec(const FluxCtx<T> &c, const DevRec &r, const double *wsol, double psol, double *fs,
-                           double *fa, int *err) {
-  const Dims &d = c.d;
-  int zz = r.zz, id = r.faceid;
-  int i = r.c[0], j = r.c[1], k = r.c[2];
-  long qc = ix(d, i, j, k);
-  double sc[3], ss[3];
-  axis_vec(sc, zz, (double)face_s_any(c.g, zz, i, j, k));
-  axis_vec(ss, zz, (double)face_s_any(c.g, zz, r.s[0], r.s[1], r.s[2]));
-  double wc[5];
-  for (int n = 0; n < 5; n++) wc[n] = full(c.inf, n, c.s.w[n * d.E + qc]);
-  if (fabs(wc[0]) < (double)1.0e-8f) raise_err(err, MGE_ERR_WALL_RHO);
-  double fs1[5], fs2[5], fs3[5];
-  cflux3(wc, full(c.inf, 5, c.s.p[qc]), sc, fs1);
-  cflux3(wsol, psol, ss, fs2);
-  for (int n = 0; n < 5; n++) fs[n] = 0.5 * (fs1[n] + fs2[n]);
-  int hi = (id >= 4);
-  int oi = i, oj = j, ok = k;
-  int dlt = hi ? -1 : 1;
-  if (zz == 1) oi += dlt;
-  else if (zz == 2) oj += dlt;
-  else ok += dlt;
-  long qo = ix(d, oi, oj, ok);
-  double wo[5], so[3];
-  for (int n = 0; n < 5; n++) wo[n] = full(c.inf, n, c.s.w[n * d.E + qo]);
-  axis_vec(so, zz, (double)face_s_any(c.g, zz, oi, oj, ok));
-  cflux3(wo, full(c.inf, 5, c.s.p[qo]), so, fs3);
-  for (int n = 0; n < 5; n++) fa[n] = 0.5 * (fs1[n] + fs3[n]);
+__device__ inline void rec_wall_faces(const FluxCtx<T> &c, const RecLine<T> &L, int zz, bool hi, double S,
+                                      const double *wsolv, double psol, double *inner, double *wall) {
+  const double vis2 = c.vis2, vis4 = c.vis4, cdis = c.cdis;
+  double ws[5], x[3][5], P[4];
+#pragma unroll
+  for (int n = 0; n < 5; n++) ws[n] = wsolv[n];
+  ws[4] = ws[4] + psol;
+#pragma unroll
+  for (int t = 0; t < 4; t++) P[t] = full(c.inf, 5, hi ? L.p[4 - t] : L.p[2 + t]);
+#pragma unroll
+  for (int t = 0; t < 3; t++)
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+      x[t][n] = full(c.inf, n, hi ? L.w[3 - t][n] : L.w[1 + t][n]);
+      if (n == 4) x[t][n] = x[t][n] + P[t];
+    }
+  const double r0 = hi ? L.rd[2] : L.rd[0], r1 = L.rd[1];
+  const double f0 = fabs(P[1] - 2.0 * P[0] + psol) / fabs(P[1] + 2.0 * P[0] + psol);
+  const double f1 = fabs(P[2] - 2.0 * P[1] + P[0]) / fabs(P[2] + 2.0 * P[1] + P[0]);
+  const double f2 = fabs(P[3] - 2.0 * P[2] + P[1]) / fabs(P[3] + 2.0 * P[2] + P[1]);
+  const double sg = hi ? 1.0 : -1.0;
+  const double epw = maxd(f0, f1), epi = maxd(epw, f2);
+  const double lamw = r0, lami = 0.5 * (r1 + r0);
+  const double w2 = vis2 * epw, w4 = dimd(vis4, w2), i2 = vis2 * epi, i4 = dimd(vis4, i2);
+  double dw[5], di[5];
+#pragma unroll
+  for (int n = 0; n < 5; n++) {
+    const double e0 = ws[n] - x[0][n], e1 = x[0][n] - x[1][n], e2 = x[1][n] - x[2][n];
+    dw[n] = sg * ((w2 * cdis) * e0 - (w4 * cdis) * (e0 - 2.0 * e0 + e1));
+    di[n] = sg * ((i2 * cdis) * e1 - (i4 * cdis) * (e0 - 2.0 * e1 + e2));
+  }
+  if (c.dissip == 0) {
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+      wall[n] = dw[n] * lamw;
+      inner[n] = di[n] * lami;
+    }
+  } else {
+    double ss[3], u1[5], u2[5];
+    axis_vec(ss, zz, S);
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+      u1[n] = hi ? x[0][n] : ws[n];
+      u2[n] = hi ? ws[n] : x[0][n];
+    }
+    dmatrix((double)c.gamma, u1, u2, dw, ss, wall);
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+      u1[n] = hi ? x[1][n] : x[0][n];
+      u2[n] = hi ? x[0][n] : x[1][n];
+    }
+    dmatrix((double)c.gamma, u1, u2, di, ss, inner);
+  }
 }
 
-// the value op o contributes (dfluxb.f90 / efluxb.f90 terms); the undo
-// terms repeat the bulk kernel's face values in T
+// cflux_st for a runtime direction (the component picked by selects)
 template <typename T>
-__device__ __attribute__((always_inline)) inline void rec_op_value(const RecArgs<T> &R, int o, double *out) {
-  const StageArgs<T> &A = R.st;
-  int2 op = R.ops[o];
-  const DevRec &r = R.recs[op.x];
-  if (op.y < OP_E_UNDO && !A.has_diss) return;
-  int zz = r.zz;
-  int s0 = zz == 1 ? r.c[0] : (zz == 2 ? r.c[1] : r.c[2]);
-  double ws[5];
-  for (int n = 0; n < 5; n++) ws[n] = R.wsol[n * R.nmir + op.x];
-  double ps = R.psol[op.x];
+__device__ inline void rec_flux(const FluxCtx<T> &c, int zz, const T *v, T p, T S, T *fs) {
   T a[5], b[5];
-  double fs1[5], fs2[5];
-  int ci = r.c[0], cj = r.c[1], ck = r.c[2];
-  switch (op.y) {
-    case OP_HI_C_UNDO:
-    case OP_LO_C_UNDO:
-      rec_dfs_any(A.fx, zz, ci, cj, ck, s0, a);
-      rec_dfs_any(A.fx, zz, ci, cj, ck, s0 + 1, b);
-      for (int n = 0; n < 5; n++) out[n] = a[n] - b[n];
-      break;
-    case OP_HI_N_UNDO:
-      rec_dfs_any(A.fx, zz, ci, cj, ck, s0 - 1, a);
-      rec_dfs_any(A.fx, zz, ci, cj, ck, s0, b);
-      for (int n = 0; n < 5; n++) out[n] = a[n] - b[n];
-      break;
-    case OP_LO_N_UNDO:
-      rec_dfs_any(A.fx, zz, ci, cj, ck, s0 + 1, a);
-      rec_dfs_any(A.fx, zz, ci, cj, ck, s0 + 2, b);
-      for (int n = 0; n < 5; n++) out[n] = a[n] - b[n];
-      break;
-    case OP_HI_C_ADD:
-    case OP_LO_C_ADD:
-      dfluxb_rec(A.fx, r, ws, ps, fs1, fs2);
-      for (int n = 0; n < 5; n++) out[n] = fs1[n] - fs2[n];
-      break;
-    case OP_HI_N_ADD:
-      dfluxb_rec(A.fx, r, ws, ps, fs1, fs2);
-      rec_dfs_any(A.fx, zz, ci, cj, ck, s0 - 1, a);
-      for (int n = 0; n < 5; n++) out[n] = (double)a[n] - fs1[n];
-      break;
-    case OP_LO_N_ADD:
-      dfluxb_rec(A.fx, r, ws, ps, fs1, fs2);
-      rec_dfs_any(A.fx, zz, ci, cj, ck, s0 + 2, a);
-      for (int n = 0; n < 5; n++) out[n] = fs2[n] - (double)a[n];
-      break;
-    case OP_E_UNDO:
-      rec_efs_any(A.fx, zz, ci, cj, ck, s0, a);
-      rec_efs_any(A.fx, zz, ci, cj, ck, s0 + 1, b);
-      for (int n = 0; n < 5; n++) out[n] = a[n] - b[n];
-      break;
-    case OP_E_ADD: {
-      double fs[5], fa[5];
-      efluxb_rec(A.fx, r, ws, ps, fs, fa, R.err);
-      bool hi = r.faceid >= 4;
-      for (int n = 0; n < 5; n++) {
-        out[n] = hi ? fa[n] : fs[n];
-        out[5 + n] = hi ? fs[n] : fa[n];
-      }
-      break;
+  cflux_st<0>(c.inf, v, p, S, fs);
+  cflux_st<1>(c.inf, v, p, S, a);
+  cflux_st<2>(c.inf, v, p, S, b);
+#pragma unroll
+  for (int n = 0; n < 5; n++) fs[n] = zz == 1 ? fs[n] : (zz == 2 ? a[n] : b[n]);
+}
+
+// the wall flux fs and the opposite-face flux fa of efluxb.f90:50-80, in FP64
+// like rec_wall_faces; the line's centre is the cut cell
+template <typename T>
+__device__ inline void rec_wall_flux(const FluxCtx<T> &c, const RecLine<T> &L, const RecOp &r, T Sc, const double *wsol,
+                                     double psol, double *fs, double *fa, int *err) {
+  const int zz = r.zz;
+  double sc[3], ss[3], wc[5], wo[5];
+  axis_vec(sc, zz, (double)Sc);
+  axis_vec(ss, zz, (double)face_s_any(c.g, zz, r.s[0], r.s[1], r.s[2]));
+#pragma unroll
+  for (int n = 0; n < 5; n++) {
+    wc[n] = full(c.inf, n, L.w[2][n]);
+    wo[n] = full(c.inf, n, r.hi ? L.w[1][n] : L.w[3][n]);
+  }
+  if (fabs(wc[0]) < (double)1.0e-8f) raise_err(err, MGE_ERR_WALL_RHO);
+  double fs1[5], fs2[5], fs3[5];
+  cflux3(wc, full(c.inf, 5, L.p[3]), sc, fs1);
+  cflux3(wsol, psol, ss, fs2);
+  // the opposite cell's own face vector: it differs from the cut cell's only
+  // along zz, which the vector does not depend on
+  cflux3(wo, full(c.inf, 5, r.hi ? L.p[2] : L.p[4]), sc, fs3);
+#pragma unroll
+  for (int n = 0; n < 5; n++) {
+    fs[n] = 0.5 * (fs1[n] + fs2[n]);
+    fa[n] = 0.5 * (fs1[n] + fs3[n]);
+  }
+}
+
+// the value op r contributes (dfluxb.f90 / efluxb.f90 terms, the Roe wall
+// face); the undo terms repeat the bulk kernel's face values in T
+template <typename T>
+__device__ __attribute__((always_inline)) inline void rec_op_value(const RecArgs<T> &R, const RecOp &r, double *out) {
+  const StageArgs<T> &A = R.st;
+  const FluxCtx<T> &c = A.fx;
+  const int kind = r.kind;
+  if (kind < OP_E_UNDO && !A.has_diss) return;
+  double ws[5];
+#pragma unroll
+  for (int n = 0; n < 5; n++) ws[n] = R.wsol[n * R.nmir + r.rec];
+  const double ps = R.psol[r.rec];
+  if (kind == OP_ROE_WALL) {
+    double ve[5], vd[5];
+    roe_wall_rec(c, r, r.hi != 0, ws, ps, (double)c.gamma, (double)A.eps, (double)c.cdis, ve, vd, R.err);
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+      out[n] = vd[n];
+      out[5 + n] = ve[n];
     }
-    case OP_ROE_WALL: {
-      double ve[5], vd[5];
-      roe_wall_rec(A.fx, r, ws, ps, (double)A.fx.gamma, (double)A.eps, (double)A.fx.cdis, ve, vd, R.err);
-      for (int n = 0; n < 5; n++) {
-        out[n] = vd[n];
-        out[5 + n] = ve[n];
-      }
-      break;
+    return;
+  }
+  // the centre: the lower of the two undone faces; the face pair's inner cell
+  // for the added terms; the cut cell for the convective terms
+  const bool add = kind == OP_HI_C_ADD || kind == OP_HI_N_ADD || kind == OP_LO_C_ADD || kind == OP_LO_N_ADD;
+  const int off = (add && r.hi) || kind == OP_HI_N_UNDO ? -1 : ((add && !r.hi) || kind == OP_LO_N_UNDO ? 1 : 0);
+  const T S = face_s_any(c.g, r.zz, r.c[0], r.c[1], r.c[2]);
+  const RecLine<T> L = rec_line(c, r, off);
+  if (kind < OP_E_UNDO) {
+    T a[5], b[5];
+    rec_face<0>(c, L, r.zz, S, a);
+    rec_face<1>(c, L, r.zz, S, b);
+    if (!add) {
+#pragma unroll
+      for (int n = 0; n < 5; n++) out[n] = a[n] - b[n];
+      return;
     }
-    default:
-      break;
+    double fi[5], fw[5];
+    rec_wall_faces(c, L, r.zz, r.hi != 0, (double)S, ws, ps, fi, fw);
+    const bool nb = kind == OP_HI_N_ADD || kind == OP_LO_N_ADD;
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+      if (r.hi) out[n] = nb ? (double)a[n] - fi[n] : fi[n] - fw[n];
+      else out[n] = nb ? fi[n] - (double)b[n] : fw[n] - fi[n];
+    }
+  } else if (kind == OP_E_UNDO) {
+    T fm[5], fc[5], fp[5];
+    rec_flux(c, r.zz, L.w[1], L.p[2], S, fm);
+    rec_flux(c, r.zz, L.w[2], L.p[3], S, fc);
+    rec_flux(c, r.zz, L.w[3], L.p[4], S, fp);
+#pragma unroll
+    for (int n = 0; n < 5; n++) out[n] = T(0.5) * (fc[n] + fm[n]) - T(0.5) * (fp[n] + fc[n]);
+  } else {
+    double fs[5], fa[5];
+    rec_wall_flux(c, L, r, S, ws, ps, fs, fa, R.err);
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+      out[n] = r.hi ? fa[n] : fs[n];
+      out[5 + n] = r.hi ? fs[n] : fa[n];
+    }
   }
 }
 
 // The wall records of a stage: each workgroup takes whole touched cells
 // with their ops (at most kRecOps), one thread per op computes its value
 // into LDS, then one thread per cell adds its ops' values in the reference
-// order (in FP64) and finishes the cell in T.
+// order (in FP64) and finishes the cell in T.  The launch lasts as long as
+// one workgroup's chain of round trips -- its range, the op, the op's line --
+// and the arithmetic of the op kinds one after another; reading each face's
+// stencil where a kind's branch needed it took 23-33 us on every level, the
+// line form takes 9-13 us (JST; Roe 8 -> 7).
 template <typename T>
 __device__ __attribute__((always_inline)) inline void k_rec_body(const RecArgs<T> &R, int bx, int, int) {
   __shared__ double val[kRecOps * 10];
-  const int2 ch = R.chunks[bx];
-  const int o0 = R.beg[ch.x], o1 = R.beg[ch.y];
+  __shared__ uint8_t kinds[kRecOps];
+  const int4 ch = R.chunks[bx];
+  const int o0 = ch.z;
   const int tid = threadIdx.x;
   const int t = ch.x + tid;
   const StageArgs<T> &A = R.st;
   const Dims &d = A.fx.d;
   const long E = d.E;
   // the cell's fw and dw, and the finish's inputs (W(0) on an unsmoothed
-  // stage, the local time step, the flags), are loaded before the op values
-  // are formed, so their round trips overlap the ops' own
+  // stage, the local time step, the flags, the forcing), are loaded before
+  // the op values are formed, so their round trips overlap the ops' own
   const bool cell = t < ch.y;
   const long q = cell ? R.tcell[t] : 0;
+  int b0 = 0, b1 = 0;
   double f[5], e[5];
-  T wnp[5] = {T(0), T(0), T(0), T(0), T(0)};
+  T wnp[5] = {T(0), T(0), T(0), T(0), T(0)}, qfp[5] = {T(0), T(0), T(0), T(0), T(0)};
   T vdt = T(0);
   uint8_t fl = 0;
   if (cell) {
+    b0 = R.beg[t];
+    b1 = R.beg[t + 1];
     for (int n = 0; n < 5; n++) {
       f[n] = A.fw[n * E + q];
       e[n] = A.dw[n * E + q];
@@ -1105,13 +1108,19 @@ __device__ __attribute__((always_inline)) inline void k_rec_body(const RecArgs<T
     vdt = A.vdtim[q];
     if (!A.smoothed && !A.lres)
       for (int n = 0; n < 5; n++) wnp[n] = A.wn[n * E + q];
+    if (A.coarse && !A.lfir1)
+      for (int n = 0; n < 5; n++) qfp[n] = A.qf[n * E + q];
   }
-  if (o0 + tid < o1) rec_op_value(R, o0 + tid, val + tid * 10);
+  if (o0 + tid < ch.w) {
+    const RecOp r = R.ops[o0 + tid];
+    kinds[tid] = r.kind;
+    rec_op_value(R, r, val + tid * 10);
+  }
   __syncthreads();
   if (!cell) return;
-  for (int o = R.beg[t]; o < R.beg[t + 1]; o++) {
-    int kind = R.ops[o].y;
-    const double *v = val + (o - o0) * 10;
+  for (int o = b0 - o0; o < b1 - o0; o++) {
+    const int kind = kinds[o];
+    const double *v = val + o * 10;
     switch (kind) {
       case OP_HI_C_UNDO:
       case OP_HI_N_UNDO:
@@ -1148,7 +1157,7 @@ __device__ __attribute__((always_inline)) inline void k_rec_body(const RecArgs<T
     ft[n] = (T)f[n];
     et[n] = (T)e[n];
   }
-  finish_cell<T, true>(A, q, ft, et, wnp, vdt, fl);
+  finish_cell<T, true>(A, q, ft, et, wnp, vdt, fl, qfp);
 }
 MGE_ENTRY_T(k_rec, RecArgs, 64, 1)
 

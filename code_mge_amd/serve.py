@@ -83,8 +83,8 @@ def level_bytes(n, es, nmir=0, mxcyc=4, viscous=False, coarse=False, psmoo=False
         sizes += [24 * E]               # limiter words (three per cell)
     if nmir:
         ntouch, nops = 2 * nmir, 6 * nmir
-        sizes += [DEVREC_BYTES * nmir, 40 * nmir, 8 * nmir, 8 * ntouch, 4 * (ntouch + 1), 8 * (nops + 1),
-                  8 * (ntouch + 1), 80 * (nops + 1)]
+        sizes += [DEVREC_BYTES * nmir, 40 * nmir, 8 * nmir, 8 * ntouch, 4 * (ntouch + 1), 48 * (nops + 1),
+                  16 * (ntouch + 1), 80 * (nops + 1)]
         sizes += [8 * nmir, 4 * (nmir + 1), 4 * nmir]   # cut cells with their record lists
     return sum(s + 64 for s in sizes)
 
