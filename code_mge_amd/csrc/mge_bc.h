@@ -252,6 +252,105 @@ __device__ __attribute__((always_inline)) inline void k_rtrms_final_body(const R
 }
 MGE_ENTRY(k_rtrms_final, RfArgs, 256, 1)
 
+// ------------------------------------------------------------------ post-smoothing update
+
+// after smoothing: w = wn - dw and the EOS on interior cells
+// (euler.f90:381-399), one thread per cell of the whole array so that the
+// accesses stream through aligned rows; the ghost shell of the previous
+// state is carried over where anything reads it before bcond rewrites it,
+// as k_ghost_copy does on unsmoothed stages
+template <typename T>
+struct UpdArgs {
+  Dims d;
+  const T *wn, *dw;
+  StateC<T> src;
+  State<T> dst;
+  T gamma;
+  Inf<T> inf;
+  // unsteady update on the finest active level: w = wn - dw/lam
+  // (euler.f90:383-393)
+  int ulam;
+  const T *vdtim;
+  const double *dtim;
+  T fn, dtstep;
+  int vt;
+  int carry;   // carry the ghost shell over
+};
+
+// the updated state of interior cell q; returns p
+template <typename T>
+__device__ inline T upd_cell(const UpdArgs<T> &U, long q, T *v) {
+  const long E = U.d.E;
+  if (U.ulam) {
+    const T lam = unsteady_lam(U.fn, U.vdtim, U.dtim, U.vt, U.dtstep, q);
+#pragma unroll
+    for (int n = 0; n < 5; n++) v[n] = U.wn[n * E + q] - U.dw[n * E + q] / lam;
+  } else {
+#pragma unroll
+    for (int n = 0; n < 5; n++) v[n] = U.wn[n * E + q] - U.dw[n * E + q];
+  }
+  return eos_st(U.gamma, U.inf, v);
+}
+
+template <typename T>
+__device__ __attribute__((always_inline)) inline void k_update_ghost_body(const UpdArgs<T> &U, int bx, int, int) {
+  const Dims &d = U.d;
+  const StateC<T> &src = U.src;
+  const State<T> &dst = U.dst;
+  const long q = bx * (long)blockDim.x + threadIdx.x;
+  if (q >= d.E) return;
+  int i, j, k;
+  if (d.E <= 0xffffffffL) {  // 32-bit index arithmetic
+    const unsigned uq = (unsigned)q, sz = (unsigned)d.sz, sy = (unsigned)d.sy;
+    const unsigned kk = uq / sz, r = uq - kk * sz, jj = r / sy;
+    i = (int)(r - jj * sy);
+    j = (int)jj;
+    k = (int)kk;
+  } else {
+    k = (int)(q / d.sz);
+    j = (int)((q - (long)k * d.sz) / d.sy);
+    i = (int)(q - (long)k * d.sz - (long)j * d.sy);
+  }
+  if (!(i >= 2 && i <= d.il && j >= 2 && j <= d.jl && k >= 2 && k <= d.kl)) {
+    if (U.carry) {
+      for (int n = 0; n < 5; n++) dst.w[n * d.E + q] = src.w[n * d.E + q];
+      dst.p[q] = src.p[q];
+    }
+    return;
+  }
+  T v[5];
+  const T p = upd_cell(U, q, v);
+  for (int n = 0; n < 5; n++) dst.w[n * d.E + q] = v[n];
+  dst.p[q] = p;
+}
+MGE_ENTRY_T(k_update_ghost, UpdArgs, 256, 1)
+
+// ---- where the boundary kernels read interior cells
+//
+// SrcState: the state buffer.  SrcUpd: the state a smoothed stage's update is
+// about to write there, formed from its inputs with the update's own
+// expressions, so that bc_cutcell and bcond can run in the update's launch.
+template <typename T>
+struct CellV {
+  T w[5];
+  T p;
+};
+template <typename T>
+struct SrcState {
+  const T *w, *p;
+  long E;
+  __device__ void load(long q, CellV<T> &o) const {
+#pragma unroll
+    for (int n = 0; n < 5; n++) o.w[n] = w[n * E + q];
+    o.p = p[q];
+  }
+};
+template <typename T>
+struct SrcUpd {
+  const UpdArgs<T> &U;
+  __device__ void load(long q, CellV<T> &o) const { o.p = upd_cell(U, q, o.w); }
+};
+
 // ------------------------------------------------------------------ bc_cutcell
 
 template <typename T>
@@ -267,18 +366,45 @@ struct CutArgs {
   int *err;
 };
 
-// bc_cutcell.f90:40-219 for steady bodies (qb = 0), in FP64
-template <typename T>
-__device__ __attribute__((always_inline)) inline void k_bc_cut_body(const CutArgs<T> &C, int bx, int, int) {
-  int m = bx * blockDim.x + threadIdx.x;
+// bc_cutcell.f90:40-219 for steady bodies (qb = 0), in FP64.  Eight threads a
+// record: each loads one cell of its cloud, six of them sum one value each in
+// the reference order, and one forms the mirror state.  With a thread per
+// record its 48 gathered loads and their sums made the launch 9.5 us for the
+// 1400 records of a 48^3 block, 5.5 us in this form.
+constexpr int kCutRecs = 32;   // records per block of 256 threads
+template <typename T, class S>
+__device__ __attribute__((always_inline)) inline void bc_cut_cells(const CutArgs<T> &C, const S &src, int bx) {
+  __shared__ double prod[6][256], sums[6][kCutRecs];
+  const int tid = threadIdx.x, slot = tid >> 3, c = tid & 7;
+  const int m = bx * kCutRecs + slot;
+  const bool upd = m < C.nupd && m != C.zero_at;
+  const DevRec &r = C.recs[upd ? m : 0];
+  int np = 0;
+  if (upd) {
+    np = r.npoint;
+    if (c < np) {
+      const double f = r.coef[c];
+      CellV<T> v;
+      src.load(r.cloud[c], v);
+#pragma unroll
+      for (int n = 0; n < 5; n++) prod[n][tid] = f * full(C.inf, n, v.w[n]);
+      prod[5][tid] = f * full(C.inf, 5, v.p);
+    }
+  }
+  __syncthreads();
+  if (upd && c < 6) {
+    double s = 0.0;
+    for (int q = 0; q < np; q++) s = s + prod[c][(slot << 3) + q];
+    sums[c][slot] = s;
+  }
+  __syncthreads();
+  if (c != 0) return;
   if (m == C.zero_at) {
     for (int n = 0; n < 5; n++) C.wsol[n * C.nmir + m] = 0.0;
     C.psol[m] = 0.0;
     return;
   }
-  if (m >= C.nupd) return;
-  const DevRec &r = C.recs[m];
-  const long E = C.d.E;
+  if (!upd) return;
   double nv[3] = {r.nvec[0], r.nvec[1], r.nvec[2]};
   double qb[3] = {0.0, 0.0, 0.0};
   double s = 0.0;
@@ -287,31 +413,10 @@ __device__ __attribute__((always_inline)) inline void k_bc_cut_body(const CutArg
   s = s + nv[2] * nv[2];
   double nn = sqrt(s);
   for (int dd = 0; dd < 3; dd++) nv[dd] = nv[dd] / nn;
-  // every cloud value is loaded before the sums use any (the loads are in
-  // flight together rather than one round trip each); the sums keep the
-  // reference order
-  const int np = r.npoint;
-  T cw[8][6];
+  double vr[5], ws[5];
 #pragma unroll
-  for (int c = 0; c < 8; c++) {
-    if (c < np) {
-      const long qc = r.cloud[c];
-#pragma unroll
-      for (int n = 0; n < 5; n++) cw[c][n] = C.s.w[n * E + qc];
-      cw[c][5] = C.s.p[qc];
-    }
-  }
-  double vr[5] = {0, 0, 0, 0, 0}, pr = 0.0;
-#pragma unroll
-  for (int n = 0; n < 5; n++)
-#pragma unroll
-    for (int c = 0; c < 8; c++)
-      if (c < np) vr[n] = vr[n] + r.coef[c] * full(C.inf, n, cw[c][n]);
-#pragma unroll
-  for (int c = 0; c < 8; c++)
-    if (c < np) pr = pr + r.coef[c] * full(C.inf, 5, cw[c][5]);
-  double psol = pr, ws[5];
-  for (int n = 0; n < 5; n++) ws[n] = vr[n];
+  for (int n = 0; n < 5; n++) ws[n] = vr[n] = sums[n][slot];
+  const double psol = sums[5][slot];
   if (C.eqntype == 0) {
     double qn = 2.0 * (nv[0] * (ws[1] - ws[0] * qb[0]) + nv[1] * (ws[2] - ws[0] * qb[1]) +
                        nv[2] * (ws[3] - ws[0] * qb[2]));
@@ -330,7 +435,11 @@ __device__ __attribute__((always_inline)) inline void k_bc_cut_body(const CutArg
   for (int n = 0; n < 5; n++) C.wsol[n * C.nmir + m] = ws[n];
   C.psol[m] = psol;
 }
-MGE_ENTRY_T(k_bc_cut, CutArgs, 64, 1)
+template <typename T>
+__device__ __attribute__((always_inline)) inline void k_bc_cut_body(const CutArgs<T> &C, int bx, int, int) {
+  bc_cut_cells(C, SrcState<T>{C.s.w, C.s.p, C.d.E}, bx);
+}
+MGE_ENTRY_T(k_bc_cut, CutArgs, 256, 1)
 
 // ------------------------------------------------------------------ bcond
 
@@ -352,49 +461,101 @@ MGE_ENTRY_T(k_bc_cut, CutArgs, 64, 1)
 // cell); such a level runs the six faces one after another inside a single
 // workgroup instead.  Far-field branch bytes are recorded where the face is
 // the cell's last writer: those are the only positions a frozen solve reads.
+enum FaceKind : unsigned { FACE_NONE = 0, FACE_FAR, FACE_SYM, FACE_PER, FACE_WALL };
 template <typename T>
 struct FacesArgs {
   Dims d;
   State<T> s;
-  int kind[6];        // faces 1..6: -20 far, -50 symmetry, -60 periodic, -80 wall, 0 not written
+  // faces 1..6, four bits each (FaceKind): a word rather than an array, whose
+  // indexing by a thread's face would put the arguments in scratch memory
+  unsigned kinds;
+  int wall;           // a FACE_WALL among them
   int seq;            // 1: faces in order inside one workgroup (a direction with one cell)
   double gamma, rho0, p0, c0, u0, v0, w0;
   double s0;          // freestream entropy rho0^gamma / p0
   Inf<T> inf;
-  uint8_t *ffdec[6];  // far field: each face's branch per ghost point, or nullptr
+  uint8_t *ffdec;     // far field: the branch per ghost point, face after face, or nullptr
   const int *frozen;
   // bc_cutcell's mirror states in the same launch (blocks nfb..): it runs
   // before bcond, reads only interior cells (the level's clouds are checked
   // on the host) and writes only wsol/psol, so the two are independent
   long nfb;           // blocks of the faces
   CutArgs<T> cut;     // cut.nmir == 0: no records in this launch
+  // cells of the launch: the first nt of the shell numbering (all, or the
+  // faces' own cells where the edges are left to k_bc_edges), then ned edge
+  // cells of bc_corner that a viscous stencil reads (0 or all twelve edges)
+  long nt, ned;
+  double gm, rgamma;  // 1/(gamma - 1), 1/gamma
+  double rinf;        // 2 c0/(gamma - 1)
+  int air;            // gamma = 7/5 up to its rounding: the powers 7/5 and 5/2 in closed form
 };
 
 template <typename T>
-struct CellV {
-  T w[5];
-  T p;
-};
+__device__ inline unsigned face_kind(const FacesArgs<T> &A, int f) {
+  return (A.kinds >> (4 * (f - 1))) & 15u;
+}
 
 // the highest-numbered face that writes cell (x, y, z) (0: none)
 template <typename T>
 __device__ inline int last_face(const FacesArgs<T> &A, int x, int y, int z) {
   const Dims &d = A.d;
   int f = 0;
-  if (x <= 1 && A.kind[0]) f = 1;
-  if (y <= 1 && A.kind[1]) f = 2;
-  if (z <= 1 && A.kind[2]) f = 3;
-  if (x >= d.ie && A.kind[3]) f = 4;
-  if (y >= d.je && A.kind[4]) f = 5;
-  if (z >= d.ke && A.kind[5]) f = 6;
+  if (x <= 1 && face_kind(A, 1)) f = 1;
+  if (y <= 1 && face_kind(A, 2)) f = 2;
+  if (z <= 1 && face_kind(A, 3)) f = 3;
+  if (x >= d.ie && face_kind(A, 4)) f = 4;
+  if (y >= d.je && face_kind(A, 5)) f = 5;
+  if (z >= d.ke && face_kind(A, 6)) f = 6;
   return f;
 }
 
-__device__ inline double pick3(int dir, double a, double b, double c) { return dir == 0 ? a : (dir == 1 ? b : c); }
+// a, b or c by direction.  The values are made opaque first: a select between
+// loads of argument fields would be turned into one load through a selected
+// field address, which puts the whole argument block in scratch memory.
+template <typename V>
+__device__ inline V pick3(int dir, V a, V b, V c) {
+  asm("" : "+v"(a), "+v"(b), "+v"(c));
+  return dir == 0 ? a : (dir == 1 ? b : c);
+}
 
 // bc_far.f90:26-284: the ghost state of a far-field face from the state at
 // phy1, in FP64 on full state values (FP32 stores deviations); components
-// are picked by selects rather than indexed by the face direction
+// are picked by selects rather than indexed by the face direction.  The two
+// branches take the same normal velocity and speed of sound from the Riemann
+// invariants and differ in where the entropy and the tangential velocity come
+// from, so a wave evaluates one of them, not both in turn.  The launch lasts
+// as long as its deepest chain of these states: with two branches of up to
+// two pow calls and chains of three faces, k_bc_faces took 9.5-18 us on every
+// level; with one branch, the powers in closed form and the edges left out it
+// takes 5-6 us.
+// x^(5/2) to rounding, as pow gives it: x^2 and sqrt(x) with their residuals
+__device__ inline double pow25(double x) {
+  const double y = x * x, ey = __builtin_fma(x, x, -y);
+  const double s = sqrt(x), es = __builtin_fma(-s, s, x);
+  const double r = y * s, er = __builtin_fma(y, s, -r);
+  return x > 0.0 ? r + (er + __builtin_fma(ey, s, y * (0.5 * es * rcp_pos(s)))) : r;
+}
+// x^(7/5) to rounding: z = x^(2/5) from an FP32 estimate z0 and the relative
+// defect e = x^2 / z0^5 - 1 (about 1e-6), z = z0 (1 + e)^(1/5); products that
+// must not lose the defect carry their FMA residuals
+__device__ inline double pow75(double x) {
+  if (!(x > 1e-12 && x < 1e12)) return pow(x, 1.4);
+  const double z0 = (double)exp2f(0.4f * log2f((float)x));
+  const double z2 = z0 * z0;   // exact: z0 has 24 bits
+  const double z4 = z2 * z2, e4 = __builtin_fma(z2, z2, -z4);
+  const double z5 = z4 * z0, e5 = __builtin_fma(z4, z0, -z5) + e4 * z0;
+  const double x2 = x * x, ex = __builtin_fma(x, x, -x2);
+  const double e = ((x2 - z5) + (ex - e5)) * rcp_pos(z5);
+  const double dz = z0 * (e * (0.2 + e * (-0.08 + 0.048 * e)));
+  const double w = x * z0, ew = __builtin_fma(x, z0, -w);
+  return w + (ew + x * dz);
+}
+// a / b from the refined reciprocal rb of b: the quotient corrected by its
+// remainder, the rounded quotient but for rare last-bit cases
+__device__ inline double div_by(double a, double b, double rb) {
+  const double q = a * rb;
+  return __builtin_fma(__builtin_fma(-b, q, a), rb, q);
+}
 template <typename T>
 __device__ inline CellV<T> far_state(const FacesArgs<T> &A, int f, CellV<T> v, uint8_t *dec,
                                                         bool rec) {
@@ -402,55 +563,29 @@ __device__ inline CellV<T> far_state(const FacesArgs<T> &A, int f, CellV<T> v, u
   const Inf<T> &fi = A.inf;
   const int dir = (f - 1) % 3;
   const double sg = f <= 3 ? -1.0 : 1.0;
-  const double fn0 = dir == 0 ? sg : 0.0, fn1 = dir == 1 ? sg : 0.0, fn2 = dir == 2 ? sg : 0.0;
-  const double gamma = A.gamma, gm = 1.0 / (gamma - 1.0);
-  const double w0 = full(fi, 0, v.w[0]), w1 = full(fi, 1, v.w[1]), w2 = full(fi, 2, v.w[2]),
-               w3 = full(fi, 3, v.w[3]);
-  double s = 0.0;
-  s = s + w1 * fn0;
-  s = s + w2 * fn1;
-  s = s + w3 * fn2;
-  const double vel_norm = s / w0;
-  bool inflow = vel_norm <= 0.0;
+  const double gamma = A.gamma, g1 = gamma - 1.0, gm = A.gm;
+  const double rho = full(fi, 0, v.w[0]), m0 = full(fi, 1, v.w[1]), m1 = full(fi, 2, v.w[2]),
+               m2 = full(fi, 3, v.w[3]), pe = full(fi, 5, v.p);
+  const double rr = rcp_pos(rho);
+  const double u0 = div_by(m0, rho, rr), u1 = div_by(m1, rho, rr), u2 = div_by(m2, rho, rr);
+  bool inflow = pick3(dir, u0, u1, u2) * sg <= 0.0;
   if (dec) {
     if (*A.frozen) inflow = *dec == 0;
     else if (rec) *dec = inflow ? 0 : 1;
   }
-  const double fnd = sg, vinfd = pick3(dir, A.u0, A.v0, A.w0);
-  double r, v0, v1, v2, pr;
-  if (inflow) {
-    double rhoe = w0;
-    double ue = pick3(dir, w1, w2, w3) / rhoe;
-    double pe = full(fi, 5, v.p);
-    double ce = sqrt(gamma * pe / rhoe);
-    double rpo = ue * fnd + 2.0 * ce / (gamma - 1.0);
-    double rmi = vinfd * fnd - 2.0 * A.c0 / (gamma - 1.0);
-    double un = 0.5 * (rpo + rmi) * fnd;
-    double ci = 0.25 * (gamma - 1.0) * (rpo - rmi);
-    v0 = dir == 0 ? un : A.u0;
-    v1 = dir == 1 ? un : A.v0;
-    v2 = dir == 2 ? un : A.w0;
-    double si = A.s0;
-    double cc = ci * ci / gamma;
-    r = pow(si * cc, gm);
-    pr = r * cc;
-  } else {
-    double rhoi = w0;
-    double vv0 = w1 / rhoi, vv1 = w2 / rhoi, vv2 = w3 / rhoi;
-    double prei = full(fi, 5, v.p);
-    double si = pow(rhoi, gamma) / prei;
-    double ci = sqrt(gamma * prei / rhoi);
-    double rpo = pick3(dir, vv0, vv1, vv2) * fnd + 2.0 * ci / (gamma - 1.0);
-    double rmi = vinfd * fnd - 2.0 * A.c0 / (gamma - 1.0);
-    double un = 0.5 * (rpo + rmi) * fnd;
-    double ce = 0.25 * (gamma - 1.0) * (rpo - rmi);
-    v0 = dir == 0 ? un : vv0;
-    v1 = dir == 1 ? un : vv1;
-    v2 = dir == 2 ? un : vv2;
-    double cc = ce * ce / gamma;
-    r = pow(si * cc, gm);
-    pr = r * cc;
-  }
+  const double rpo = pick3(dir, u0, u1, u2) * sg + div_by(2.0 * sqrt(div_by(gamma * pe, rho, rr)), g1, gm);
+  const double rmi = pick3(dir, A.u0, A.v0, A.w0) * sg - A.rinf;
+  const double un = 0.5 * (rpo + rmi) * sg;
+  const double ci = 0.25 * g1 * (rpo - rmi);
+  const double cc = div_by(ci * ci, gamma, A.rgamma);
+  double si = A.s0;
+  if (!inflow) si = (A.air ? pow75(rho) : pow(rho, gamma)) / pe;
+  const double x = si * cc;
+  const double r = A.air ? pow25(x) : pow(x, gm);
+  const double pr = r * cc;
+  const double v0 = dir == 0 ? un : (inflow ? A.u0 : u0);
+  const double v1 = dir == 1 ? un : (inflow ? A.v0 : u1);
+  const double v2 = dir == 2 ? un : (inflow ? A.w0 : u2);
   o.w[0] = stored(fi, 0, r);
   o.w[1] = stored(fi, 1, r * v0);
   o.w[2] = stored(fi, 2, r * v1);
@@ -460,81 +595,215 @@ __device__ inline CellV<T> far_state(const FacesArgs<T> &A, int f, CellV<T> v, u
   return o;
 }
 
-template <typename T, int D>
-__device__ __attribute__((always_inline)) inline void face_chain(const FacesArgs<T> &A, int x, int y, int z,
-                                                                 bool top, CellV<T> &o);
+template <typename T, int D, class S>
+__device__ __attribute__((always_inline)) inline void face_chain(const FacesArgs<T> &A, const S &src, int x, int y,
+                                                                 int z, bool top, CellV<T> &o);
 
-// face f's value in its ghost cell (x, y, z) (bc_far.f90, bc_symm.f90,
-// bc_periodic.f90, bc_wall.f90), its sources taken as face_chain<D> of
-// them; `top`: the thread's own cell (it records the far-field branch)
-template <typename T, int D>
-__device__ __attribute__((always_inline)) inline void face_step(const FacesArgs<T> &A, int f, int x, int y, int z,
-                                                                bool top, CellV<T> &o) {
+// the source cell of ghost cell (x, y, z) through face f (in place); false in
+// the second ghost layer of the face's direction
+template <typename T>
+__device__ inline bool face_source(const FacesArgs<T> &A, int f, int &x, int &y, int &z) {
   const Dims &d = A.d;
   const int dir = (f - 1) % 3;
   const bool lo = f <= 3;
-  const int nl = dir == 0 ? d.il : (dir == 1 ? d.jl : d.kl);
+  const int nl = pick3(dir, d.il, d.jl, d.kl);
   const int cd = dir == 0 ? x : (dir == 1 ? y : z);
   const bool l1 = lo ? cd == 1 : cd == nl + 1;  // first ghost layer
-  const int kind = A.kind[f - 1];
-  // source index along dir: phy1 (far field, the first layer, the wall's
-  // pressure) or phy2 (the second layer)
-  const int p1 = kind == -60 ? (lo ? nl : 2) : (lo ? 2 : nl);
-  const int p2 = kind == -60 ? (lo ? nl - 1 : 3) : (lo ? 3 : nl - 1);
-  const int sd = (kind == -20 || l1) ? p1 : p2;
-  const int sx = dir == 0 ? sd : x, sy = dir == 1 ? sd : y, sz = dir == 2 ? sd : z;
-  face_chain<T, D>(A, sx, sy, sz, false, o);
-  if (kind == -20) {
+  const unsigned kind = face_kind(A, f);
+  // phy1 (far field, the first layer) or phy2 (the second layer)
+  const bool near = kind == FACE_FAR || l1;
+  const int sd = kind == FACE_PER ? (lo ? (near ? nl : nl - 1) : (near ? 2 : 3))
+                                  : (lo ? (near ? 2 : 3) : (near ? nl : nl - 1));
+  x = dir == 0 ? sd : x;
+  y = dir == 1 ? sd : y;
+  z = dir == 2 ? sd : z;
+  return l1;
+}
+
+// face f's value o in its ghost cell (x, y, z) (bc_far.f90, bc_symm.f90,
+// bc_periodic.f90, bc_wall.f90) from its source cell's, but for the wall's
+// pressure in the second layer; `rec`: record the far-field branch
+template <typename T>
+__device__ __attribute__((always_inline)) inline void face_apply(const FacesArgs<T> &A, int f, int x, int y, int z,
+                                                                 bool rec, CellV<T> &o) {
+  const Dims &d = A.d;
+  const int dir = (f - 1) % 3;
+  const bool lo = f <= 3;
+  const unsigned kind = face_kind(A, f);
+  if (kind == FACE_FAR) {
     uint8_t *dec = nullptr;
-    if (A.ffdec[f - 1]) {
+    if (A.ffdec) {
       const int a = dir == 0 ? y : x, c2 = dir == 2 ? y : z;
-      const int amax = dir == 0 ? d.jb : d.ib;
-      dec = A.ffdec[f - 1] + a + (long)(amax + 1) * c2;
+      const int amax = pick3(dir, d.jb, d.ib, d.ib);
+      const long s0 = (long)(d.jb + 1) * (d.kb + 1), s1 = (long)(d.ib + 1) * (d.kb + 1), s2 = d.sz;
+      dec = A.ffdec + (lo ? 0 : s0 + s1 + s2) + (dir > 0 ? s0 : 0) + (dir > 1 ? s1 : 0) + a + (long)(amax + 1) * c2;
     }
-    o = far_state(A, f, o, dec, top && l1);
+    o = far_state(A, f, o, dec, rec);
     return;
   }
   const Inf<T> &fi = A.inf;
-  if (kind == -50 || kind == -80) {
+  if (kind == FACE_SYM || kind == FACE_WALL) {
 #pragma unroll
     for (int n = 1; n < 4; n++)
-      if (kind == -80 || n == 1 + dir) o.w[n] = stored(fi, n, -full(fi, n, o.w[n]));
+      if (kind == FACE_WALL || n == 1 + dir) o.w[n] = stored(fi, n, -full(fi, n, o.w[n]));
   }
-  if (kind == -80 && !l1) {  // bc_wall: the second ghost layer takes the pressure of phy1
+}
+
+// face f's value in its ghost cell, its sources taken as face_chain<D> of
+// them; `top`: the thread's own cell (it records the far-field branch)
+template <typename T, int D, class S>
+__device__ __attribute__((always_inline)) inline void face_step(const FacesArgs<T> &A, const S &src, int f, int x,
+                                                                int y, int z, bool top, CellV<T> &o) {
+  int sx = x, sy = y, sz = z;
+  const bool l1 = face_source(A, f, sx, sy, sz);
+  face_chain<T, D>(A, src, sx, sy, sz, false, o);
+  face_apply(A, f, x, y, z, top && l1, o);
+  if (face_kind(A, f) == FACE_WALL && !l1) {  // bc_wall: the second ghost layer takes the pressure of phy1
+    const int dir = (f - 1) % 3, p1 = f <= 3 ? 2 : pick3(dir, A.d.il, A.d.jl, A.d.kl);
     CellV<T> v;
-    face_chain<T, D>(A, dir == 0 ? p1 : x, dir == 1 ? p1 : y, dir == 2 ? p1 : z, false, v);
+    face_chain<T, D>(A, src, dir == 0 ? p1 : x, dir == 1 ? p1 : y, dir == 2 ? p1 : z, false, v);
     o.p = v.p;
   }
 }
 
 // the value bcond leaves in cell (x, y, z), with at most D faces writing it
-template <typename T, int D>
-__device__ __attribute__((always_inline)) inline void face_chain(const FacesArgs<T> &A, int x, int y, int z,
-                                                                 bool top, CellV<T> &o) {
+template <typename T, int D, class S>
+__device__ __attribute__((always_inline)) inline void face_chain(const FacesArgs<T> &A, const S &src, int x, int y,
+                                                                 int z, bool top, CellV<T> &o) {
   if constexpr (D > 0) {
     const int f = last_face(A, x, y, z);
     if (f != 0) {
-      face_step<T, D - 1>(A, f, x, y, z, top, o);
+      face_step<T, D - 1>(A, src, f, x, y, z, top, o);
       return;
     }
   }
-  const Dims &d = A.d;
-  const long q = ix(d, x, y, z), E = d.E;
+  src.load(ix(A.d, x, y, z), o);
+}
+
+// the same for any ghost cell.  Without wall faces each step has one source
+// cell, so the chain is a loop around one copy of the face rules; the nested
+// form, which a wall's pressure needs, holds a copy per step and branch, and
+// its instructions alone (fetched cold) made the edges' launch take 24-27 us
+// where the loop takes 11 us.
+template <typename T, class S>
+__device__ __attribute__((always_inline)) inline void face_chain_any(const FacesArgs<T> &A, const S &src, int x, int y,
+                                                                     int z, bool top, CellV<T> &o) {
+  if (A.wall) {  // uniform
+    face_chain<T, 3>(A, src, x, y, z, top, o);
+    return;
+  }
+  int f[3], cx[3], cy[3], cz[3], n = 0;
+  bool l1 = false;
 #pragma unroll
-  for (int n = 0; n < 5; n++) o.w[n] = A.s.w[n * E + q];
-  o.p = A.s.p[q];
+  for (int t = 0; t < 3; t++) {
+    f[t] = last_face(A, x, y, z);
+    cx[t] = x;
+    cy[t] = y;
+    cz[t] = z;
+    if (f[t] == 0) continue;
+    const bool l = face_source(A, f[t], x, y, z);
+    if (t == 0) l1 = l;
+    n = t + 1;
+  }
+  src.load(ix(A.d, x, y, z), o);
+#pragma unroll 1
+  for (int t = n - 1; t >= 0; t--)
+    face_apply(A, pick3(t, f[0], f[1], f[2]), pick3(t, cx[0], cx[1], cx[2]), pick3(t, cy[0], cy[1], cy[2]),
+               pick3(t, cz[0], cz[1], cz[2]), top && t == 0 && l1, o);
+}
+
+template <typename T>
+__device__ inline void put_cell(const State<T> &s, long E, long q, const CellV<T> &o) {
+#pragma unroll
+  for (int n = 0; n < 5; n++) s.w[n * E + q] = o.w[n];
+  s.p[q] = o.p;
+}
+
+// edge cell t of the first ghost layer with an interior third index, of the
+// 4 (nk + nj + ni) that bc_corner.f90:23-137 extrapolates: its indices g and,
+// along the edge's two directions da < db, the interior neighbours' indices
+// (na, nb); false past the last
+__device__ inline bool edge_at(const Dims &d, long t, int *g, int *da, int *db, int *na, int *nb) {
+  const long n1 = 4L * d.nk, n2 = 4L * d.nj, n3 = 4L * d.ni;
+  int dir;
+  if (t < n1) dir = 2;
+  else if (t < n1 + n2) { dir = 1; t -= n1; }
+  else if (t < n1 + n2 + n3) { dir = 0; t -= n1 + n2; }
+  else return false;
+  const int x = 2 + (int)(t >> 2), ha = (int)(t & 1), hb = (int)(t >> 1) & 1;
+  *da = dir == 0 ? 1 : 0;
+  *db = dir == 2 ? 1 : 2;
+  const int la = pick3(*da, d.il, d.jl, d.jl), lb = pick3(*db, d.jl, d.jl, d.kl);
+  const int ga = ha ? la + 1 : 1, gb = hb ? lb + 1 : 1;
+  *na = ha ? la : 2;
+  *nb = hb ? lb : 2;
+  g[0] = dir == 0 ? x : ga;
+  g[1] = dir == 1 ? x : (dir == 0 ? ga : gb);
+  g[2] = dir == 2 ? x : gb;
+  return true;
+}
+
+// the extrapolated value of such an edge cell from the face ghosts next to it,
+// evaluated here (they are written by other threads of this launch).  The
+// i-edge at (je, 1) reads its own target and adds and subtracts one cell
+// (bc_corner.f90:120).
+template <typename T, class S>
+__device__ inline bool edge_value(const FacesArgs<T> &A, const S &src, long t, long *q, CellV<T> &o) {
+  const Dims &d = A.d;
+  int g[3], da, db, na, nb;
+  if (!edge_at(d, t, g, &da, &db, &na, &nb)) return false;
+  *q = ix(d, g[0], g[1], g[2]);
+  const bool self = da == 1 && g[1] == d.je && g[2] == 1;
+  CellV<T> a, b, c;
+  // (na, gb) and (ga, nb); the reference's sums start with the first on k- and
+  // j-edges and on the i-edge at (je, ke) and (1, ke)
+  const int ax = da == 0 ? na : g[0], ay = da == 1 ? na : g[1], az = g[2];
+  const int bx = g[0], by = db == 1 ? nb : g[1], bz = db == 2 ? nb : g[2];
+  const int cx = da == 0 ? na : g[0], cy = da == 1 ? na : (db == 1 ? nb : g[1]), cz = db == 2 ? nb : g[2];
+  src.load(ix(d, cx, cy, cz), c);
+  if (self) {
+    face_chain<T, 2>(A, src, g[0], g[1], g[2], false, a);
+    b = c;
+  } else {
+    face_chain<T, 1>(A, src, ax, ay, az, false, a);
+    face_chain<T, 1>(A, src, bx, by, bz, false, b);
+  }
+#pragma unroll
+  for (int n = 0; n < 5; n++) o.w[n] = a.w[n] + b.w[n] - c.w[n];
+  o.p = eos_st((T)A.gamma, A.inf, o.w);
+  return true;
+}
+
+// one block of the boundary cells: the shell's (nt of them) and the edges'
+template <typename T, class S>
+__device__ __attribute__((always_inline)) inline void faces_cells(const FacesArgs<T> &A, const S &src, long bx) {
+  const Dims &d = A.d;
+  const long t = bx * blockDim.x + threadIdx.x;
+  CellV<T> o;
+  if (t >= A.nt) {
+    long q;
+    if (t < A.nt + A.ned && edge_value(A, src, t - A.nt, &q, o)) put_cell(A.s, d.E, q, o);
+    return;
+  }
+  int x, y, z;
+  if (!shell_cell_by_depth(d, t, x, y, z)) return;
+  if (last_face(A, x, y, z) == 0) return;
+  if (A.nt == face_cells(d)) face_chain<T, 1>(A, src, x, y, z, true, o);  // uniform: no edge cells among them
+  else face_chain_any(A, src, x, y, z, true, o);
+  put_cell(A.s, d.E, ix(d, x, y, z), o);
 }
 
 template <typename T>
 __device__ __attribute__((always_inline)) inline void k_bc_faces_body(const FacesArgs<T> &A, int bx, int, int) {
   const Dims &d = A.d;
+  const SrcState<T> src{A.s.w, A.s.p, d.E};
   if (A.seq) {  // one workgroup: the faces in order, as bcond.f90
     for (int f = 1; f <= 6; f++) {
-      if (A.kind[f - 1] == 0) continue;
+      if (face_kind(A, f) == FACE_NONE) continue;
       const int dir = (f - 1) % 3;
-      const int nl = dir == 0 ? d.il : (dir == 1 ? d.jl : d.kl);
+      const int nl = pick3(dir, d.il, d.jl, d.kl);
       const int g1 = f <= 3 ? 1 : nl + 1, g2 = f <= 3 ? 0 : nl + 2;  // the two ghost layers
-      const int amax = dir == 0 ? d.jb : d.ib, cmax = dir == 2 ? d.jb : d.kb;
+      const int amax = pick3(dir, d.jb, d.ib, d.ib), cmax = pick3(dir, d.kb, d.kb, d.jb);
       const long npos = (long)(amax + 1) * (cmax + 1);
       for (long m = threadIdx.x; m < npos; m += blockDim.x) {
         const int a = (int)(m % (amax + 1)), c2 = (int)(m / (amax + 1));
@@ -545,16 +814,10 @@ __device__ __attribute__((always_inline)) inline void k_bc_faces_body(const Face
         if (dir == 0) { x1 = g1; x2 = g2; y1 = y2 = a; z1 = z2 = c2; }
         else if (dir == 1) { y1 = g1; y2 = g2; x1 = x2 = a; z1 = z2 = c2; }
         else { z1 = g1; z2 = g2; x1 = x2 = a; y1 = y2 = c2; }
-        face_step<T, 0>(A, f, x1, y1, z1, true, v1);
-        face_step<T, 0>(A, f, x2, y2, z2, false, v2);
-        const long E = d.E, q1 = ix(d, x1, y1, z1), q2 = ix(d, x2, y2, z2);
-#pragma unroll
-        for (int n = 0; n < 5; n++) {
-          A.s.w[n * E + q2] = v2.w[n];
-          A.s.w[n * E + q1] = v1.w[n];
-        }
-        A.s.p[q2] = v2.p;
-        A.s.p[q1] = v1.p;
+        face_step<T, 0>(A, src, f, x1, y1, z1, true, v1);
+        face_step<T, 0>(A, src, f, x2, y2, z2, false, v2);
+        put_cell(A.s, d.E, ix(d, x2, y2, z2), v2);
+        put_cell(A.s, d.E, ix(d, x1, y1, z1), v1);
       }
       __syncthreads();
     }
@@ -564,31 +827,33 @@ __device__ __attribute__((always_inline)) inline void k_bc_faces_body(const Face
     k_bc_cut_body(A.cut, (int)(bx - A.nfb), 0, 0);
     return;
   }
-  const long t = (long)bx * blockDim.x + threadIdx.x;
-  int x, y, z;
-  if (!shell_cell_by_depth(d, t, x, y, z)) return;
-  if (last_face(A, x, y, z) == 0) return;
-  CellV<T> o;
-  face_chain<T, 3>(A, x, y, z, true, o);
-  const long q = ix(d, x, y, z), E = d.E;
-  for (int n = 0; n < 5; n++) A.s.w[n * E + q] = o.w[n];
-  A.s.p[q] = o.p;
+  faces_cells(A, src, bx);
 }
 MGE_ENTRY_T(k_bc_faces, FacesArgs, 256, 1)
 
-// the ordered edge extrapolation of bc_corner.f90 (one target cell)
+// The update of a smoothed stage with bc_cutcell and bcond in the same
+// launch: the ghost and mirror cells read only interior cells, which their
+// threads update for themselves (SrcUpd) instead of waiting for the update's
+// launch.  Their blocks come first, being the longer ones.  6-8 us on levels
+// of up to 48^3 cells (before: an update of 3-7 us, then a boundary launch of
+// 10-15 us), 25 us on 96^3 (18 + 18 us).
 template <typename T>
-__device__ inline void edge_fill(const Dims &d, State<T> s, T gamma, const Inf<T> &f, int ti, int tj, int tk, int ai,
-                                 int aj, int ak, int bi, int bj, int bk, int ci, int cj, int ck) {
-  const long E = d.E;
-  long qt = ix(d, ti, tj, tk), qa = ix(d, ai, aj, ak), qb = ix(d, bi, bj, bk), qc = ix(d, ci, cj, ck);
-  T v[5];
-  for (int n = 0; n < 5; n++) {
-    v[n] = s.w[n * E + qa] + s.w[n * E + qb] - s.w[n * E + qc];
-    s.w[n * E + qt] = v[n];
+struct UpdFacesArgs {
+  FacesArgs<T> f;
+  UpdArgs<T> u;
+  long nb0;   // blocks of the faces and the records
+};
+template <typename T>
+__device__ __attribute__((always_inline)) inline void k_update_faces_body(const UpdFacesArgs<T> &A, int bx, int, int) {
+  if (bx >= A.nb0) {
+    k_update_ghost_body(A.u, (int)(bx - A.nb0), 0, 0);
+  } else if (bx >= A.f.nfb) {
+    bc_cut_cells(A.f.cut, SrcUpd<T>{A.u}, (int)(bx - A.f.nfb));
+  } else {
+    faces_cells(A.f, SrcUpd<T>{A.u}, bx);
   }
-  s.p[qt] = eos_st(gamma, f, v);
 }
+MGE_ENTRY_T(k_update_faces, UpdFacesArgs, 256, 1)
 
 // bc_corner.f90:23-157.  Every edge cell of the first ghost layer is
 // t = a + b - c of three cells that no edge writes (face ghosts and interior
@@ -702,6 +967,84 @@ __device__ __attribute__((always_inline)) inline void k_bc_corner_body(const Cor
   s.p[qt] = eos_st(C.gamma, C.inf, v);
 }
 MGE_ENTRY_T(k_bc_corner, CornerArgs, 256, 1)
+
+// The edge and corner cells of the shell where all six faces are written and
+// no direction has one cell, in one launch after the faces' own cells: the
+// chain of faces for the cells bc_corner leaves, its extrapolation for the
+// others.  The i-edge at (je, 1), which reads its own target, and the corner
+// cells that read it take its chain value here, so no thread reads a cell
+// another one writes.
+template <typename T>
+__device__ __attribute__((always_inline)) inline void k_bc_edges_body(const FacesArgs<T> &A, int bx, int, int) {
+  const Dims &d = A.d;
+  const SrcState<T> src{A.s.w, A.s.p, d.E};
+  int x, y, z;
+  if (!shell_cell_by_depth(d, face_cells(d) + bx * (long)blockDim.x + threadIdx.x, x, y, z)) return;
+  const int il = d.il, jl = d.jl, kl = d.kl, ie = d.ie, je = d.je, ke = d.ke;
+  const T gamma = (T)A.gamma;
+  // first-layer ghost index per direction (0 interior or second layer)
+  const bool g0 = x == 1 || x == ie, g1 = y == 1 || y == je, g2 = z == 1 || z == ke;
+  const int nx = x == 1 ? 2 : il, ny = y == 1 ? 2 : jl, nz = z == 1 ? 2 : kl;
+  const int ng = (x < 2 || x > il) + (y < 2 || y > jl) + (z < 2 || z > kl);
+  const bool corner = g0 && g1 && g2, iedge = g1 && g2 && !corner;
+  const bool kjedge = ng == 2 && g0 && (g1 || g2);   // k- and j-edges, interior third index
+  const bool self = g1 && g2 && y == je && z == 1;   // the i-edge that reads its own target, and its corners
+  const bool out = iedge && !self && (x < 2 || x > il);
+  const bool plain = !(corner || iedge || kjedge);
+  // the chain values this cell needs: its own (plain), the self-reading edge
+  // cell's, the two neighbours of an i-edge cell beyond an i face (cells of
+  // this launch), and its own for the far-field branch that the second
+  // layer's cells read at a first-layer cell whose value is extrapolated
+  CellV<T> o, a{}, b{}, c;
+#pragma unroll 1
+  for (int t = 0; t < 3; t++) {
+    const bool need = t == 0 ? plain || self || out : (t == 1 ? out : !plain && A.ffdec && !*A.frozen);
+    if (!need) continue;
+    const int ci = self && corner && t == 0 ? nx : x;
+    const int cj = out && t == 0 ? ny : y, ck = out && t == 1 ? nz : z;
+    face_chain_any(A, src, ci, cj, ck, t == 2 || (t == 0 && (plain || (self && !corner))), o);
+    if (t == 0) a = o;
+    if (t == 1) b = o;
+  }
+  auto at = [&](int i, int j, int k, CellV<T> &v) { src.load(ix(d, i, j, k), v); };
+  auto sum = [&](CellV<T> &v) {
+#pragma unroll
+    for (int n = 0; n < 5; n++) v.w[n] = a.w[n] + b.w[n] - c.w[n];
+  };
+  if (plain) {
+    o = a;
+  } else if (kjedge) {
+    at(nx, y, z, a);
+    at(x, g1 ? ny : y, g1 ? z : nz, b);
+    at(nx, g1 ? ny : y, g1 ? z : nz, c);
+    sum(o);
+  } else {
+    // the i-edge cell (i, y, z) (bc_corner.f90:101-137): this one, or the corner's neighbour
+    const int i = corner ? nx : x;
+    at(i, ny, nz, c);
+    if (self) {
+      b = c;
+    } else if (!out) {
+      at(i, ny, z, a);
+      at(i, y, nz, b);
+    }
+    sum(o);
+    if (corner) {  // from its three edge cells
+      const T two = T(2), three = T(3);
+      CellV<T> ej, ek;
+      at(nx, ny, z, a);
+      at(x, ny, nz, b);
+      sum(ej);
+      at(nx, y, nz, a);
+      sum(ek);
+#pragma unroll
+      for (int n = 0; n < 5; n++) o.w[n] = (o.w[n] + ej.w[n] + ek.w[n]) * two / three - c.w[n];
+    }
+  }
+  if (!plain) o.p = eos_st(gamma, A.inf, o.w);
+  put_cell(A.s, d.E, ix(d, x, y, z), o);
+}
+MGE_ENTRY_T(k_bc_edges, FacesArgs, 256, 1)
 
 // ------------------------------------------------------------------ misc kernels
 

@@ -89,7 +89,6 @@ struct Level {
   std::vector<double> hv[3];
   uint8_t *ffdec = nullptr;  // far-field branch per ghost point of the six faces (ffreeze > 0)
   unsigned long long *lim = nullptr;  // limiter words per direction and cell (Roe r2, lfreeze > 0)
-  long ffoff[7] = {0, 0, 0, 0, 0, 0, 0};
   void *rw[3] = {nullptr, nullptr, nullptr}, *pw[3] = {nullptr, nullptr, nullptr};
   uint8_t *flags = nullptr, *marker = nullptr;
   void *dx = nullptr, *dy = nullptr, *dz = nullptr;
@@ -395,29 +394,19 @@ bool ghosts_rewritten(const Level &L) {
   return all;
 }
 
-// Of the kernels a steady Euler solve runs between two bcond calls on a
-// level, none reads a ghost cell with two or three ghost indices (the edge
-// and corner cells bc_corner writes): the stage kernels, the time step and
-// the smoothing read along one axis at a time, the faces' chains start from
-// interior cells when all six faces are written, and the cut-cell clouds are
-// interior.  There a stage's bcond leaves bc_corner for later and marks the
-// level; the corners are formed (from the faces as they stand, the values
-// bcond.f90:42 would have formed after the last stage) before anything that
-// does read them: the prolongation from the level, the copy ws of the state,
-// the end of a cycle, and the host reading the state.
-bool corners_lazy(const mge_case *h, const Level &L) {
-  return h->lazy_corners && h->prm.eqntype == 0 && ghosts_rewritten(L);
-}
-
-// bc_corner.f90 on buffer buf of the level (no blocks unless run)
-template <class T>
-void launch_corners(mge_case *h, Level &L, int buf, bool run) {
-  const Dims &d = L.d;
-  const mge_params &P = h->prm;
-  const int items = 4 * (d.kl - 1) + 4 * (d.jl - 1) + 4 * (d.ib + 1) + 8;
-  LAUNCHT(h, "k_bc_corner", k_bc_corner, T, run ? dim3((items + 255) / 256) : dim3(0), dim3(256),
-          (CornerArgs<T>{L.d, stm<T>(L, buf), (T)P.gamma, make_inf<T>(P)}));
-}
+// Of the kernels a solve runs between two bcond calls on a level, none reads
+// a ghost cell with two or three ghost indices (an edge or corner cell of the
+// shell), except that the viscous stencils read the edge cells bc_corner
+// extrapolates: the stage kernels, the time step and the smoothing read along
+// one axis at a time, the faces' chains start from interior cells when all
+// six faces are written, and the cut-cell clouds are interior.  There bcond
+// writes the faces' own cells (laminar: and those edge cells, in the same
+// launch) and leaves the others to k_bc_edges, marking the level; it runs
+// (from the faces as they stand, the values bcond.f90:16-42 would have formed
+// after the last stage) before anything that does read them: the prolongation
+// from the level, the copy ws of the state, the end of a cycle, and the host
+// reading the state.
+bool corners_lazy(const mge_case *h, const Level &L) { return h->lazy_corners && ghosts_rewritten(L); }
 
 template <class T>
 CutArgs<T> cut_args(mge_case *h, Level &L, int buf) {
@@ -437,16 +426,17 @@ CutArgs<T> cut_args(mge_case *h, Level &L, int buf) {
   return C;
 }
 
-// bcond; with `cut`, bc_cutcell's records go into the faces' launch; with
-// `lazy`, bc_corner is left for ensure_corners
+// the six faces' arguments on buffer buf; returns < 0 on a bad face, else
+// the warning code
 template <class T>
-int do_bcond(mge_case *h, Level &L, int buf, const CutArgs<T> *cut = nullptr, bool lazy = false) {
+int faces_args(mge_case *h, Level &L, int buf, bool lazy, FacesArgs<T> *out) {
   const mge_params &P = h->prm;
-  int warn = MGE_OK;
-  FacesArgs<T> F{};
-  F.d = L.d;
+  const Dims &d = L.d;
+  int warn = MGE_OK, active = 0;
+  FacesArgs<T> &F = *out;
+  F = FacesArgs<T>{};
+  F.d = d;
   F.s = stm<T>(L, buf);
-  int active = 0;
   for (int f = 1; f <= 6; f++) {
     int t = L.bctype[f - 1];
     if (t == 0 || (t != -20 && t != -50 && t != -60 && t != -80)) {
@@ -455,33 +445,68 @@ int do_bcond(mge_case *h, Level &L, int buf, const CutArgs<T> *cut = nullptr, bo
     }
     if (t == -60 && f <= 3 && L.bctype[f + 2] != -60)
       return set_err(MGE_ERR_PERIODIC, "Periodic boundary must appear in pairs");
-    F.kind[f - 1] = t;
-    F.ffdec[f - 1] = (t == -20 && L.ffdec) ? L.ffdec + L.ffoff[f - 1] : nullptr;
+    const unsigned kind = t == -20 ? FACE_FAR : (t == -50 ? FACE_SYM : (t == -60 ? FACE_PER : FACE_WALL));
+    F.kinds |= kind << (4 * (f - 1));
+    if (kind == FACE_WALL) F.wall = 1;
     active++;
   }
-  F.seq = (L.d.ni < 2 || L.d.nj < 2 || L.d.nk < 2) ? 1 : 0;
+  F.seq = (d.ni < 2 || d.nj < 2 || d.nk < 2) ? 1 : 0;
   F.gamma = P.gamma; F.rho0 = P.rho0; F.p0 = P.p0; F.c0 = P.c0;
   F.s0 = std::pow(P.rho0, P.gamma) / P.p0;
+  F.gm = 1.0 / (P.gamma - 1.0);
+  F.rgamma = 1.0 / P.gamma;
+  F.rinf = 2.0 * P.c0 / (P.gamma - 1.0);
+  F.air = std::fabs(P.gamma - 1.4) < 1e-15;
   F.u0 = P.u0; F.v0 = P.v0; F.w0 = P.w0;
   F.inf = make_inf<T>(P);
   F.frozen = h->ffrozen;
-  {
-    F.nfb = active == 0 ? 0 : (F.seq ? 1 : (shell_cells(L.d) + 255) / 256);
-    long ncb = 0;
-    if (cut) {
-      F.cut = *cut;
-      ncb = (cut->nmir + 255) / 256;
-    }
-    LAUNCHT(h, "k_bc_faces", k_bc_faces, T, dim3((unsigned)(F.nfb + ncb)), dim3(256), F);
+  F.ffdec = L.ffdec;
+  F.nt = ghosts_rewritten(L) ? face_cells(d) : shell_cells(d);
+  F.ned = lazy && P.eqntype == 1 ? 4L * (d.ni + d.nj + d.nk) : 0;
+  F.nfb = active == 0 ? 0 : (F.seq ? 1 : (F.nt + F.ned + 255) / 256);
+  return warn;
+}
+
+// the edge and corner cells after the faces, on buffer buf (no blocks unless
+// run): bc_corner.f90, and with it the rest of the shell where the faces'
+// launch leaves that to it
+template <class T>
+void launch_corners(mge_case *h, Level &L, int buf, bool run) {
+  const Dims &d = L.d;
+  const mge_params &P = h->prm;
+  if (ghosts_rewritten(L)) {
+    FacesArgs<T> F{};
+    if (run) faces_args<T>(h, L, buf, false, &F);
+    const long n = shell_cells(d) - face_cells(d);
+    LAUNCHT(h, "k_bc_corner", k_bc_edges, T, run ? flat_grid(n) : dim3(0), dim3(256), F);
+    return;
   }
+  const int items = 4 * (d.kl - 1) + 4 * (d.jl - 1) + 4 * (d.ib + 1) + 8;
+  LAUNCHT(h, "k_bc_corner", k_bc_corner, T, run ? dim3((items + 255) / 256) : dim3(0), dim3(256),
+          (CornerArgs<T>{L.d, stm<T>(L, buf), (T)P.gamma, make_inf<T>(P)}));
+}
+
+// bcond; with `cut`, bc_cutcell's records go into the faces' launch; with
+// `lazy`, the edge and corner cells are left for ensure_corners
+template <class T>
+int do_bcond(mge_case *h, Level &L, int buf, const CutArgs<T> *cut = nullptr, bool lazy = false) {
+  FacesArgs<T> F;
+  const int warn = faces_args<T>(h, L, buf, lazy, &F);
+  if (warn < 0) return warn;
+  long ncb = 0;
+  if (cut) {
+    F.cut = *cut;
+    ncb = (cut->nmir + kCutRecs - 1) / kCutRecs;
+  }
+  LAUNCHT(h, "k_bc_faces", k_bc_faces, T, dim3((unsigned)(F.nfb + ncb)), dim3(256), F);
   launch_corners<T>(h, L, buf, !lazy);
   L.corner_stale = lazy;
   return warn;
 }
 
-// bc_corner on the level's current state if a lazy bcond left it (a launch
-// with no blocks otherwise, so that every case of a batch records the same
-// launches)
+// the edge and corner cells of the level's current state if a lazy bcond left
+// them (a launch with no blocks otherwise, so that every case of a batch
+// records the same launches)
 template <class T>
 void ensure_corners(mge_case *h, Level &L) {
   launch_corners<T>(h, L, L.cur, L.corner_stale);
@@ -491,28 +516,61 @@ void ensure_corners(mge_case *h, Level &L) {
 template <class T>
 int do_bc_cutcell(mge_case *h, Level &L, int buf) {
   if (L.nmir == 0) {
-    LAUNCHT(h, "k_bc_cut", k_bc_cut, T, dim3(0), dim3(64), CutArgs<T>{});
+    LAUNCHT(h, "k_bc_cut", k_bc_cut, T, dim3(0), dim3(256), CutArgs<T>{});
     return MGE_OK;
   }
-  LAUNCHT(h, "k_bc_cut", k_bc_cut, T, dim3((L.nmir + 63) / 64), dim3(64), cut_args<T>(h, L, buf));
+  LAUNCHT(h, "k_bc_cut", k_bc_cut, T, dim3((L.nmir + kCutRecs - 1) / kCutRecs), dim3(256), cut_args<T>(h, L, buf));
   return L.zero_at >= 0 ? MGE_WARN_ZERO_CLOUD : MGE_OK;
+}
+
+// the update of a smoothed stage: with the stage's bc_cutcell and bcond in
+// its launch (true) where the boundary reads interior cells only and leaves
+// the edges for later, else by itself
+template <class T>
+int do_update(mge_case *h, Level &L, const UpdArgs<T> &U, int buf, bool *with_bc, int *warn) {
+  const dim3 gu = flat_grid(L.d.E);
+  *with_bc = corners_lazy(h, L);
+  if (!*with_bc) {
+    LAUNCHT(h, "k_update_ghost", k_update_ghost, T, gu, dim3(256), U);
+    return MGE_OK;
+  }
+  UpdFacesArgs<T> A{};
+  const int rc = faces_args<T>(h, L, buf, true, &A.f);
+  if (rc < 0) return rc;
+  if (rc > 0) *warn = rc;
+  A.u = U;
+  A.nb0 = A.f.nfb;
+  if (L.nmir > 0) {
+    A.f.cut = cut_args<T>(h, L, buf);
+    A.nb0 += (L.nmir + kCutRecs - 1) / kCutRecs;
+    if (L.zero_at >= 0) *warn = MGE_WARN_ZERO_CLOUD;
+  }
+  LAUNCHT(h, "k_update_ghost", k_update_faces, T, dim3((unsigned)(A.nb0 + gu.x)), dim3(256), A);
+  return MGE_OK;
 }
 
 // bc_cutcell then bcond, as each RK stage ends (euler.f90): one launch for
 // both when the level's clouds lie in the interior and its faces run in
-// parallel (k_bc_cut keeps its place in the sequence with no blocks, so
-// every case of a batch records the same launches)
+// parallel, none when the update's launch held them (`done`); launches with
+// no blocks keep the sequence, so that every case of a batch records the
+// same one
 template <class T>
-int do_cut_bcond(mge_case *h, Level &L, int buf, int *warn) {
+int do_cut_bcond(mge_case *h, Level &L, int buf, bool done, int *warn) {
   const Dims &d = L.d;
   const bool seq = d.ni < 2 || d.nj < 2 || d.nk < 2;
   const bool lazy = corners_lazy(h, L);
-  if (L.nmir == 0 || !L.cut_interior || seq) {
+  if (!done && (L.nmir == 0 || !L.cut_interior || seq)) {
     int rc = do_bc_cutcell<T>(h, L, buf);
     if (rc > 0) *warn = rc;
     return do_bcond<T>(h, L, buf, nullptr, lazy);
   }
-  LAUNCHT(h, "k_bc_cut", k_bc_cut, T, dim3(0), dim3(64), CutArgs<T>{});
+  LAUNCHT(h, "k_bc_cut", k_bc_cut, T, dim3(0), dim3(256), CutArgs<T>{});
+  if (done) {
+    LAUNCHT(h, "k_bc_faces", k_bc_faces, T, dim3(0), dim3(256), FacesArgs<T>{});
+    launch_corners<T>(h, L, buf, false);
+    L.corner_stale = true;
+    return MGE_OK;
+  }
   if (L.zero_at >= 0) *warn = MGE_WARN_ZERO_CLOUD;
   const CutArgs<T> C = cut_args<T>(h, L, buf);
   return do_bcond<T>(h, L, buf, &C, lazy);
@@ -816,6 +874,7 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       LAUNCHT(h, "k_rec", k_rec, T, dim3((unsigned)L.nchunk), dim3(kRecOps), R);
     }
     if (lres) return MGE_OK;
+    bool bc_done = false;
     if (A.smoothed && P.smoother == 1) {
       // psmoo with progon3's sweep: x, y, then z lines (psmoo.f90:40-87)
       PsmooArgs<T> S{d, dwp, tp<T>(L.eps), tp<T>(L.eps) + 3 * E};
@@ -834,7 +893,7 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       U.dtstep = A.dtstep;
       U.vt = A.vt;
       U.carry = ghosts_rewritten(L) ? 0 : 1;
-      LAUNCHT(h, "k_update_ghost", k_update_ghost, T, flat_grid(E), dim3(256), U);
+      CHKRC(do_update<T>(h, L, U, dst, &bc_done, &warn));
     } else if (A.smoothed) {
       SmoothArgs<T> S;
       S.d = d;
@@ -874,7 +933,7 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       U.dtstep = A.dtstep;
       U.vt = A.vt;
       U.carry = ghosts_rewritten(L) ? 0 : 1;
-      LAUNCHT(h, "k_update_ghost", k_update_ghost, T, flat_grid(E), dim3(256), U);
+      CHKRC(do_update<T>(h, L, U, dst, &bc_done, &warn));
     } else {
       // the ghost shell of the new state is the old one until bcond; when
       // bcond rewrites every ghost cell nothing reads the copy and it is
@@ -882,7 +941,7 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       LAUNCHT(h, "k_ghost_copy", k_ghost_copy, T, ghosts_rewritten(L) ? dim3(0) : flat_grid(shell_cells(d)), dim3(256),
               (GhostArgs<T>{d, stc<T>(L, src), stm<T>(L, dst)}));
     }
-    int rc = do_cut_bcond<T>(h, L, dst, &warn);
+    int rc = do_cut_bcond<T>(h, L, dst, bc_done, &warn);
     if (rc < 0) return rc;
     if (rc > 0) warn = rc;
     src = dst;
@@ -921,7 +980,7 @@ bool levels_nest(const Level &c, const Level &f) {
 
 // the grid of a transfer onto level L that also forms p on every cell of L
 // (XferArgs::eos): the cells' grid and then enough z-slices of blocks for
-// the ghost shell
+// the ghost shell, unless the bcond that follows rewrites all of it
 template <class T>
 dim3 xfer_eos_grid(XferArgs<T> &X, Level &L, const mge_params &P, dim3 g) {
   const long per = (long)g.x * g.y * 256;
@@ -932,6 +991,7 @@ dim3 xfer_eos_grid(XferArgs<T> &X, Level &L, const mge_params &P, dim3 g) {
   X.gx = (int)g.x;
   X.gy = (int)g.y;
   X.gz0 = (int)g.z;
+  if (ghosts_rewritten(L)) return g;
   return dim3(g.x, g.y, g.z + (unsigned)((shell_cells(L.d) + per - 1) / per));
 }
 
@@ -964,7 +1024,7 @@ int do_movco(mge_case *h, int mgl) {
   // past its grid the ghost shell's (the EOS pass over the level)
   const dim3 gr = xfer_eos_grid(X, c, h->prm, cell_grid(c.d));
   LAUNCHT(h, "k_restrict", k_restrict, T, gr, cell_block(), X);
-  return do_bcond<T>(h, c, c.cur);
+  return do_bcond<T>(h, c, c.cur, nullptr, corners_lazy(h, c));
 }
 
 template <class T>
@@ -1007,7 +1067,7 @@ int do_movfin(mge_case *h, int mgl, int mlvl) {
     const dim3 gp = xfer_eos_grid(X, f, h->prm, cell_grid(f.d));
     LAUNCHT(h, "k_prolong", k_prolong, T, gp, cell_block(), X);
   }
-  return do_bcond<T>(h, f, f.cur);
+  return do_bcond<T>(h, f, f.cur, nullptr, corners_lazy(h, f));
 }
 
 // unsteady: both earlier physical time levels start from the current state
@@ -1023,6 +1083,11 @@ int init_time_levels(mge_case *h, Level &L) {
 int shift_time_levels(mge_case *h) {
   for (int l = 1; l <= h->nlevel; l++) {
     Level &L = h->lv[l];
+    if (L.corner_stale)
+      by_type(h, [&](auto z) {
+        ensure_corners<decltype(z)>(h, L);
+        return MGE_OK;
+      });
     const size_t n = h->es * 5 * (size_t)L.d.E;
     HIPCHK(hipMemcpyAsync(L.w2, L.w1, n, hipMemcpyDeviceToDevice, h->stream));
     HIPCHK(hipMemcpyAsync(L.w1, L.S[L.cur], n, hipMemcpyDeviceToDevice, h->stream));
@@ -2018,12 +2083,9 @@ int mge_level_define(mge_case *h, int lvl, int ni, int nj, int nk, const double 
   CHKRC(dalloc(L, &L.rtrms, L.mxcyc + 1));
   CHKRC(dalloc(L, &L.force, 3));
   if (h->prm.ffreeze > 0.0) {
-    for (int f = 1; f <= 6; f++) {
-      const int dir = (f - 1) % 3;
-      const long amax = dir == 0 ? d.jb : d.ib, cmax = dir == 2 ? d.jb : d.kb;
-      L.ffoff[f] = L.ffoff[f - 1] + (amax + 1) * (cmax + 1);
-    }
-    CHKRC(dalloc(L, &L.ffdec, L.ffoff[6]));
+    // the two faces of each direction, whole with their edges
+    const long nj4 = d.jb + 1, nk4 = d.kb + 1;
+    CHKRC(dalloc(L, &L.ffdec, 2 * (nj4 * nk4 + d.sy * nk4 + d.sz)));
   }
   if (h->prm.lfreeze > 0.0 && h->prm.distype == 2) {
     // every byte starts "not recorded" (255): the ghost cells, whose values
@@ -2786,6 +2848,9 @@ int mge_set_kc(mge_case *h, int lvl, int kc) {
 
 int mge_set_freeze(mge_case *h, int far, int lim) {
   if (!h) return set_err(MGE_ERR_ARG, "null handle");
+  // cells awaiting k_bc_edges take the branch their bcond would have taken
+  for (int l = 1; l <= h->nlevel; l++)
+    if (h->lv[l].defined) sync_corners(h, h->lv[l]);
   const int v[2] = {far ? 1 : 0, lim ? 1 : 0};
   HIPCHK(h2d_sync(h->ffrozen, v, sizeof(v), h->stream));
   return MGE_OK;

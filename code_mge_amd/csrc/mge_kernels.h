@@ -72,12 +72,13 @@ __device__ inline bool shell_cell(const Dims &d, long t, int &x, int &y, int &z)
 // layer fastest, j and k faces with it slowest), then the twelve edges' 4 x 4 ghost pairs along their
 // interior, then the 4 x 4 x 4 corner cells.  Consecutive threads then take
 // the same faces, so a wave of k_bc_faces runs one chain shape.
-__host__ __device__ inline bool shell_cell_by_depth(const Dims &d, long t, int &x, int &y, int &z) {
-  const long ni = d.ni, nj = d.nj, nk = d.nk;
-  auto g = [](long m, int e) { return m < 2 ? (int)m : e + (int)m - 2; };
-  long n = 4 * nj * nk;
+template <typename I>
+__host__ __device__ inline bool shell_cell_at(const Dims &d, I t, int &x, int &y, int &z) {
+  const I ni = d.ni, nj = d.nj, nk = d.nk;
+  auto g = [](I m, int e) { return m < 2 ? (int)m : e + (int)m - 2; };
+  I n = 4 * nj * nk;
   if (t < n) {  // the i faces' four layers fastest: a row's ghost cells side by side
-    const long r = t / 4;
+    const I r = t / 4;
     x = g(t % 4, d.ie);
     y = 2 + (int)(r % nj);
     z = 2 + (int)(r / nj);
@@ -86,7 +87,7 @@ __host__ __device__ inline bool shell_cell_by_depth(const Dims &d, long t, int &
   t -= n;
   n = 4 * ni * nk;
   if (t < n) {
-    const long r = t % (ni * nk);
+    const I r = t % (ni * nk);
     y = g(t / (ni * nk), d.je);
     x = 2 + (int)(r % ni);
     z = 2 + (int)(r / ni);
@@ -95,7 +96,7 @@ __host__ __device__ inline bool shell_cell_by_depth(const Dims &d, long t, int &
   t -= n;
   n = 4 * ni * nj;
   if (t < n) {
-    const long r = t % (ni * nj);
+    const I r = t % (ni * nj);
     z = g(t / (ni * nj), d.ke);
     x = 2 + (int)(r % ni);
     y = 2 + (int)(r / ni);
@@ -104,7 +105,7 @@ __host__ __device__ inline bool shell_cell_by_depth(const Dims &d, long t, int &
   t -= n;
   n = 16 * ni;
   if (t < n) {
-    const long m = t / ni;
+    const I m = t / ni;
     x = 2 + (int)(t % ni);
     y = g(m & 3, d.je);
     z = g(m >> 2, d.ke);
@@ -113,7 +114,7 @@ __host__ __device__ inline bool shell_cell_by_depth(const Dims &d, long t, int &
   t -= n;
   n = 16 * nj;
   if (t < n) {
-    const long m = t / nj;
+    const I m = t / nj;
     y = 2 + (int)(t % nj);
     x = g(m & 3, d.ie);
     z = g(m >> 2, d.ke);
@@ -122,7 +123,7 @@ __host__ __device__ inline bool shell_cell_by_depth(const Dims &d, long t, int &
   t -= n;
   n = 16 * nk;
   if (t < n) {
-    const long m = t / nk;
+    const I m = t / nk;
     z = 2 + (int)(t % nk);
     x = g(m & 3, d.ie);
     y = g(m >> 2, d.je);
@@ -136,6 +137,17 @@ __host__ __device__ inline bool shell_cell_by_depth(const Dims &d, long t, int &
     return true;
   }
   return false;
+}
+// (in 32-bit index arithmetic where the block allows it: a 64-bit division is
+// some hundred instructions, and a boundary launch is as long as one thread's)
+__host__ __device__ inline bool shell_cell_by_depth(const Dims &d, long t, int &x, int &y, int &z) {
+  if (d.E <= 0xffffffffL) return shell_cell_at<unsigned>(d, (unsigned)t, x, y, z);
+  return shell_cell_at<long>(d, t, x, y, z);
+}
+
+// how many of those are the faces' own cells (one ghost index), which come first
+__host__ __device__ inline long face_cells(const Dims &d) {
+  return 4L * d.nj * d.nk + 4L * d.ni * d.nk + 4L * d.ni * d.nj;
 }
 
 __host__ __device__ inline long shell_cells(const Dims &d) {

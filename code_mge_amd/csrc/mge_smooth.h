@@ -1,5 +1,5 @@
-// mge_smooth.h -- implicit residual smoothing (psmoo_old.f90) and the
-// post-smoothing update, templated on the bulk type T.
+// mge_smooth.h -- implicit residual smoothing (psmoo_old.f90), templated on
+// the bulk type T.
 //
 // psmoo_old solves, for every grid line and each direction in turn, the
 // constant-coefficient tridiagonal system (1+2 eps) x_s - eps (x_(s-1) +
@@ -483,70 +483,6 @@ __device__ __attribute__((always_inline)) inline void k_smooth_z_body(const Smoo
   smooth_line(S.dw + n * d.E, S.flags, ix(d, i, j, 0), d.sz, d.kl, S.e1, S.r1, S.e2, S.bb);
 }
 MGE_ENTRY_T_XCD(k_smooth_z, SmoothArgs, 64, 1)
-
-// after smoothing: w = wn - dw and the EOS on interior cells
-// (euler.f90:381-399), one thread per cell of the whole array so that the
-// accesses stream through aligned rows; the ghost shell of the previous
-// state is carried over where anything reads it before bcond rewrites it,
-// as k_ghost_copy does on unsmoothed stages
-template <typename T>
-struct UpdArgs {
-  Dims d;
-  const T *wn, *dw;
-  StateC<T> src;
-  State<T> dst;
-  T gamma;
-  Inf<T> inf;
-  // unsteady update on the finest active level: w = wn - dw/lam
-  // (euler.f90:383-393)
-  int ulam;
-  const T *vdtim;
-  const double *dtim;
-  T fn, dtstep;
-  int vt;
-  int carry;   // carry the ghost shell over
-};
-
-template <typename T>
-__device__ __attribute__((always_inline)) inline void k_update_ghost_body(const UpdArgs<T> &U, int bx, int, int) {
-  const Dims &d = U.d;
-  const T *wn = U.wn, *dw = U.dw;
-  const StateC<T> &src = U.src;
-  const State<T> &dst = U.dst;
-  const T gamma = U.gamma;
-  const long q = bx * (long)blockDim.x + threadIdx.x;
-  if (q >= d.E) return;
-  int i, j, k;
-  if (d.E <= 0xffffffffL) {  // 32-bit index arithmetic
-    const unsigned uq = (unsigned)q, sz = (unsigned)d.sz, sy = (unsigned)d.sy;
-    const unsigned kk = uq / sz, r = uq - kk * sz, jj = r / sy;
-    i = (int)(r - jj * sy);
-    j = (int)jj;
-    k = (int)kk;
-  } else {
-    k = (int)(q / d.sz);
-    j = (int)((q - (long)k * d.sz) / d.sy);
-    i = (int)(q - (long)k * d.sz - (long)j * d.sy);
-  }
-  if (!(i >= 2 && i <= d.il && j >= 2 && j <= d.jl && k >= 2 && k <= d.kl)) {
-    if (U.carry) {
-      for (int n = 0; n < 5; n++) dst.w[n * d.E + q] = src.w[n * d.E + q];
-      dst.p[q] = src.p[q];
-    }
-    return;
-  }
-  T v[5];
-  if (U.ulam) {
-    const T lam = unsteady_lam(U.fn, U.vdtim, U.dtim, U.vt, U.dtstep, q);
-    for (int n = 0; n < 5; n++) v[n] = wn[n * d.E + q] - dw[n * d.E + q] / lam;
-  } else {
-    for (int n = 0; n < 5; n++) v[n] = wn[n * d.E + q] - dw[n * d.E + q];
-  }
-  for (int n = 0; n < 5; n++) dst.w[n * d.E + q] = v[n];
-  dst.p[q] = eos_st(gamma, U.inf, v);
-}
-MGE_ENTRY_T(k_update_ghost, UpdArgs, 256, 1)
-
 
 // ---- psmoo (psmoo.f90:1-95) with progon3's sweep (progon3.f90:1-62) ------
 // Rows (1+2e_r) x_r - e_r x_{r-1} - e_r x_{r+1} = d_r along each line of
