@@ -35,6 +35,7 @@
 #include "mge_smooth.h"
 #include "mge_stage.h"
 #include "mge_visc.h"
+#include "mge_xfer.h"
 
 using namespace mge;
 
@@ -163,6 +164,7 @@ struct mge_case {
   std::vector<Level> lv;
   hipStream_t stream = nullptr;
   int *err = nullptr;
+  HostWord *word = nullptr;   // pinned: residual and error flag as last published
   bool timing = false;
   std::vector<Timer> pending;
   std::vector<hipEvent_t> pool;
@@ -352,17 +354,18 @@ Level *get_level(mge_case *h, int lvl) {
   return L->defined ? L : nullptr;
 }
 
-int check_err(mge_case *h) {
+// waits for the case's work; its error flag, and with r the value *r in h->word
+int check_err(mge_case *h, const double *r = nullptr) {
   if (h->launch_err != hipSuccess) {
     char b[256];
     snprintf(b, sizeof b, "kernel launch failed: %s", hipGetErrorString(h->launch_err));
     h->launch_err = hipSuccess;
     return set_err(MGE_ERR_HIP, b);
   }
-  int e = 0;
-  if (hipMemcpyAsync(&e, h->err, sizeof(int), hipMemcpyDeviceToHost, h->stream) != hipSuccess)
-    return set_err(MGE_ERR_HIP, "error-flag copy failed");
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, h->stream, r, (const int *)h->err, h->word);
+  if (hipGetLastError() != hipSuccess) return set_err(MGE_ERR_HIP, "error-flag read failed");
   if (hipStreamSynchronize(h->stream) != hipSuccess) return set_err(MGE_ERR_HIP, "stream sync failed");
+  const int e = h->word->err;
   if (h->timing) resolve_timers(h);
   if (e < 0) {
     const char *m = "device error";
@@ -1203,8 +1206,9 @@ int ffreeze_test(mge_case *h, int mlvl, int ncyc) {
 int read_rtrms(mge_case *h, int mlvl, int ncyc, double *r) {
   Level &B = h->lv[mlvl];
   int c = ncyc >= 1 && ncyc <= B.mxcyc ? ncyc : 0;
-  HIPCHK(hipMemcpyAsync(r, B.rtrms + c, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  return check_err(h);
+  const int e = check_err(h, B.rtrms + c);
+  *r = h->word->r;
+  return e;
 }
 
 // solver.f90:119-261, one physical time step at level itime (steady flow:
@@ -2001,7 +2005,9 @@ int mge_case_create(const mge_params *prm, int nlevel, mge_case **out) {
     return set_err(MGE_ERR_HIP, "hipStreamCreate failed");
   }
   if (hipMalloc(&h->err, sizeof(int)) != hipSuccess || hipMalloc(&h->ffrozen, 2 * sizeof(int)) != hipSuccess ||
-      hipMalloc(&h->ffini, sizeof(double)) != hipSuccess) {
+      hipMalloc(&h->ffini, sizeof(double)) != hipSuccess ||
+      hipHostMalloc((void **)&h->word, sizeof(HostWord), hipHostMallocDefault) != hipSuccess) {
+    if (h->ffini) hipFree(h->ffini);
     if (h->err) hipFree(h->err);
     if (h->ffrozen) hipFree(h->ffrozen);
     hipStreamDestroy(h->stream);
@@ -2011,6 +2017,7 @@ int mge_case_create(const mge_params *prm, int nlevel, mge_case **out) {
   clear_sync(h->err, sizeof(int));
   clear_sync(h->ffrozen, 2 * sizeof(int));
   clear_sync(h->ffini, sizeof(double));
+  xfer_user(1);
   *out = h;
   return MGE_OK;
 }
@@ -2027,8 +2034,10 @@ int mge_case_destroy(mge_case *h) {
   hipFree(h->err);
   hipFree(h->ffrozen);
   hipFree(h->ffini);
+  hipHostFree(h->word);
   hipStreamDestroy(h->stream);
   delete h;
+  xfer_user(-1);
   return MGE_OK;
 }
 
@@ -2214,8 +2223,8 @@ int mge_euler(mge_case *h, int lvl, int blk, int itime, int ncyc, int mgl, int m
   if (rc < 0) return rc;
   if (rtrms && !lres) {
     int c = ncyc >= 1 && ncyc <= L->mxcyc ? ncyc : 0;
-    HIPCHK(hipMemcpyAsync(rtrms, L->rtrms + c, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    int e = check_err(h);
+    int e = check_err(h, L->rtrms + c);
+    *rtrms = h->word->r;
     if (e < 0) return e;
   }
   return rc;
@@ -2347,20 +2356,23 @@ int mge_download(mge_case *h, int lvl, int blk, const char *field, double *out) 
   void *p = field_ptr(*L, h->es, field, &n);
   if (!p) return set_err(MGE_ERR_ARG, "unknown field");
   if (!h->fp32) {
-    HIPCHK(hipMemcpyAsync(out, p, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(xfer(h->dev, h->stream, p, sizeof(double) * n, false,
+                [&](size_t o, const char *t, size_t len) { std::memcpy((char *)out + o, t, len); }));
     return check_err(h);
   }
-  std::vector<float> t(n);
-  HIPCHK(hipMemcpyAsync(t.data(), p, sizeof(float) * n, hipMemcpyDeviceToHost, h->stream));
-  int e = check_err(h);
   const int nc = state_field(field);
   const Inf<float> f = make_inf<float>(h->prm);
   const long E = L->d.E;
-  for (long q = 0; q < n; q++) {
-    double off = nc == 5 ? (double)f.w[q / E] : (nc == 1 ? (double)f.p : 0.0);
-    out[q] = (double)t[q] + off;
-  }
-  return e;
+  HIPCHK(xfer(h->dev, h->stream, p, sizeof(float) * n, false, [&](size_t o, const char *t, size_t len) {
+    const float *v = (const float *)t;
+    const long q0 = (long)(o / sizeof(float)), q1 = q0 + (long)(len / sizeof(float));
+    for (long q = q0; q < q1;) {  // component by component: one offset each
+      const long c = q / E, qe = std::min(q1, (c + 1) * E);
+      const double off = nc == 5 ? (double)f.w[c] : (nc == 1 ? (double)f.p : 0.0);
+      for (; q < qe; q++) out[q] = (double)v[q - q0] + off;
+    }
+  }));
+  return check_err(h);
 }
 
 int mge_upload(mge_case *h, int lvl, int blk, const char *field, const double *in) {
@@ -2370,17 +2382,23 @@ int mge_upload(mge_case *h, int lvl, int blk, const char *field, const double *i
   long n;
   void *p = field_ptr(*L, h->es, field, &n);
   if (!p) return set_err(MGE_ERR_ARG, "unknown field");
-  HIPCHK(hipStreamSynchronize(h->stream));
+  if (!h->fp32) {
+    HIPCHK(xfer(h->dev, h->stream, p, sizeof(double) * n, true,
+                [&](size_t o, char *t, size_t len) { std::memcpy(t, (const char *)in + o, len); }));
+    return MGE_OK;
+  }
   const int nc = state_field(field);
-  if (!h->fp32 || nc == 0) return put_bulk(h, p, in, n);
   const Inf<float> f = make_inf<float>(h->prm);
   const long E = L->d.E;
-  std::vector<float> t(n);
-  for (long q = 0; q < n; q++) {
-    double off = nc == 5 ? (double)f.w[q / E] : (double)f.p;
-    t[q] = (float)(in[q] - off);
-  }
-  HIPCHK(h2d_sync(p, t.data(), sizeof(float) * n, h->stream));
+  HIPCHK(xfer(h->dev, h->stream, p, sizeof(float) * n, true, [&](size_t o, char *t, size_t len) {
+    float *v = (float *)t;
+    const long q0 = (long)(o / sizeof(float)), q1 = q0 + (long)(len / sizeof(float));
+    for (long q = q0; q < q1;) {
+      const long c = q / E, qe = std::min(q1, (c + 1) * E);
+      const double off = nc == 5 ? (double)f.w[c] : (nc == 1 ? (double)f.p : 0.0);
+      for (; q < qe; q++) v[q - q0] = (float)(in[q] - off);
+    }
+  }));
   return MGE_OK;
 }
 
@@ -2602,7 +2620,9 @@ int do_upload_solut(mge_case *h, Level &L, double ptot, double *host, int nval) 
                  freestream_mach(h->prm), ptot, nval == 11, nc, dev};
   hipLaunchKernelGGL(k_upload_solut<T>, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, h->stream, A);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(host, dev, sizeof(double) * nval * nc, hipMemcpyDeviceToHost, h->stream);
+  if (e == hipSuccess)
+    e = xfer(h->dev, h->stream, dev, sizeof(double) * nval * nc, false,
+             [&](size_t o, const char *t, size_t len) { std::memcpy((char *)host + o, t, len); });
   hipError_t f = hipFreeAsync(dev, h->stream);
   if (e == hipSuccess) e = f;
   if (e != hipSuccess) return set_err(MGE_ERR_HIP, hipGetErrorString(e));
