@@ -94,7 +94,6 @@ struct Level {
   uint8_t *flags = nullptr, *marker = nullptr;
   void *dx = nullptr, *dy = nullptr, *dz = nullptr;
   void *piv = nullptr;  // e1x,e2x,e1y,e2y,e1z,e2z,1/e1x,1/e1y,1/e1z each npiv
-  void *fax = nullptr;  // -bb/e1x
   int npiv = 0;
   int nmir = 0, nupd = 0, zero_at = -1;
   bool cut_interior = false;  // every cloud cell inside the ghost shell (bcond writes none of them)
@@ -528,11 +527,14 @@ int do_bc_cutcell(mge_case *h, Level &L, int buf) {
 
 // the update of a smoothed stage: with the stage's bc_cutcell and bcond in
 // its launch (true) where the boundary reads interior cells only and leaves
-// the edges for later, else by itself
+// the edges for later, else by itself.  Beyond 2^21 cells (128^3) the launch
+// is no longer the cost and the boundary's registers slow the update's
+// streaming: 192^3 FP32 106 us in one, 78 + 22 us apart; 128^3 58 and 44 + 14
+// us FP64; 96^3 26 and 21 + 10 us
 template <class T>
 int do_update(mge_case *h, Level &L, const UpdArgs<T> &U, int buf, bool *with_bc, int *warn) {
   const dim3 gu = flat_grid(L.d.E);
-  *with_bc = corners_lazy(h, L);
+  *with_bc = corners_lazy(h, L) && (long)L.d.ni * L.d.nj * L.d.nk <= 1L << 21;
   if (!*with_bc) {
     LAUNCHT(h, "k_update_ghost", k_update_ghost, T, gu, dim3(256), U);
     return MGE_OK;
@@ -797,6 +799,81 @@ bool stage_gen(const StageArgs<T> &A) {
 
 
 
+// the y (DIR 1) or z (DIR 2) lines of psmoo_old (no blocks unless run)
+template <class T, int DIR>
+void launch_lines(mge_case *h, const char *name, const SmoothArgs<T> &S, bool run) {
+  const Dims &d = S.d;
+  const int n = DIR == 1 ? d.nj : d.nk, other = DIR == 1 ? d.nk : d.nj;
+  const SegShape sh = seg_shape(n);
+  if (!run || sh.sx == 0) {
+    const dim3 g = run ? dim3((d.ni + 63) / 64, other, 5) : dim3(0);
+    if (DIR == 1) LAUNCHT(h, name, k_smooth_y, T, g, dim3(64), S);
+    else LAUNCHT(h, name, k_smooth_z, T, g, dim3(64), S);
+    return;
+  }
+  // threads for the segments of the line, in steps that let a batch's cases share a launch
+  int G = 1;
+  while (G * sh.len < n) G *= 2;
+  const dim3 g((d.ni + sh.sx - 1) / sh.sx, other, 5), b(sh.sx * std::max(G, 64 / sh.sx));
+#define SEGL(SX, N) \
+  launch(h, name, (const void *)&k_smooth_seg<T, SX, N, DIR>, (const void *)&k_smooth_seg_b<T, SX, N, DIR>, g, b, S)
+  if (sh.sx == 64) {
+    if (sh.len == 4) SEGL(64, 4);
+    else if (sh.len == 8) SEGL(64, 8);
+    else SEGL(64, 16);
+  } else if (sh.sx == 32) {
+    if (sh.len == 8) SEGL(32, 8);
+    else SEGL(32, 16);
+  } else {
+    SEGL(16, 16);
+  }
+#undef SEGL
+}
+
+// psmoo_old on dw: x, y, then z lines (three launches recorded whatever the
+// level uses, so that every case of a batch records the same sequence)
+template <class T>
+void do_smooth(mge_case *h, Level &L) {
+  const Dims &d = L.d;
+  SmoothArgs<T> S;
+  S.d = d;
+  S.dw = tp<T>(L.dw);
+  S.flags = L.flags;
+  S.bb = (T)h->smoo_bb;
+  const T *piv = tp<T>(L.piv);
+  const int np = L.npiv;
+  S.e1 = piv;
+  S.e2 = piv + np;
+  S.r1 = piv + 6 * np;
+  const int cls = xy_class(d.ni, d.nj);
+  if (cls >= 0) {
+    SmoothXYArgs<T> A{d, S.dw, S.flags, piv, piv + np, piv + 6 * np, piv + 2 * np, piv + 3 * np, piv + 7 * np, S.bb};
+    const dim3 g(d.nk, 5), b(kXY[cls].threads);
+#define XY(C) launch(h, "k_smooth_x", (const void *)&k_smooth_xy<T, C>, (const void *)&k_smooth_xy_b<T, C>, g, b, A)
+    if (cls == 0) XY(0);
+    else XY(1);
+#undef XY
+  } else {
+    const long nl = (long)d.nj * d.nk;
+#define XSEG(N)                                                                                          \
+  launch(h, "k_smooth_x", (const void *)&k_smooth_xseg<T, N>, (const void *)&k_smooth_xseg_b<T, N>,      \
+         dim3((unsigned)((nl + xseg_rows<N>() - 1) / xseg_rows<N>()), 5), dim3(xseg_rows<N>() * N / 16), S)
+    if (d.ni <= 128) XSEG(128);
+    else if (d.ni <= 256) XSEG(256);
+    else if (d.ni <= 512) XSEG(512);
+    else LAUNCHT(h, "k_smooth_x", k_smooth_x_seq, T, flat_grid(nl * 5), dim3(256), S);
+#undef XSEG
+  }
+  S.e1 = piv + 2 * np;
+  S.e2 = piv + 3 * np;
+  S.r1 = piv + 7 * np;
+  launch_lines<T, 1>(h, "k_smooth_y", S, cls < 0);
+  S.e1 = piv + 4 * np;
+  S.e2 = piv + 5 * np;
+  S.r1 = piv + 8 * np;
+  launch_lines<T, 2>(h, "k_smooth_z", S, true);
+}
+
 // euler.f90; the residual norm only when want_res (a cycle reads it on the
 // finest active level only; its launches then have no blocks elsewhere)
 template <class T>
@@ -898,35 +975,7 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       U.carry = ghosts_rewritten(L) ? 0 : 1;
       CHKRC(do_update<T>(h, L, U, dst, &bc_done, &warn));
     } else if (A.smoothed) {
-      SmoothArgs<T> S;
-      S.d = d;
-      S.dw = dwp;
-      S.flags = L.flags;
-      S.bb = (T)h->smoo_bb;
-      T *piv = tp<T>(L.piv);
-      S.e1 = piv;
-      S.e2 = piv + L.npiv;
-      S.fa = tp<T>(L.fax);
-      S.r1 = piv + 6 * L.npiv;
-      long nwave = (long)d.nj * d.nk * 5;
-      auto gxk = [&](int K) { return dim3((unsigned)(((nwave + K - 1) / K * 64 + 255) / 256)); };
-#define XSCAN(C)                                                                                            \
-  launch(h, "k_smooth_x", (const void *)&k_smooth_x_scan<C, T>, (const void *)&k_smooth_x_scan_b<C, T>,     \
-         gxk(xscan_lines<C>()), dim3(256), S)
-      if (d.ni <= 64) XSCAN(1);
-      else if (d.ni <= 128) XSCAN(2);
-      else if (d.ni <= 256) XSCAN(4);
-      else if (d.ni <= 512) XSCAN(8);
-      else LAUNCHT(h, "k_smooth_x", k_smooth_x_seq, T, flat_grid(nwave), dim3(256), S);
-#undef XSCAN
-      S.e1 = piv + 2 * L.npiv;
-      S.e2 = piv + 3 * L.npiv;
-      S.r1 = piv + 7 * L.npiv;
-      LAUNCHT(h, "k_smooth_y", k_smooth_y, T, dim3((d.ni + 63) / 64, d.nk, 5), dim3(64), S);
-      S.e1 = piv + 4 * L.npiv;
-      S.e2 = piv + 5 * L.npiv;
-      S.r1 = piv + 8 * L.npiv;
-      LAUNCHT(h, "k_smooth_z", k_smooth_z, T, dim3((d.ni + 63) / 64, d.nj, 5), dim3(64), S);
+      do_smooth<T>(h, L);
       UpdArgs<T> U{d, (const T *)tp<T>(L.S[w0]), (const T *)dwp, stc<T>(L, src), stm<T>(L, dst),
                    (T)P.gamma, make_inf<T>(P)};
       U.ulam = A.ulam == 2;
@@ -2083,7 +2132,6 @@ int mge_level_define(mge_case *h, int lvl, int ni, int nj, int nk, const double 
   CHKRC(dalloc_bytes(L, &L.dz, es * nmax));
   L.npiv = nmax;
   CHKRC(dalloc_bytes(L, &L.piv, es * 9 * nmax));
-  CHKRC(dalloc_bytes(L, &L.fax, es * nmax));
   dim3 g = cell_grid(d);
   L.npartial = (long)g.x * g.y * ((g.z + kRtrmsPlanes - 1) / kRtrmsPlanes);
   CHKRC(dalloc(L, &L.partial, L.npartial));
@@ -2153,10 +2201,6 @@ int mge_level_define(mge_case *h, int lvl, int ni, int nj, int nk, const double 
     }
   }
   CHKRC(put_bulk(h, L.piv, piv.data(), piv.size()));
-  std::vector<double> fa(nmax, 0.0);
-  if (h->prm.smoo > 0.0)
-    for (int i = 2; i <= d.il && i < nmax; i++) fa[i] = h->prm.smoo / piv[i];  // -bb/e1, bb = -smoo
-  CHKRC(put_bulk(h, L.fax, fa.data(), nmax));
   // flags: fluid bit with the ghost copies of init_metric.f90:207-218
   std::vector<uint8_t> bl(E, 1);
   auto X = [&](int i, int j, int k) { return ix(d, i, j, k); };

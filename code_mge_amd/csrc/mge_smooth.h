@@ -7,6 +7,8 @@
 // on the line length (psmoo.f90:134-166); blank cells are skipped (their
 // value is kept and they do not feed the recurrence).
 #pragma once
+#include <algorithm>
+
 #include "mge_kernels.h"
 
 namespace mge {
@@ -17,7 +19,6 @@ struct SmoothArgs {
   T *dw;
   const uint8_t *flags;
   const T *e1, *e2;  // pivots of this direction (psmoo.f90:134-166)
-  const T *fa;       // -bb/e1 (x lines: affine-map form of the forward step)
   const T *r1;       // 1/e1, rounded once from the FP64 pivots
   T bb;
 };
@@ -32,180 +33,6 @@ __device__ __attribute__((always_inline)) inline T piv_div(T x, const T *__restr
   if constexpr (kDelta<T>) return x / e1[s];
   else return x * r1[s];
 }
-
-// a lane moves its CPL cells as pairs when CPL is even, the line's first
-// cell (i = 2) sits on a pair boundary (so does every lane's first cell,
-// i0 - 2 being a multiple of CPL) and all its cells are inside the line
-template <int CPL, typename T>
-__device__ __attribute__((always_inline)) inline bool xscan_pairs(const T *row, int i0, int il) {
-  if constexpr (CPL % 2 != 0) return false;
-  else return ((reinterpret_cast<uintptr_t>(row + 2) & (2 * sizeof(T) - 1)) == 0) && i0 + CPL - 1 <= il;
-}
-
-// psmoo.f90:171-188 (x lines): one wavefront per K consecutive (j,k)
-// lines of a component.  Lane l owns CPL consecutive cells of each line, so
-// loads and stores are coalesced.  Both recurrences are first composed as
-// affine maps (forward y_i = A_i y_(i-1) + B_i, backward z_i = C_i z_(i+1)
-// + y_i), scanned across the wave, and then every lane re-evaluates its own
-// cells with the reference formula from the scanned boundary value.  Only
-// the lane-boundary values differ from the sequential evaluation (by a few
-// ulp); blank cells keep their value as in the reference.  The K lines are
-// independent: their loads are in flight together and their shuffles
-// interleave, and the pivots of the lane's cells are loaded once for all K.
-template <int CPL, int K, typename T>
-__device__ __attribute__((always_inline)) inline void smooth_x_scan(const SmoothArgs<T> &S, int bx) {
-  const Dims &d = S.d;
-  const int lane = threadIdx.x & 63;
-  // the wave index is uniform: keep the line arithmetic scalar
-  const int wave = __builtin_amdgcn_readfirstlane((int)((bx * (long)blockDim.x + threadIdx.x) >> 6));
-  const int nl = d.nj * d.nk;
-  const int nlines = nl * 5;
-  const int l0 = wave * K;
-  if (l0 >= nlines) return;  // uniform per wave
-  const int il = d.il, ni = d.ni;
-  const int i0 = 2 + lane * CPL;
-  // pivots: e1 (FP32 divides by it) or 1/e1 (FP64 multiplies), -bb/e1, e2
-  T pv[CPL], pa[CPL], pe2[CPL];
-  bool ok[CPL];
-#pragma unroll
-  for (int c = 0; c < CPL; c++) {
-    const int i = i0 + c;
-    ok[c] = i <= il;
-    const int ic = ok[c] ? i : 2;
-    pv[c] = kDelta<T> ? S.e1[ic] : S.r1[ic];
-    pa[c] = S.fa[ic];
-    pe2[c] = S.e2[ic];
-  }
-  auto pdiv = [](T x, T p) { if constexpr (kDelta<T>) return x / p; else return x * p; };
-  T r[K][CPL];
-  bool fl[K][CPL], lv[K];
-  long base[K], fbase[K];
-#pragma unroll
-  for (int t = 0; t < K; t++) {
-    lv[t] = l0 + t < nlines;
-    const int lc = lv[t] ? l0 + t : l0;  // a missing line repeats the first; it is never stored
-    const int n = lc / nl;
-    const int l = lc - n * nl;
-    const int j = 2 + l % d.nj, k = 2 + l / d.nj;
-    fbase[t] = ix(d, 0, j, k);
-    base[t] = (long)n * d.E + fbase[t];
-    if (xscan_pairs<CPL>(S.dw + base[t], i0, il)) {
-      const Pair<T> *pp = reinterpret_cast<const Pair<T> *>(S.dw + base[t] + i0);
-#pragma unroll
-      for (int h = 0; h < CPL / 2; h++) {
-        const Pair<T> v = pp[h];
-        r[t][2 * h] = v.x;
-        r[t][2 * h + 1] = v.y;
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < CPL; c++) r[t][c] = ok[c] ? S.dw[base[t] + i0 + c] : T(0);
-    }
-#pragma unroll
-    for (int c = 0; c < CPL; c++) fl[t][c] = ok[c] && (S.flags[fbase[t] + i0 + c] & F_FLUID);
-  }
-  // forward: lane composite of y_i = A_i y_(i-1) + B_i
-  T Al[K], Bl[K];
-#pragma unroll
-  for (int t = 0; t < K; t++) {
-    Al[t] = T(1);
-    Bl[t] = T(0);
-#pragma unroll
-    for (int c = 0; c < CPL; c++) {
-      const int i = i0 + c;
-      T A, B;
-      if (!ok[c]) { A = T(1); B = T(0); }
-      else if (!fl[t][c]) { A = T(0); B = r[t][c]; }
-      else if (i == 2) { A = T(0); B = pdiv(r[t][c], pv[c]); }
-      else { A = pa[c]; B = pdiv(r[t][c], pv[c]); }
-      Bl[t] = A * Bl[t] + B;
-      Al[t] = A * Al[t];
-    }
-  }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-#pragma unroll
-    for (int t = 0; t < K; t++) {
-      T Ap = __shfl_up(Al[t], off, 64), Bp = __shfl_up(Bl[t], off, 64);
-      if (lane >= off) {
-        Bl[t] = Al[t] * Bp + Bl[t];
-        Al[t] = Al[t] * Ap;
-      }
-    }
-  }
-  // re-evaluate the lane's cells from the incoming value (y kept in r)
-#pragma unroll
-  for (int t = 0; t < K; t++) {
-    T yp = __shfl_up(Bl[t], 1, 64);
-    if (lane == 0) yp = T(0);
-#pragma unroll
-    for (int c = 0; c < CPL; c++) {
-      const int i = i0 + c;
-      T v = r[t][c];
-      if (ok[c] && fl[t][c]) v = (i == 2) ? pdiv(r[t][c], pv[c]) : pdiv(r[t][c] - S.bb * yp, pv[c]);
-      r[t][c] = v;
-      yp = v;
-    }
-  }
-  // backward: z_i = C_i z_(i+1) + y_i, C_i = -e2_i on fluid cells 2..ni
-  T Cl[K], Dl[K];
-#pragma unroll
-  for (int t = 0; t < K; t++) {
-    Cl[t] = T(1);
-    Dl[t] = T(0);
-#pragma unroll
-    for (int c = CPL - 1; c >= 0; c--) {
-      const int i = i0 + c;
-      T C, Dv;
-      if (!ok[c]) { C = T(1); Dv = T(0); }
-      else if (fl[t][c] && i <= ni) { C = -pe2[c]; Dv = r[t][c]; }
-      else { C = T(0); Dv = r[t][c]; }
-      Dl[t] = C * Dl[t] + Dv;
-      Cl[t] = C * Cl[t];
-    }
-  }
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-#pragma unroll
-    for (int t = 0; t < K; t++) {
-      T Cn = __shfl_down(Cl[t], off, 64), Dn = __shfl_down(Dl[t], off, 64);
-      if (lane + off < 64) {
-        Dl[t] = Cl[t] * Dn + Dl[t];
-        Cl[t] = Cl[t] * Cn;
-      }
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < K; t++) {
-    T zn = __shfl_down(Dl[t], 1, 64);
-    if (lane == 63) zn = T(0);
-#pragma unroll
-    for (int c = CPL - 1; c >= 0; c--) {
-      const int i = i0 + c;
-      if (!ok[c]) continue;
-      if (fl[t][c] && i <= ni) r[t][c] = r[t][c] - pe2[c] * zn;
-      zn = r[t][c];
-    }
-    if (!lv[t]) continue;
-    if (xscan_pairs<CPL>(S.dw + base[t], i0, il)) {
-      // blank cells are written back with the value they were read with
-      Pair<T> *pp = reinterpret_cast<Pair<T> *>(S.dw + base[t] + i0);
-#pragma unroll
-      for (int h = 0; h < CPL / 2; h++) pp[h] = Pair<T>{r[t][2 * h], r[t][2 * h + 1]};
-    } else {
-#pragma unroll
-      for (int c = 0; c < CPL; c++)
-        if (fl[t][c]) S.dw[base[t] + i0 + c] = r[t][c];
-    }
-  }
-}
-
-// lines per wave of the x scan: four lines of up to 256 cells share a
-// wave, 512-cell lines take one (measured at 256^3 with single loads: one,
-// two and four lines per wave give 527, 512 and 477 us in FP64, 409, 339
-// and 324 us in FP32; with pairs, four lines 408 us FP64, 298 us FP32)
-template <int CPL>
-constexpr int xscan_lines() { return CPL >= 8 ? 1 : 4; }
 
 // sequential x lines for blocks wider than 512 cells
 template <typename T>
@@ -228,22 +55,6 @@ __device__ __attribute__((always_inline)) inline void smooth_x_seq(const SmoothA
   }
 }
 
-// x-line entry points: one per scan width (cells per lane, chosen from
-// the line length) and the sequential form; a batch launches each width
-// once over the cases that use it
-template <int CPL, typename T>
-__global__ void __launch_bounds__(256) k_smooth_x_scan(SmoothArgs<T> S) {
-  smooth_x_scan<CPL, xscan_lines<CPL>()>(S, (int)blockIdx.x);
-}
-template <int CPL, typename T>
-__global__ void __launch_bounds__(256) k_smooth_x_scan_b(const SmoothArgs<T> *As, const int4 *cg, int nc,
-                                                         const int *act) {
-  const int b = (int)blockIdx.x;
-  const int c = batch_case(cg, nc, b);
-  const int4 g = cg[c];
-  if (!act[g.w]) return;
-  smooth_x_scan<CPL, xscan_lines<CPL>()>(As[c], b - g.x);
-}
 template <typename T>
 __device__ __attribute__((always_inline)) inline void k_smooth_x_seq_body(const SmoothArgs<T> &S, int bx, int, int) {
   smooth_x_seq(S, bx);
@@ -337,130 +148,7 @@ __device__ __attribute__((always_inline)) inline void line_sweep(T *__restrict__
 #undef PR_B
 }
 
-// The same recurrences with three passes over the line instead of four:
-// the forward sweep keeps only the value y at the end of every chunk of CH
-// cells (in LDS, one slot per thread and chunk) and writes nothing; the
-// backward sweep, chunk by chunk from the end, re-reads the chunk's input,
-// recomputes its forward values from the checkpoint (the same operations,
-// so the same bits) and writes the final values.  The next chunk's loads
-// are issued before the current chunk's recurrence in both sweeps.  Lines
-// of up to CH * MAXC cells.
-template <int CH, int MAXC, typename T, typename CK>
-__device__ __attribute__((always_inline)) inline void line_sweep_ck(T *__restrict__ D, const uint8_t *__restrict__ F,
-                                                                    long b0, long st, int nl, const T *__restrict__ e1,
-                                                                    const T *__restrict__ r1, const T *__restrict__ e2,
-                                                                    T bb, CK ck) {
-  const int ncell = nl - 1;
-  const int nfull = ncell / CH;
-  T A[CH], B[CH], Y[CH];
-  unsigned ma = 0, mb = 0;
-  // full chunks: unconditional loads (the chunk index is clamped by the
-  // caller), so the next chunk's loads stay in flight under counted waits
-#define LDC(BUF, MK, c)                                               \
-  {                                                                   \
-    MK = 0;                                                           \
-    _Pragma("unroll") for (int t = 0; t < CH; t++) {                  \
-      long q_ = b0 + (long)(2 + (c) * CH + t) * st;                   \
-      BUF[t] = D[q_];                                                 \
-      MK |= (F[q_] & F_FLUID) ? (1u << t) : 0u;                       \
-    }                                                                 \
-  }
-#define FWD(BUF, MK, c, OUT)                                          \
-  _Pragma("unroll") for (int t = 0; t < CH; t++) {                    \
-    T m_ = ((MK >> t) & 1u) ? T(1) : T(0);                            \
-    y = m_ * piv_div(BUF[t] - bb * y, e1, r1, 2 + (c) * CH + t);      \
-    OUT                                                               \
-  }
-#define BWD(MK, c)                                                    \
-  _Pragma("unroll") for (int t = CH - 1; t >= 0; t--) {               \
-    int s_ = 2 + (c) * CH + t;                                        \
-    T m_ = ((MK >> t) & 1u) ? T(1) : T(0);                            \
-    z = Y[t] - m_ * (e2[s_] * z);                                     \
-    D[b0 + (long)s_ * st] = z;                                        \
-  }
-  // ---- forward: checkpoints after every full chunk, then the tail
-  T y = T(0);
-  if (nfull > 0) {
-    LDC(A, ma, 0);
-    for (int c = 0; c < nfull; c += 2) {
-      int c1 = c + 1 < nfull ? c + 1 : c;
-      LDC(B, mb, c1);
-      FWD(A, ma, c, ;);
-      ck[c] = y;
-      if (c + 1 >= nfull) break;
-      int c2 = c + 2 < nfull ? c + 2 : c + 1;
-      LDC(A, ma, c2);
-      FWD(B, mb, c + 1, ;);
-      ck[c + 1] = y;
-    }
-  }
-  // ---- backward: the tail (recomputed from the last checkpoint) ...
-  T z = T(0);
-  {
-    T yt = nfull > 0 ? ck[nfull - 1] : T(0);
-    const int s0 = 2 + nfull * CH;
-    T Yt[CH];
-    y = yt;
-    for (int s_ = s0; s_ <= nl; s_++) {
-      long q_ = b0 + (long)s_ * st;
-      T m_ = (F[q_] & F_FLUID) ? T(1) : T(0);
-      y = m_ * piv_div(D[q_] - bb * y, e1, r1, s_);
-      Yt[s_ - s0] = y;
-    }
-    for (int s_ = nl; s_ >= s0; s_--) {
-      long q_ = b0 + (long)s_ * st;
-      T m_ = (F[q_] & F_FLUID) ? T(1) : T(0);
-      z = Yt[s_ - s0] - m_ * (e2[s_] * z);
-      D[q_] = z;
-    }
-  }
-  // ... then the full chunks from the end, each recomputed from the
-  // checkpoint before it
-  if (nfull > 0) {
-    LDC(A, ma, nfull - 1);
-    for (int c = nfull - 1; c >= 0; c -= 2) {
-      int c1 = c >= 1 ? c - 1 : 0;
-      LDC(B, mb, c1);
-      y = c > 0 ? ck[c - 1] : T(0);
-      FWD(A, ma, c, Y[t] = y;);
-      BWD(ma, c);
-      if (c < 1) break;
-      int c2 = c >= 2 ? c - 2 : 0;
-      LDC(A, ma, c2);
-      y = c - 1 > 0 ? ck[c - 2] : T(0);
-      FWD(B, mb, c - 1, Y[t] = y;);
-      BWD(mb, c - 1);
-    }
-  }
-#undef LDC
-#undef FWD
-#undef BWD
-}
-
-// y/z line: the three-pass sweep for lines of up to 256 cells, else the
-// four-pass one.  16 checkpoints of one wave take 8 KB of LDS in FP64 and
-// the four-pass form runs 8-cell chunks, so neither limits the waves per
-// CU below what the three-pass registers allow (measured at 256^3: 4% faster
-// in FP64 and 17% in FP32 than 32 checkpoints and 16-cell fallback chunks).
-template <typename T>
-__device__ __attribute__((always_inline)) inline void smooth_line(T *D, const uint8_t *F, long b0, long st, int nl,
-                                                                  const T *e1, const T *r1, const T *e2, T bb) {
-  constexpr int CH = 16, MAXC = 16;
-  __shared__ T ck[MAXC][64];
-  if (nl - 1 <= CH * MAXC && blockDim.x * blockDim.y <= 64) {
-    // ck[c][lane]: the lanes of one chunk index sit side by side
-    T *mine = &ck[0][threadIdx.x + blockDim.x * threadIdx.y];
-    struct Col {
-      T *p;
-      __device__ T &operator[](int c) const { return p[c * 64]; }
-    } col{mine};
-    line_sweep_ck<CH, MAXC>(D, F, b0, st, nl, e1, r1, e2, bb, col);
-  } else {
-    line_sweep<8>(D, F, b0, st, nl, e1, r1, e2, bb);
-  }
-}
-
-// psmoo.f90:190-206 (y lines); thread per (i,k) and component
+// psmoo.f90:190-206 (y lines of more than 512 cells); thread per (i,k) and component
 template <typename T>
 __device__ __attribute__((always_inline)) inline void k_smooth_y_body(const SmoothArgs<T> &S, int bx, int by, int bz) {
   const Dims &d = S.d;
@@ -468,11 +156,11 @@ __device__ __attribute__((always_inline)) inline void k_smooth_y_body(const Smoo
   int k = 2 + by;
   int n = bz;
   if (i > d.il) return;
-  smooth_line(S.dw + n * d.E, S.flags, ix(d, i, 0, k), d.sy, d.jl, S.e1, S.r1, S.e2, S.bb);
+  line_sweep<8>(S.dw + n * d.E, S.flags, ix(d, i, 0, k), d.sy, d.jl, S.e1, S.r1, S.e2, S.bb);
 }
 MGE_ENTRY_T_XCD(k_smooth_y, SmoothArgs, 64, 1)
 
-// psmoo.f90:209-237 (z lines); thread per (i,j) and component
+// psmoo.f90:209-237 (z lines of more than 512 cells); thread per (i,j) and component
 template <typename T>
 __device__ __attribute__((always_inline)) inline void k_smooth_z_body(const SmoothArgs<T> &S, int bx, int by, int bz) {
   const Dims &d = S.d;
@@ -480,9 +168,405 @@ __device__ __attribute__((always_inline)) inline void k_smooth_z_body(const Smoo
   int j = 2 + by;
   int n = bz;
   if (i > d.il) return;
-  smooth_line(S.dw + n * d.E, S.flags, ix(d, i, j, 0), d.sz, d.kl, S.e1, S.r1, S.e2, S.bb);
+  line_sweep<8>(S.dw + n * d.E, S.flags, ix(d, i, j, 0), d.sz, d.kl, S.e1, S.r1, S.e2, S.bb);
 }
 MGE_ENTRY_T_XCD(k_smooth_z, SmoothArgs, 64, 1)
+
+// ---- lines in segments ---------------------------------------------------
+//
+// A line split into segments of L cells, one thread each, all of its cells in
+// registers and the segments joined through LDS.  Both
+// recurrences are evaluated within the segment from zero, giving the
+// segment's map from the value entering it to the value leaving it; every
+// thread then runs through the maps before (backward: after) it and
+// re-evaluates its cells with the reference formula from the value entering.
+// Branch-free: a cell's fluid bit selects its pivots or zeros (blank cells
+// hold dw = +-0, see line_sweep, and come out as 0), and the places past the
+// line's end count as blank; a branch per cell would wait for every LDS read
+// by itself (64^3 in k_smooth_xy: 25 us with branches, 13 without).
+// Called by all threads of the workgroup (barriers); sa, sb, sc, sd: LDS of
+// G x nline values each; `act` threads hold segment g of line `line`.
+template <typename T>
+struct SegPiv {   // a line's pivots, in LDS, indexed by cell from 0
+  const T *e1, *r1, *e2;
+};
+// x / e1 on a fluid cell, 0 on a blank one (rm: r1 or 0).  FP64 multiplies by
+// the reciprocal pivot; FP32 corrects the product by its remainder, which
+// gives the quotient the reference's division gives
+template <typename T>
+__device__ inline T seg_div(T x, T e1, T rm) {
+  const T q = x * rm;
+  if constexpr (kDelta<T>) return __builtin_fmaf(__builtin_fmaf(-e1, q, x), rm, q);
+  else return q;
+}
+template <int L, typename T>
+__device__ __attribute__((always_inline)) inline void seg_solve(bool act, T (&r)[L], unsigned fl, int s0, int g, int G,
+                                                                int line, int nline, const SegPiv<T> &P, T bb, T *sa,
+                                                                T *sb, T *sc, T *sd) {
+  auto rm = [&](int c) { return (fl >> c) & 1u ? P.r1[s0 + c] : T(0); };
+  auto e1 = [&](int c) { if constexpr (kDelta<T>) return P.e1[s0 + c]; else return T(0); };
+  auto qm = [&](int c) { return (fl >> c) & 1u ? P.e2[s0 + c] : T(0); };
+  T A = T(1), B = T(0);
+#pragma unroll
+  for (int c = 0; c < L; c++) {
+    const T m = rm(c);
+    B = seg_div(r[c] - bb * B, e1(c), m);
+    A = A * (-bb * m);
+  }
+  if (act) {
+    sa[g * nline + line] = A;
+    sb[g * nline + line] = B;
+  }
+  __syncthreads();
+  T y = T(0);
+  for (int q = 0; q < G - 1; q++) {   // uniform; the maps before this segment
+    const T ny = sa[q * nline + line] * y + sb[q * nline + line];
+    y = q < g ? ny : y;
+  }
+  T C = T(1), D = T(0);
+#pragma unroll
+  for (int c = 0; c < L; c++) {
+    y = seg_div(r[c] - bb * y, e1(c), rm(c));
+    r[c] = y;
+  }
+  // backward: z = y - e2 z', e2 = 0 on the line's last cell
+#pragma unroll
+  for (int c = L - 1; c >= 0; c--) {
+    const T m = qm(c);
+    D = r[c] - m * D;
+    C = -(m * C);
+  }
+  if (act) {
+    sc[g * nline + line] = C;
+    sd[g * nline + line] = D;
+  }
+  __syncthreads();
+  T z = T(0);
+  for (int q = G - 1; q > 0; q--) {
+    const T nz = sc[q * nline + line] * z + sd[q * nline + line];
+    z = q > g ? nz : z;
+  }
+#pragma unroll
+  for (int c = L - 1; c >= 0; c--) {
+    z = r[c] - qm(c) * z;
+    r[c] = z;
+  }
+}
+
+// x and y lines of a level whose k planes fit the LDS: a workgroup holds one
+// plane of one component, solves its x lines, then its y lines, and writes it
+// once.  In x a wave's lanes take neighbouring rows (the row length is odd in
+// LDS, so they fall on different banks), in y neighbouring columns.  The
+// separate launches read and write the field twice and, on small levels, wait
+// for one thread's walk along a whole line.  The plane's memory also carries
+// the segments' maps while its cells are in registers.  FP64, x and y sweeps
+// as they were -> this: 32^3 13.7 -> 6 us, 48^3 19 -> 8 us, 64^3 31 -> 13 us.
+template <typename T>
+struct SmoothXYArgs {
+  Dims d;
+  T *dw;
+  const uint8_t *flags;
+  const T *e1x, *e2x, *r1x, *e1y, *e2y, *r1y;
+  T bb;
+};
+// plane classes: cells of LDS (rows of nx | 1), mask words, pivots per
+// direction, threads, segment length.  Planes of more than 64 x 65 cells leave
+// too few workgroups a CU: 128 x 128 x 4 took 21 us in one launch, 11 in two.
+struct XYClass {
+  int cells, words, piv, threads, seg;
+};
+constexpr XYClass kXY[2] = {{2560, 128, 264, 512, 8}, {4416, 256, 264, 512, 8}};
+// the class that holds an nx x ny plane (-1: none)
+inline int xy_class(int nx, int ny) {
+  for (int c = 0; c < 2; c++) {
+    const XYClass &K = kXY[c];
+    const int gx = (nx + K.seg - 1) / K.seg, gy = (ny + K.seg - 1) / K.seg;
+    const long lx = (long)ny * gx, ly = (long)nx * gy;
+    if ((long)(nx | 1) * ny <= K.cells && (long)ny * ((nx + 63) / 64) <= K.words && lx <= K.threads &&
+        ly <= K.threads && 4 * std::max(lx, ly) <= K.cells && std::max(gx, gy) * K.seg <= K.piv)
+      return c;
+  }
+  return -1;
+}
+
+template <typename T, int CLS>
+__device__ __attribute__((always_inline)) inline void k_smooth_xy_body(const SmoothXYArgs<T> &S, int bx, int by) {
+  constexpr XYClass K = kXY[CLS];
+  constexpr int L = K.seg, NP = kDelta<T> ? 3 : 2;
+  __shared__ T pl[K.cells];
+  __shared__ T pv[2][NP][K.piv];   // x, y: 1/e1, e2 (and e1 in FP32)
+  __shared__ unsigned long long mk[K.words];
+  const Dims &d = S.d;
+  const int nx = d.ni, ny = d.nj, P = nx | 1, nch = (nx + 63) >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int t = tid; t < K.piv; t += K.threads) {
+    const int ix2 = 2 + min(t, nx - 1), iy2 = 2 + min(t, ny - 1);
+    pv[0][0][t] = S.r1x[ix2];
+    pv[0][1][t] = S.e2x[ix2];
+    pv[1][0][t] = S.r1y[iy2];
+    pv[1][1][t] = S.e2y[iy2];
+    if constexpr (kDelta<T>) {
+      pv[0][NP - 1][t] = S.e1x[ix2];
+      pv[1][NP - 1][t] = S.e1y[iy2];
+    }
+  }
+  // rows by groups of lp lanes (a power of two), RW rows a wave
+  const int lp = nx > 32 ? 64 : (nx > 16 ? 32 : (nx > 8 ? 16 : 8));
+  const int sub = lane / lp, l = lane & (lp - 1), RW = 64 / lp;
+  const long base = ix(d, 2, 2, 2 + bx);
+  T *D = S.dw + by * d.E + base;
+  const uint8_t *F = S.flags + base;
+  constexpr int NW = K.threads / 64, U = 8;
+  for (int ch = 0; ch < nch; ch++) {
+    const int i = (ch << 6) + l, ic = min(i, nx - 1);
+    for (int t0 = wave * RW + sub; t0 - sub < ny; t0 += NW * RW * U) {
+      T v[U];
+      uint8_t f[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const long q = (long)min(t0 + u * NW * RW, ny - 1) * d.sy + ic;
+        v[u] = D[q];
+        f[u] = F[q];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int row = t0 + u * NW * RW;
+        const unsigned long long b = __ballot(i < nx && (f[u] & F_FLUID));
+        if (row < ny) {
+          if (i < nx) pl[row * P + i] = v[u];
+          if (l == 0) mk[ch * ny + row] = lp == 64 ? b : (b >> (sub * lp)) & ((1ull << lp) - 1ull);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  T r[L];
+  {  // x lines
+    const int G = (nx + L - 1) / L, line = tid % ny, g = tid / ny;
+    const bool act = g < G;
+    const int i0 = act ? g * L : 0, m = act ? min(L, nx - i0) : 0;
+    const int c0 = i0 >> 6, sh = i0 & 63;
+    unsigned fl = (unsigned)(mk[c0 * ny + line] >> sh);
+    if (sh + L > 64) fl |= c0 + 1 < nch ? (unsigned)(mk[(c0 + 1) * ny + line] << (64 - sh)) : 0u;
+    const T *row = pl + line * P;
+#pragma unroll
+    for (int c = 0; c < L; c++) r[c] = row[min(i0 + c, nx - 1)];
+    __syncthreads();
+    const int n = G * ny;
+    seg_solve<L>(act, r, fl, i0, g, G, line, ny, SegPiv<T>{pv[0][NP - 1], pv[0][0], pv[0][1]}, S.bb, pl, pl + n,
+                 pl + 2 * n, pl + 3 * n);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < L; c++)
+      if (c < m) pl[line * P + i0 + c] = r[c];
+  }
+  __syncthreads();
+  {  // y lines
+    const int G = (ny + L - 1) / L, line = tid % nx, g = tid / nx;
+    const bool act = g < G;
+    const int j0 = act ? g * L : 0, m = act ? min(L, ny - j0) : 0;
+    unsigned fl = 0;
+    const unsigned long long *mc = mk + (line >> 6) * ny;
+#pragma unroll
+    for (int c = 0; c < L; c++) {
+      const int j = min(j0 + c, ny - 1);
+      r[c] = pl[j * P + line];
+      fl |= ((unsigned)(mc[j] >> (line & 63)) & (j0 + c < ny ? 1u : 0u)) << c;
+    }
+    __syncthreads();
+    const int n = G * nx;
+    seg_solve<L>(act, r, fl, j0, g, G, line, nx, SegPiv<T>{pv[1][NP - 1], pv[1][0], pv[1][1]}, S.bb, pl, pl + n,
+                 pl + 2 * n, pl + 3 * n);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < L; c++)
+      if (c < m) pl[(j0 + c) * P + line] = r[c];
+  }
+  __syncthreads();
+  for (int ch = 0; ch < nch; ch++) {
+    const int i = (ch << 6) + l;
+    if (i >= nx) continue;
+#pragma unroll 4
+    for (int row = wave * RW + sub; row < ny; row += NW * RW) D[(long)row * d.sy + i] = pl[row * P + i];
+  }
+}
+template <typename T, int CLS>
+__global__ void __launch_bounds__(kXY[CLS].threads) k_smooth_xy(SmoothXYArgs<T> S) {
+  k_smooth_xy_body<T, CLS>(S, (int)blockIdx.x, (int)blockIdx.y);
+}
+template <typename T, int CLS>
+__global__ void __launch_bounds__(kXY[CLS].threads)
+    k_smooth_xy_b(const SmoothXYArgs<T> *As, const int4 *cg, int nc, const int *act) {
+  const int b = (int)blockIdx.x;
+  const int c = batch_case(cg, nc, b);
+  const int4 g = cg[c];
+  if (!act[g.w]) return;
+  const int l = b - g.x;
+  k_smooth_xy_body<T, CLS>(As[c], l % g.y, l / g.y);
+}
+
+// y (DIR 1) or z (DIR 2) lines in segments: a workgroup takes SX lines that
+// lie side by side in x, one thread a segment of L cells, so the field is read
+// once and written once and no thread walks a whole line.  Lines of up to 16
+// cells are one segment (64 lines a wave), up to 256 cells 32 lines in 16
+// segments of 8 or 16, up to 512 cells 16 lines in 32.  Bound by the field's
+// one read and write where the level is large.  Thread per line before ->
+// this, y lines: 256^3 FP64 421 -> 296 us (4.6 TB/s), FP32 243 -> 183 us;
+// 128^3 46 -> 32 us; 512 x 512 x 4 105 -> 26 us.
+struct SegShape {
+  int sx, len;   // lines side by side, cells per segment (0: too long)
+};
+inline SegShape seg_shape(int n) {
+  if (n <= 16) return SegShape{64, n <= 4 ? 4 : (n <= 8 ? 8 : 16)};
+  if (n <= 256) return SegShape{32, n <= 128 ? 8 : 16};
+  return n <= 512 ? SegShape{16, 16} : SegShape{0, 0};
+}
+template <typename T, int SX, int L, int DIR>
+__device__ __attribute__((always_inline)) inline void k_smooth_seg_body(const SmoothArgs<T> &S, int bx, int by,
+                                                                        int bz) {
+  constexpr int NP = kDelta<T> ? 3 : 2, GM = SX == 64 ? 1 : 512 / SX;
+  __shared__ T sh[4][GM * SX], pv[NP][L * GM];
+  const Dims &d = S.d;
+  const int n = DIR == 1 ? d.nj : d.nk, G = (n + L - 1) / L;
+  const long st = DIR == 1 ? d.sy : d.sz;
+  const int line = threadIdx.x & (SX - 1), g = threadIdx.x / SX;
+  const int i = 2 + bx * SX + line;
+  const bool act = g < G && i <= d.il;
+  const int s0 = g < G ? g * L : 0, m = act ? min(L, n - s0) : 0;
+  const long q0 = DIR == 1 ? ix(d, min(i, d.il), 2, 2 + by) : ix(d, min(i, d.il), 2 + by, 2);
+  T *D = S.dw + bz * d.E + q0;
+  const uint8_t *F = S.flags + q0;
+  T r[L];
+  unsigned fl = 0;
+#pragma unroll
+  for (int c = 0; c < L; c++) {
+    const long o = (long)min(s0 + c, n - 1) * st;
+    r[c] = D[o];
+    fl |= (F[o] & F_FLUID && s0 + c < n ? 1u : 0u) << c;
+  }
+  for (int t = threadIdx.x; t < G * L; t += blockDim.x) {
+    const int s = 2 + min(t, n - 1);
+    pv[0][t] = S.r1[s];
+    pv[1][t] = S.e2[s];
+    if constexpr (kDelta<T>) pv[NP - 1][t] = S.e1[s];
+  }
+  __syncthreads();
+  seg_solve<L>(act, r, fl, s0, g, G, line, SX, SegPiv<T>{pv[NP - 1], pv[0], pv[1]}, S.bb, sh[0], sh[1], sh[2], sh[3]);
+#pragma unroll
+  for (int c = 0; c < L; c++)
+    if (c < m) D[(long)(s0 + c) * st] = r[c];
+}
+template <typename T, int SX, int L, int DIR>
+__global__ void __launch_bounds__(SX == 64 ? 64 : 512) k_smooth_seg(SmoothArgs<T> S) {
+  int bx, by, bz;
+  xcd_block(bx, by, bz);
+  k_smooth_seg_body<T, SX, L, DIR>(S, bx, by, bz);
+}
+template <typename T, int SX, int L, int DIR>
+__global__ void __launch_bounds__(SX == 64 ? 64 : 512)
+    k_smooth_seg_b(const SmoothArgs<T> *As, const int4 *cg, int nc, const int *act) {
+  const int b = (int)blockIdx.x;
+  const int c = batch_case(cg, nc, b);
+  const int4 g = cg[c];
+  if (!act[g.w]) return;
+  const int l = b - g.x;
+  k_smooth_seg_body<T, SX, L, DIR>(As[c], l % g.y, (l / g.y) % g.z, l / (g.y * g.z));
+}
+
+// x lines in segments of 16 cells, where the planes do not fit k_smooth_xy:
+// a workgroup stages 16 (N = 128: 32) rows of up to N cells in LDS (whole rows,
+// so loads and stores are coalesced), each thread takes a segment.  With lines
+// scanned across a wave's lanes by shuffles -> this: 256^3 FP64 399 -> 286 us
+// (4.7 TB/s), FP32 291 -> 201 us; 128^3 54 -> 48 us; 96^3 33 -> 24 us.
+template <int N>
+constexpr int xseg_rows() { return N == 128 ? 32 : 16; }
+template <typename T, int N>
+__device__ __attribute__((always_inline)) inline void k_smooth_xseg_body(const SmoothArgs<T> &S, int bx, int by) {
+  constexpr int NP = kDelta<T> ? 3 : 2, L = 16, kXR = xseg_rows<N>(), NT = kXR * N / L, NW = NT / 64;
+  __shared__ T pl[kXR * (N + 1)], pv[NP][N];
+  __shared__ unsigned long long mk[kXR * N / 64];
+  const Dims &d = S.d;
+  const int nx = d.ni, P = nx | 1, nch = (nx + 63) >> 6, G = (nx + L - 1) / L;
+  const int nl = d.nj * d.nk, l0 = bx * kXR, rows = min(kXR, nl - l0);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  T *D = S.dw + by * d.E;
+  auto at = [&](int row) {   // the first cell of the workgroup's row
+    const int l = l0 + min(row, rows - 1), k = l / d.nj;
+    return ix(d, 2, 2 + l - k * d.nj, 2 + k);
+  };
+  for (int t = tid; t < G * L; t += NT) {
+    const int s = 2 + min(t, nx - 1);
+    pv[0][t] = S.r1[s];
+    pv[1][t] = S.e2[s];
+    if constexpr (kDelta<T>) pv[NP - 1][t] = S.e1[s];
+  }
+  constexpr int RW = kXR / NW;                      // rows of a wave
+  constexpr int U = N / 64;                         // chunks of a row
+#pragma unroll 2
+  for (int u = 0; u < RW; u++) {
+    const int row = wave * RW + u;
+    const long q = at(row);
+    T v[U];
+    uint8_t f[U];
+#pragma unroll
+    for (int c = 0; c < U; c++) {
+      const int i = min(c * 64 + lane, nx - 1);
+      v[c] = D[q + i];
+      f[c] = S.flags[q + i];
+    }
+#pragma unroll
+    for (int c = 0; c < U; c++) {
+      const int i = c * 64 + lane;
+      const unsigned long long b = __ballot(i < nx && (f[c] & F_FLUID));
+      if (i < nx) pl[row * P + i] = v[c];
+      if (lane == 0) mk[c * kXR + row] = b;
+    }
+  }
+  __syncthreads();
+  const int line = tid & (kXR - 1), g = tid / kXR;
+  const bool act = g < G;
+  const int i0 = act ? g * L : 0, m = act ? min(L, nx - i0) : 0;
+  const unsigned fl = (unsigned)(mk[(i0 >> 6) * kXR + line] >> (i0 & 63)) & 0xffffu;
+  T r[L];
+#pragma unroll
+  for (int c = 0; c < L; c++) r[c] = pl[line * P + min(i0 + c, nx - 1)];
+  __syncthreads();
+  const int n = G * kXR;
+  seg_solve<L>(act, r, fl, i0, g, G, line, kXR, SegPiv<T>{pv[NP - 1], pv[0], pv[1]}, S.bb, pl, pl + n, pl + 2 * n,
+               pl + 3 * n);
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < L; c++)
+    if (c < m) pl[line * P + i0 + c] = r[c];
+  __syncthreads();
+#pragma unroll 2
+  for (int u = 0; u < RW; u++) {
+    const int row = wave * RW + u;
+    if (row >= rows) break;
+    const long q = at(row);
+#pragma unroll
+    for (int c = 0; c < U; c++) {
+      const int i = c * 64 + lane;
+      if (i < nx) D[q + i] = pl[row * P + i];   // blank cells: as they were read
+    }
+  }
+}
+template <typename T, int N>
+__global__ void __launch_bounds__(xseg_rows<N>() * N / 16) k_smooth_xseg(SmoothArgs<T> S) {
+  int bx, by, bz;
+  xcd_block(bx, by, bz);
+  k_smooth_xseg_body<T, N>(S, bx, by);
+}
+template <typename T, int N>
+__global__ void __launch_bounds__(xseg_rows<N>() * N / 16)
+    k_smooth_xseg_b(const SmoothArgs<T> *As, const int4 *cg, int nc, const int *act) {
+  const int b = (int)blockIdx.x;
+  const int c = batch_case(cg, nc, b);
+  const int4 g = cg[c];
+  if (!act[g.w]) return;
+  const int l = b - g.x;
+  k_smooth_xseg_body<T, N>(As[c], l % g.y, l / g.y);
+}
 
 // ---- psmoo (psmoo.f90:1-95) with progon3's sweep (progon3.f90:1-62) ------
 // Rows (1+2e_r) x_r - e_r x_{r-1} - e_r x_{r+1} = d_r along each line of
