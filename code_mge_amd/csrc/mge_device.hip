@@ -117,10 +117,8 @@ struct Level {
   int tj = 0;                   // tuned or forced tile rows of the stage kernels (0: tile_pick's)
   bool tuned = false;           // kc and tj come from the autotuner (a batch picks its own)
   int btj = 0, bkc = 0;         // the batch's common choice while the case is recorded into it (0: none)
-  void *vprim = nullptr;        // Navier-Stokes: velocity and temperature per cell (4E)
-  int nvcell = 0;               // cut cells with wall records (viscous wall terms)
-  long *vcell = nullptr;
-  int *vbeg = nullptr, *vrec = nullptr;
+  int *vtile = nullptr;         // Navier-Stokes: wall records by tile of the viscous kernel
+  ViscRec *vrec = nullptr;
   int mxcyc = 1;
   std::vector<void *> allocs;
   size_t bytes = 0;  // device bytes of the level
@@ -622,6 +620,10 @@ int do_timestep(mge_case *h, Level &L, bool need_dt = true) {
 
 // ---- euler -------------------------------------------------------------------
 
+dim3 visc_grid(const Dims &d) {
+  return dim3((d.ni + kVX - 1) / kVX, (d.nj + kVY - 1) / kVY, (d.nk + kVZ - 1) / kVZ);
+}
+
 // arguments of the viscous kernels on state buffer buf
 template <class T>
 ViscArgs<T> visc_args(mge_case *h, Level &L, int buf, T cdis, T blend, int m) {
@@ -631,7 +633,6 @@ ViscArgs<T> visc_args(mge_case *h, Level &L, int buf, T cdis, T blend, int m) {
   V.s = stc<T>(L, buf);
   V.flags = L.flags;
   V.g = geo<T>(L);
-  V.prim = tp<T>(L.vprim);
   V.fw = tp<T>(L.fw);
   V.inf = make_inf<T>(P);
   V.uinf[0] = (T)P.u0;
@@ -644,6 +645,11 @@ ViscArgs<T> visc_args(mge_case *h, Level &L, int buf, T cdis, T blend, int m) {
   V.cdis = cdis;
   V.blend = blend;
   V.m = m;
+  V.vtile = L.vtile;
+  V.vrec = L.vrec;
+  V.wsol = L.wsol;
+  V.psol = L.psol;
+  V.nmir = L.nmir;
   return V;
 }
 
@@ -911,10 +917,7 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
     A.fw_in = P.eqntype == 1 && A.has_diss;
     if (A.fw_in) {
       ViscArgs<T> V = visc_args<T>(h, L, src, A.fx.cdis, A.blend, m);
-      LAUNCHT(h, "k_visc_prim", k_visc_prim, T, flat_grid(E), dim3(256), V);
-      LAUNCHT(h, "k_visc", k_visc, T, cell_grid(d), cell_block(), V);
-      LAUNCHT(h, "k_visc_wall", k_visc_wall, T, dim3((L.nvcell + 63) / 64), dim3(64),
-              (ViscWallArgs<T>{V, L.recs, L.wsol, L.psol, L.nmir, L.vcell, L.vbeg, L.vrec, L.nvcell}));
+      LAUNCHT(h, "k_visc", k_visc, T, visc_grid(d), dim3(kVNT), V);
     }
     {
       // algorithmic bytes per cell: read W^(m-1); write W^(m) and read W^(0)
@@ -1564,38 +1567,38 @@ int build_records(mge_case *h, Level &L, int nmir, const mge_cutrec *recs) {
   CHKRC(dalloc(L, &L.chunks, chunks.size() + 1));
   CHKRC(dalloc(L, &L.opval, (opv.size() + 1) * 10));  // the wall force's per-record terms
   HIPCHK(h2d_sync(L.recs, dr.data(), sizeof(DevRec) * nmir, h->stream));
-  {
-    // cut cells with wall records, in order of their first record, and
-    // their records in record order (viscous wall terms)
-    std::map<long, int> slot;
-    std::vector<long> vc;
-    std::vector<std::vector<int>> lists;
+  if (h->prm.eqntype == 1) {
+    // the wall records sorted by tile of the viscous kernel, cell of the
+    // tile and record
+    const dim3 vg = visc_grid(d);
+    std::vector<int> vt((size_t)vg.x * vg.y * vg.z + 1, 0);
+    std::vector<std::pair<long, int>> order(nmir);  // tile and cell, record
+    constexpr int ncell = kVX * kVY * kVZ;
     for (int m = 0; m < nmir; m++) {
-      long qc = ix(d, recs[m].ccid[0], recs[m].ccid[1], recs[m].ccid[2]);
-      auto it = slot.find(qc);
-      int sl;
-      if (it == slot.end()) {
-        sl = (int)vc.size();
-        slot[qc] = sl;
-        vc.push_back(qc);
-        lists.emplace_back();
-      } else {
-        sl = it->second;
+      const int x = recs[m].ccid[0] - 2, y = recs[m].ccid[1] - 2, z = recs[m].ccid[2] - 2;
+      const long tile = ((long)(z / kVZ) * vg.y + y / kVY) * vg.x + x / kVX;
+      order[m] = {tile * ncell + ((z % kVZ) * kVY + y % kVY) * kVX + x % kVX, m};
+      vt[tile + 1]++;
+    }
+    for (size_t t = 1; t < vt.size(); t++) vt[t] += vt[t - 1];
+    std::sort(order.begin(), order.end());
+    std::vector<ViscRec> vr(nmir);
+    for (int o = 0; o < nmir; o++) {
+      const mge_cutrec &r = recs[order[o].second];
+      ViscRec &v = vr[o];
+      v.m = order[o].second;
+      v.cell = (int)(order[o].first % ncell);
+      v.dir = r.zz - 1;
+      v.hi = r.faceid >= 4;
+      for (int a = 0; a < 3; a++) {
+        v.c[a] = r.ccid[a];
+        v.s[a] = r.scid[a];
       }
-      lists[sl].push_back(m);
     }
-    std::vector<int> vb(1, 0), vr;
-    for (auto &l : lists) {
-      vr.insert(vr.end(), l.begin(), l.end());
-      vb.push_back((int)vr.size());
-    }
-    L.nvcell = (int)vc.size();
-    CHKRC(dalloc(L, &L.vcell, vc.size()));
-    CHKRC(dalloc(L, &L.vbeg, vb.size()));
+    CHKRC(dalloc(L, &L.vtile, vt.size()));
     CHKRC(dalloc(L, &L.vrec, vr.size()));
-    HIPCHK(h2d_sync(L.vcell, vc.data(), sizeof(long) * vc.size(), h->stream));
-    HIPCHK(h2d_sync(L.vbeg, vb.data(), sizeof(int) * vb.size()));
-    HIPCHK(h2d_sync(L.vrec, vr.data(), sizeof(int) * vr.size()));
+    HIPCHK(h2d_sync(L.vtile, vt.data(), sizeof(int) * vt.size(), h->stream));
+    HIPCHK(h2d_sync(L.vrec, vr.data(), sizeof(ViscRec) * vr.size()));
   }
   HIPCHK(h2d_sync(L.tcell, tcell.data(), sizeof(long) * tcell.size(), h->stream));
   HIPCHK(h2d_sync(L.beg, begv.data(), sizeof(int) * begv.size()));
@@ -2150,7 +2153,6 @@ int mge_level_define(mge_case *h, int lvl, int ni, int nj, int nk, const double 
     CHKRC(dalloc(L, &L.lim, 3 * E));
     HIPCHK(fill_sync(L.lim, 0xff, (size_t)E * 3 * sizeof(unsigned long long)));
   }
-  if (h->prm.eqntype == 1) CHKRC(dalloc_bytes(L, &L.vprim, es * 4 * E));
   if (h->prm.execmode == 1) {
     CHKRC(dalloc_bytes(L, &L.w1, es * 5 * E));
     CHKRC(dalloc_bytes(L, &L.w2, es * 5 * E));

@@ -73,8 +73,6 @@ def level_bytes(n, es, nmir=0, mxcyc=4, viscous=False, coarse=False, psmoo=False
     ngrid = -(-ni // 64) * -(-nj // 4) * -(-nk // 8)   # residual-norm partials (8 planes per block)
     sizes = [es * 6 * E] * 3 + [es * 5 * E] * 5 + [es * E] * 2 + [E] * 2
     sizes += [es * nmax] * 3 + [es * 9 * nmax, 8 * ngrid, 8, 8, 8 * (mxcyc + 1), 24]
-    if viscous:
-        sizes += [es * 4 * E]           # velocity and temperature
     if coarse:
         sizes += [es * 5 * E]           # correction w - ws
     if psmoo:
@@ -85,7 +83,8 @@ def level_bytes(n, es, nmir=0, mxcyc=4, viscous=False, coarse=False, psmoo=False
         ntouch, nops = 2 * nmir, 6 * nmir
         sizes += [DEVREC_BYTES * nmir, 40 * nmir, 8 * nmir, 8 * ntouch, 4 * (ntouch + 1), 48 * (nops + 1),
                   16 * (ntouch + 1), 80 * (nops + 1)]
-        sizes += [8 * nmir, 4 * (nmir + 1), 4 * nmir]   # cut cells with their record lists
+        if viscous:                     # the viscous kernel's records by 16 x 4 x 4 tile
+            sizes += [4 * (-(-ni // 16) * -(-nj // 4) * -(-nk // 4) + 1), 40 * nmir]
     return sum(s + 64 for s in sizes)
 
 
