@@ -305,6 +305,17 @@ __device__ inline void xcd_block(int &bx, int &by, int &bz) {
     NAME##_body(As[c], l % g.y, (l / g.y) % g.z, l / (g.y * g.z));                                     \
   }
 
+// x / h from r = 1/h: the product corrected by its remainder, which is the
+// quotient the division gives
+__device__ inline float quot(float x, float h, float r) {
+  const float q = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-h, q, x), r, q);
+}
+__device__ inline double quot(double x, double h, double r) {
+  const double q = x * r;
+  return __builtin_fma(__builtin_fma(-h, q, x), r, q);
+}
+
 template <typename T>
 __device__ inline T dimd(T a, T b) { return a > b ? a - b : T(0); }
 template <typename T>

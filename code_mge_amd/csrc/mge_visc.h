@@ -76,17 +76,6 @@ __device__ inline void visc_prim(const ViscArgs<T> &A, bool fluid, const T *w, T
   for (int a = 0; a < 4; a++) o[a] = fluid ? o[a] : T(0);
 }
 
-// x / h from r = 1/h: the product corrected by its remainder, which is the
-// quotient the division gives
-__device__ inline float visc_div(float x, float h, float r) {
-  const float q = x * r;
-  return __builtin_fmaf(__builtin_fmaf(-h, q, x), r, q);
-}
-__device__ inline double visc_div(double x, double h, double r) {
-  const double q = x * r;
-  return __builtin_fma(__builtin_fma(-h, q, x), r, q);
-}
-
 // one face: pL/pR velocity + temperature of the two cells (FP32: deviations,
 // u0 the freestream velocity), dn their normal derivatives, t1*/t2* the
 // tangential velocity derivatives of the two cells; momentum and energy flux
@@ -155,7 +144,7 @@ __device__ inline void visc_dt(const ViscLds<T> &L, const ViscAxis<T, N> &X, int
   const T h1 = fp ? X.hm[c + 1] : X.hm[c], r1 = fp ? X.rm[c + 1] : X.rm[c];
   const T h = fp && fm ? X.hc[c] : h1, r = fp && fm ? X.rc[c] : r1;
 #pragma unroll
-  for (int a = 0; a < 3; a++) out[a] = visc_div(L.pr[a][oh] - L.pr[a][ol], h, r);
+  for (int a = 0; a < 3; a++) out[a] = quot(L.pr[a][oh] - L.pr[a][ol], h, r);
 }
 
 // thread t's face of direction DIR: its flux into the buffer
@@ -175,7 +164,7 @@ __device__ inline void visc_bulk_face(const ViscArgs<T> &A, const ViscLds<T> &L,
     for (int a = 0; a < 4; a++) {
       pL[a] = L.pr[a][oL];
       pR[a] = L.pr[a][oR];
-      dn[a] = visc_div(pR[a] - pL[a], hn, rn);
+      dn[a] = quot(pR[a] - pL[a], hn, rn);
     }
     if constexpr (DIR == 0) {
       visc_dt(L, L.y, oL, kVSY, y, t1L);
