@@ -1438,7 +1438,7 @@ int do_wall_force(mge_case *h, Level &L) {
     hipLaunchKernelGGL(k_wall_visc_terms<T>, dim3((L.nmir + 63) / 64), dim3(64), 0, h->stream, V,
                        (const DevRec *)L.recs, (const double *)L.wsol, (const double *)L.psol, L.nmir, L.opval);
   }
-  hipLaunchKernelGGL(k_wall_sum, dim3(1), dim3(64), 0, h->stream, (const double *)L.opval, L.nmir, L.force);
+  hipLaunchKernelGGL(k_wall_sum, dim3(1), dim3(kSumT), 0, h->stream, (const double *)L.opval, L.nmir, L.force);
   return MGE_OK;
 }
 
