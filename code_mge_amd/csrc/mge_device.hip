@@ -101,10 +101,8 @@ struct Level {
   DevRec *recs = nullptr;
   double *wsol = nullptr, *psol = nullptr;
   std::vector<mge_cutrec> hrecs;
-  long *tcell = nullptr;
-  int *beg = nullptr;
+  RecSlot *cells = nullptr;  // k_rec's touched cells and ops, kRecOps places a workgroup
   RecOp *ops = nullptr;
-  int4 *chunks = nullptr;  // k_rec's workgroups (touched cells and ops)
   int nchunk = 0;
   double *opval = nullptr;
   double *partial = nullptr;
@@ -949,10 +947,8 @@ int do_euler(mge_case *h, Level &L, int ncyc, int mgl, int mlvl, int lres, int l
       R.wsol = L.wsol;
       R.psol = L.psol;
       R.nmir = L.nmir;
-      R.tcell = L.tcell;
-      R.beg = L.beg;
+      R.cells = L.cells;
       R.ops = L.ops;
-      R.chunks = L.chunks;
       R.err = h->err;
       LAUNCHT(h, "k_rec", k_rec, T, dim3((unsigned)L.nchunk), dim3(kRecOps), R);
     }
@@ -1546,25 +1542,30 @@ int build_records(mge_case *h, Level &L, int nmir, const mge_cutrec *recs) {
     begv.push_back((int)opv.size());
   }
   const int ntouch = (int)tcell.size();
-  // workgroups of k_rec: consecutive touched cells with at most kRecOps ops
-  std::vector<int4> chunks;
-  auto add_chunk = [&](int t0, int t1) { chunks.push_back(make_int4(t0, t1, begv[t0], begv[t1])); };
+  // workgroups of k_rec: consecutive touched cells with at most kRecOps ops,
+  // each with kRecOps places for its cells and ops
+  RecOp no_op{};
+  no_op.rec = -1;
+  std::vector<RecSlot> cells;
+  std::vector<RecOp> ops;
+  L.nchunk = 0;
   for (int t = 0, t0 = 0; t < ntouch; t++) {
     if (begv[t + 1] - begv[t] > kRecOps) return set_err(MGE_ERR_ARG, "too many wall ops on one cell");
-    if (begv[t + 1] - begv[t0] > kRecOps) {
-      add_chunk(t0, t);
+    if (t == 0 || begv[t + 1] - begv[t0] > kRecOps) {
       t0 = t;
+      L.nchunk++;
+      cells.resize((size_t)L.nchunk * kRecOps, RecSlot{-1, 0, 0});
+      ops.resize((size_t)L.nchunk * kRecOps, no_op);
     }
-    if (t == ntouch - 1) add_chunk(t0, ntouch);
+    const size_t base = (size_t)(L.nchunk - 1) * kRecOps;
+    cells[base + t - t0] = RecSlot{tcell[t], begv[t] - begv[t0], begv[t + 1] - begv[t0]};
+    std::copy(opv.begin() + begv[t], opv.begin() + begv[t + 1], ops.begin() + base + begv[t] - begv[t0]);
   }
-  L.nchunk = (int)chunks.size();
   CHKRC(dalloc(L, &L.recs, nmir));
   CHKRC(dalloc(L, &L.wsol, (size_t)5 * nmir));
   CHKRC(dalloc(L, &L.psol, nmir));
-  CHKRC(dalloc(L, &L.tcell, tcell.size()));
-  CHKRC(dalloc(L, &L.beg, begv.size()));
-  CHKRC(dalloc(L, &L.ops, opv.size() + 1));
-  CHKRC(dalloc(L, &L.chunks, chunks.size() + 1));
+  CHKRC(dalloc(L, &L.cells, cells.size() + 1));
+  CHKRC(dalloc(L, &L.ops, ops.size() + 1));
   CHKRC(dalloc(L, &L.opval, (opv.size() + 1) * 10));  // the wall force's per-record terms
   HIPCHK(h2d_sync(L.recs, dr.data(), sizeof(DevRec) * nmir, h->stream));
   if (h->prm.eqntype == 1) {
@@ -1600,10 +1601,8 @@ int build_records(mge_case *h, Level &L, int nmir, const mge_cutrec *recs) {
     HIPCHK(h2d_sync(L.vtile, vt.data(), sizeof(int) * vt.size(), h->stream));
     HIPCHK(h2d_sync(L.vrec, vr.data(), sizeof(ViscRec) * vr.size()));
   }
-  HIPCHK(h2d_sync(L.tcell, tcell.data(), sizeof(long) * tcell.size(), h->stream));
-  HIPCHK(h2d_sync(L.beg, begv.data(), sizeof(int) * begv.size()));
-  if (!opv.empty()) HIPCHK(h2d_sync(L.ops, opv.data(), sizeof(RecOp) * opv.size()));
-  if (!chunks.empty()) HIPCHK(h2d_sync(L.chunks, chunks.data(), sizeof(int4) * chunks.size()));
+  if (!ops.empty()) HIPCHK(h2d_sync(L.ops, ops.data(), sizeof(RecOp) * ops.size(), h->stream));
+  if (!cells.empty()) HIPCHK(h2d_sync(L.cells, cells.data(), sizeof(RecSlot) * cells.size()));
   std::vector<uint8_t> fl(d.E);
   HIPCHK(d2h_sync(fl.data(), L.flags, d.E, h->stream));
   for (long q : tcell) fl[q] |= F_TOUCHED;

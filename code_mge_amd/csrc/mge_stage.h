@@ -88,10 +88,19 @@ struct StageArgs {
 // by the host so that one load, not a chain through the record, precedes the
 // op's stencil loads
 struct alignas(16) RecOp {
-  int rec;                  // record (mirror state)
+  int rec;                  // record (mirror state); -1: no op in this place
   uint8_t kind, zz, hi, pad;
   int c[3], s[3];           // cut cell, solid cell
   long qc;                  // cell index of the cut cell
+};
+
+// ops of one workgroup of k_rec (its threads); no touched cell has more
+// than 36 (6 records as cut cell x 4, 6 as neighbour x 2)
+constexpr int kRecOps = 64;
+// a touched cell and the range of its ops in its workgroup
+struct alignas(16) RecSlot {
+  long q;                   // cell index; -1: no cell in this place
+  int o0, o1;
 };
 
 template <typename T>
@@ -100,16 +109,10 @@ struct RecArgs {
   const double *wsol;       // 5*nmir, component-major
   const double *psol;
   int nmir;
-  const long *tcell;        // touched cells
-  const int *beg;           // op range of each touched cell (ntouch+1)
-  const RecOp *ops;         // fw ops then dw ops per cell
-  const int4 *chunks;       // touched cells [x, y) of each workgroup and their ops [z, w), at most kRecOps
+  const RecSlot *cells;     // touched cells, kRecOps places a workgroup
+  const RecOp *ops;         // fw ops then dw ops per cell, kRecOps places a workgroup
   int *err;
 };
-
-// ops of one workgroup of k_rec (its threads); no touched cell has more
-// than 36 (6 records as cut cell x 4, 6 as neighbour x 2)
-constexpr int kRecOps = 64;
 
 // the Roe wall-face term of a record (defined with the Roe scheme)
 template <typename T, class R>
@@ -824,7 +827,7 @@ __device__ inline RecLine<T> rec_line(const FluxCtx<T> &c, const RecOp &r, int o
   const long st = r.zz == 1 ? 1L : (r.zz == 2 ? d.sy : d.sz);
   // sums of products rather than selects between fields (see face_s_any)
   const int nl = (r.zz == 1) * d.il + (r.zz == 2) * d.jl + (r.zz == 3) * d.kl;
-  const int a = (r.zz == 1 ? r.c[0] : (r.zz == 2 ? r.c[1] : r.c[2])) + off;
+  const int a = (r.zz == 1) * r.c[0] + (r.zz == 2) * r.c[1] + (r.zz == 3) * r.c[2] + off;
   const long q = r.qc + (long)off * st;
   L.a = a;
   L.ne = nl + 1;
@@ -1072,34 +1075,33 @@ __device__ __attribute__((always_inline)) inline void rec_op_value(const RecArgs
 // with their ops (at most kRecOps), one thread per op computes its value
 // into LDS, then one thread per cell adds its ops' values in the reference
 // order (in FP64) and finishes the cell in T.  The launch lasts as long as
-// one workgroup's chain of round trips -- its range, the op, the op's line --
+// one workgroup's chain of round trips -- the op, the op's line --
 // and the arithmetic of the op kinds one after another; reading each face's
 // stencil where a kind's branch needed it took 23-33 us on every level, the
-// line form takes 9-13 us (JST; Roe 8 -> 7).
+// line form takes 9-13 us (JST; Roe 8 -> 7).  Ops and cells lie at places
+// given by the block and thread (empty ones marked), not behind a range that
+// is loaded first: mean over the levels of 128 x 128 x 4 9.9 -> 9.6 us, of 96^3
+// 12.7 -> 11.9 us, of 70 x 37 x 19 (Roe) 8.4 -> 7.6 us.
 template <typename T>
 __device__ __attribute__((always_inline)) inline void k_rec_body(const RecArgs<T> &R, int bx, int, int) {
   __shared__ double val[kRecOps * 10];
   __shared__ uint8_t kinds[kRecOps];
-  const int4 ch = R.chunks[bx];
-  const int o0 = ch.z;
   const int tid = threadIdx.x;
-  const int t = ch.x + tid;
+  const RecSlot sl = R.cells[(long)bx * kRecOps + tid];
+  const RecOp r = R.ops[(long)bx * kRecOps + tid];
   const StageArgs<T> &A = R.st;
   const Dims &d = A.fx.d;
   const long E = d.E;
   // the cell's fw and dw, and the finish's inputs (W(0) on an unsmoothed
   // stage, the local time step, the flags, the forcing), are loaded before
   // the op values are formed, so their round trips overlap the ops' own
-  const bool cell = t < ch.y;
-  const long q = cell ? R.tcell[t] : 0;
-  int b0 = 0, b1 = 0;
+  const bool cell = sl.q >= 0;
+  const long q = cell ? sl.q : 0;
   double f[5], e[5];
   T wnp[5] = {T(0), T(0), T(0), T(0), T(0)}, qfp[5] = {T(0), T(0), T(0), T(0), T(0)};
   T vdt = T(0);
   uint8_t fl = 0;
   if (cell) {
-    b0 = R.beg[t];
-    b1 = R.beg[t + 1];
     for (int n = 0; n < 5; n++) {
       f[n] = A.fw[n * E + q];
       e[n] = A.dw[n * E + q];
@@ -1111,14 +1113,13 @@ __device__ __attribute__((always_inline)) inline void k_rec_body(const RecArgs<T
     if (A.coarse && !A.lfir1)
       for (int n = 0; n < 5; n++) qfp[n] = A.qf[n * E + q];
   }
-  if (o0 + tid < ch.w) {
-    const RecOp r = R.ops[o0 + tid];
+  if (r.rec >= 0) {
     kinds[tid] = r.kind;
     rec_op_value(R, r, val + tid * 10);
   }
   __syncthreads();
   if (!cell) return;
-  for (int o = b0 - o0; o < b1 - o0; o++) {
+  for (int o = sl.o0; o < sl.o1; o++) {
     const int kind = kinds[o];
     const double *v = val + o * 10;
     switch (kind) {

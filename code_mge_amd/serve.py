@@ -65,8 +65,8 @@ def level_bytes(n, es, nmir=0, mxcyc=4, viscous=False, coarse=False, psmoo=False
     padded by 64 bytes); wall-record arrays at their upper bound; a level
     below the finest also holds the prolongation's correction; the
     variable-coefficient smoother holds its coefficients and sweep scratch;
-    limiter freezing three 8-byte words per cell; the wall-record workgroup
-    ranges at one per touched cell at most"""
+    limiter freezing three 8-byte words per cell; the wall ops' places in
+    workgroups of 64 at twice the ops at most"""
     ni, nj, nk = n
     E = (ni + 4) * (nj + 4) * (nk + 4)
     nmax = max(ni, nj, nk) + 5
@@ -80,9 +80,9 @@ def level_bytes(n, es, nmir=0, mxcyc=4, viscous=False, coarse=False, psmoo=False
     if lfreeze:
         sizes += [24 * E]               # limiter words (three per cell)
     if nmir:
-        ntouch, nops = 2 * nmir, 6 * nmir
-        sizes += [DEVREC_BYTES * nmir, 40 * nmir, 8 * nmir, 8 * ntouch, 4 * (ntouch + 1), 48 * (nops + 1),
-                  16 * (ntouch + 1), 80 * (nops + 1)]
+        nops = 6 * nmir
+        nplace = 2 * nops + 64          # places of wall ops and cells: two workgroups of 64 hold over 64 ops
+        sizes += [DEVREC_BYTES * nmir, 40 * nmir, 8 * nmir, 16 * nplace, 48 * nplace, 80 * (nops + 1)]
         if viscous:                     # the viscous kernel's records by 16 x 4 x 4 tile
             sizes += [4 * (-(-ni // 16) * -(-nj // 4) * -(-nk // 4) + 1), 40 * nmir]
     return sum(s + 64 for s in sizes)
