@@ -93,7 +93,9 @@ struct Level {
   void *rw[3] = {nullptr, nullptr, nullptr}, *pw[3] = {nullptr, nullptr, nullptr};
   uint8_t *flags = nullptr, *marker = nullptr;
   void *dx = nullptr, *dy = nullptr, *dz = nullptr;
-  void *piv = nullptr;  // e1x,e2x,e1y,e2y,e1z,e2z,1/e1x,1/e1y,1/e1z each npiv
+  void *piv = nullptr;  // e1x,e2x,e1y,e2y,e1z,e2z each npiv
+  double *rpiv = nullptr;  // 1/e1x,1/e1y,1/e1z each npiv
+  void *fax = nullptr;  // FP32: -bb/e1x
   int npiv = 0;
   int nmir = 0, nupd = 0, zero_at = -1;
   bool cut_interior = false;  // every cloud cell inside the ghost shell (bcond writes none of them)
@@ -808,7 +810,7 @@ template <class T, int DIR>
 void launch_lines(mge_case *h, const char *name, const SmoothArgs<T> &S, bool run) {
   const Dims &d = S.d;
   const int n = DIR == 1 ? d.nj : d.nk, other = DIR == 1 ? d.nk : d.nj;
-  const SegShape sh = seg_shape(n);
+  const SegShape sh = seg_shape<T>(n);
   if (!run || sh.sx == 0) {
     const dim3 g = run ? dim3((d.ni + 63) / 64, other, 5) : dim3(0);
     if (DIR == 1) LAUNCHT(h, name, k_smooth_y, T, g, dim3(64), S);
@@ -846,35 +848,43 @@ void do_smooth(mge_case *h, Level &L) {
   S.bb = (T)h->smoo_bb;
   const T *piv = tp<T>(L.piv);
   const int np = L.npiv;
-  S.e1 = piv;
   S.e2 = piv + np;
-  S.r1 = piv + 6 * np;
-  const int cls = xy_class(d.ni, d.nj);
+  S.r1 = L.rpiv;
+  S.fa = tp<T>(L.fax);
+  const long nl = (long)d.nj * d.nk;
+  const int cls = xy_class<T>(d.ni, d.nj);
   if (cls >= 0) {
-    SmoothXYArgs<T> A{d, S.dw, S.flags, piv, piv + np, piv + 6 * np, piv + 2 * np, piv + 3 * np, piv + 7 * np, S.bb};
+    SmoothXYArgs<T> A{d, S.dw, S.flags, piv + np, piv + 3 * np, L.rpiv, L.rpiv + np, S.fa, S.bb};
     const dim3 g(d.nk, 5), b(kXY[cls].threads);
 #define XY(C) launch(h, "k_smooth_x", (const void *)&k_smooth_xy<T, C>, (const void *)&k_smooth_xy_b<T, C>, g, b, A)
     if (cls == 0) XY(0);
     else XY(1);
 #undef XY
+  } else if (d.ni > 512) {
+    LAUNCHT(h, "k_smooth_x", k_smooth_x_seq, T, flat_grid(nl * 5), dim3(256), S);
+  } else if constexpr (kDelta<T>) {
+#define XSCAN(C)                                                                                          \
+  launch(h, "k_smooth_x", (const void *)&k_smooth_x_scan<C>, (const void *)&k_smooth_x_scan_b<C>,         \
+         dim3((unsigned)(((nl * 5 + xscan_lines<C>() - 1) / xscan_lines<C>() + 3) / 4)), dim3(256), S)
+    if (d.ni <= 64) XSCAN(1);
+    else if (d.ni <= 128) XSCAN(2);
+    else if (d.ni <= 256) XSCAN(4);
+    else XSCAN(8);
+#undef XSCAN
   } else {
-    const long nl = (long)d.nj * d.nk;
 #define XSEG(N)                                                                                          \
-  launch(h, "k_smooth_x", (const void *)&k_smooth_xseg<T, N>, (const void *)&k_smooth_xseg_b<T, N>,      \
+  launch(h, "k_smooth_x", (const void *)&k_smooth_xseg<N>, (const void *)&k_smooth_xseg_b<N>,            \
          dim3((unsigned)((nl + xseg_rows<N>() - 1) / xseg_rows<N>()), 5), dim3(xseg_rows<N>() * N / 16), S)
     if (d.ni <= 128) XSEG(128);
     else if (d.ni <= 256) XSEG(256);
-    else if (d.ni <= 512) XSEG(512);
-    else LAUNCHT(h, "k_smooth_x", k_smooth_x_seq, T, flat_grid(nl * 5), dim3(256), S);
+    else XSEG(512);
 #undef XSEG
   }
-  S.e1 = piv + 2 * np;
   S.e2 = piv + 3 * np;
-  S.r1 = piv + 7 * np;
+  S.r1 = L.rpiv + np;
   launch_lines<T, 1>(h, "k_smooth_y", S, cls < 0);
-  S.e1 = piv + 4 * np;
   S.e2 = piv + 5 * np;
-  S.r1 = piv + 8 * np;
+  S.r1 = L.rpiv + 2 * np;
   launch_lines<T, 2>(h, "k_smooth_z", S, true);
 }
 
@@ -2133,7 +2143,9 @@ int mge_level_define(mge_case *h, int lvl, int ni, int nj, int nk, const double 
   CHKRC(dalloc_bytes(L, &L.dy, es * nmax));
   CHKRC(dalloc_bytes(L, &L.dz, es * nmax));
   L.npiv = nmax;
-  CHKRC(dalloc_bytes(L, &L.piv, es * 9 * nmax));
+  CHKRC(dalloc_bytes(L, &L.piv, es * 6 * nmax));
+  CHKRC(dalloc(L, &L.rpiv, 3 * nmax));
+  if (h->fp32) CHKRC(dalloc_bytes(L, &L.fax, es * nmax));
   dim3 g = cell_grid(d);
   L.npartial = (long)g.x * g.y * ((g.z + kRtrmsPlanes - 1) / kRtrmsPlanes);
   CHKRC(dalloc(L, &L.partial, L.npartial));
@@ -2182,7 +2194,7 @@ int mge_level_define(mge_case *h, int lvl, int ni, int nj, int nk, const double 
     L.hv[2].assign(zv, zv + d.kb + 1);
   }
   // smoothing pivots (psmoo.f90:134-166), computed once on the host in FP64
-  std::vector<double> piv((size_t)9 * nmax, 0.0);
+  std::vector<double> piv((size_t)6 * nmax, 0.0), rpiv((size_t)3 * nmax, 0.0);
   if (h->prm.smoo > 0.0) {
     double aa = 1.0 + 2.0 * h->prm.smoo, bb = -h->prm.smoo;
     int nn[3] = {ni, nj, nk};
@@ -2197,11 +2209,18 @@ int mge_level_define(mge_case *h, int lvl, int ni, int nj, int nk, const double 
         e2[s] = bb / e1[s];
       }
       e1[l] = aa - bb * e2[lm];
-      double *r1 = &piv[(size_t)(6 + a) * nmax];
-      for (int s = 2; s <= l; s++) r1[s] = 1.0 / e1[s];
+      double *r1 = &rpiv[(size_t)a * nmax];
+      for (int s = 2; s <= l; s++) r1[s] = 1.0 / (h->fp32 ? (double)(float)e1[s] : e1[s]);
     }
   }
   CHKRC(put_bulk(h, L.piv, piv.data(), piv.size()));
+  HIPCHK(h2d_sync(L.rpiv, rpiv.data(), sizeof(double) * rpiv.size(), h->stream));
+  if (L.fax) {
+    std::vector<double> fa(nmax, 0.0);
+    if (h->prm.smoo > 0.0 && ni >= 2)
+      for (int i = 2; i <= d.il; i++) fa[i] = h->prm.smoo / piv[i];  // bb = -smoo
+    CHKRC(put_bulk(h, L.fax, fa.data(), fa.size()));
+  }
   // flags: fluid bit with the ghost copies of init_metric.f90:207-218
   std::vector<uint8_t> bl(E, 1);
   auto X = [&](int i, int j, int k) { return ix(d, i, j, k); };

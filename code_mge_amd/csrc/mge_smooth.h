@@ -18,20 +18,21 @@ struct SmoothArgs {
   Dims d;
   T *dw;
   const uint8_t *flags;
-  const T *e1, *e2;  // pivots of this direction (psmoo.f90:134-166)
-  const T *r1;       // 1/e1, rounded once from the FP64 pivots
+  const T *e2;       // pivots of this direction (psmoo.f90:134-166)
+  const double *r1;  // 1/e1, e1 rounded to T first
+  const T *fa;       // x lines in FP32: -bb/e1
   T bb;
 };
 
-// The forward step's division by the pivot e1_s.  FP64 multiplies by the
-// reciprocal pivot instead (one rounding more per cell, a few ulp over a
-// line, and no FP64 division on the recurrence's critical path); FP32
-// divides, as the reference does.
+// The forward step's division by the pivot e1, r its reciprocal in FP64.
+// FP64 multiplies by the reciprocal (one rounding more per cell, a few ulp over
+// a line, and no FP64 division on the recurrence's critical path).  In FP32
+// this is the quotient the division gives, bit for bit: a quotient of two
+// 24-bit numbers that is no FP32 midpoint lies at least 2^-25 ulp from one, and
+// the FP64 product is within 2^-28 ulp of it.
 template <typename T>
-__device__ __attribute__((always_inline)) inline T piv_div(T x, const T *__restrict__ e1,
-                                                           const T *__restrict__ r1, int s) {
-  if constexpr (kDelta<T>) return x / e1[s];
-  else return x * r1[s];
+__device__ __attribute__((always_inline)) inline T piv_div(T x, double r) {
+  return (T)((double)x * r);
 }
 
 // sequential x lines for blocks wider than 512 cells
@@ -46,9 +47,9 @@ __device__ __attribute__((always_inline)) inline void smooth_x_seq(const SmoothA
   int j = 2 + (int)(l % d.nj), k = 2 + (int)(l / d.nj);
   T *D = S.dw + n * d.E;
   long b0 = ix(d, 0, j, k);
-  if (S.flags[b0 + 2] & F_FLUID) D[b0 + 2] = piv_div(D[b0 + 2], S.e1, S.r1, 2);
+  if (S.flags[b0 + 2] & F_FLUID) D[b0 + 2] = piv_div(D[b0 + 2], S.r1[2]);
   for (int i = 3; i <= d.il; i++)
-    if (S.flags[b0 + i] & F_FLUID) D[b0 + i] = piv_div(D[b0 + i] - S.bb * D[b0 + i - 1], S.e1, S.r1, i);
+    if (S.flags[b0 + i] & F_FLUID) D[b0 + i] = piv_div(D[b0 + i] - S.bb * D[b0 + i - 1], S.r1[i]);
   for (int i = 2; i <= d.ni; i++) {
     int ir = d.il + 1 - i;
     if (S.flags[b0 + ir] & F_FLUID) D[b0 + ir] = D[b0 + ir] - S.e2[ir] * D[b0 + ir + 1];
@@ -72,9 +73,9 @@ MGE_ENTRY_T(k_smooth_x_seq, SmoothArgs, 256, 1)
 // at s = nl with z(nl+1) = 0 and e2(nl) = 0, which returns y(nl) there.
 template <int CH, typename T>
 __device__ __attribute__((always_inline)) inline void line_sweep(T *__restrict__ D, const uint8_t *__restrict__ F,
-                                                                 long b0, long st, int nl, const T *__restrict__ e1,
-                                                                 const T *__restrict__ r1, const T *__restrict__ e2,
-                                                                 T bb) {
+                                                                 long b0, long st, int nl,
+                                                                 const double *__restrict__ r1,
+                                                                 const T *__restrict__ e2, T bb) {
   const int ncell = nl - 1;
   const int nfull = ncell / CH;
   T A[CH], B[CH], MA[CH], MB[CH];
@@ -88,7 +89,7 @@ __device__ __attribute__((always_inline)) inline void line_sweep(T *__restrict__
 #define PR_F(BUF, MK, c)                                              \
   _Pragma("unroll") for (int t = 0; t < CH; t++) {                    \
     int s_ = 2 + (c) * CH + t;                                        \
-    y = MK[t] * piv_div(BUF[t] - bb * y, e1, r1, s_);                 \
+    y = MK[t] * piv_div(BUF[t] - bb * y, r1[s_]);                 \
     D[b0 + (long)s_ * st] = y;                                        \
   }
 #define LD_B(BUF, MK, c)                                              \
@@ -119,7 +120,7 @@ __device__ __attribute__((always_inline)) inline void line_sweep(T *__restrict__
   for (int s_ = 2 + nfull * CH; s_ <= nl; s_++) {
     long q_ = b0 + (long)s_ * st;
     T m_ = (F[q_] & F_FLUID) ? T(1) : T(0);
-    y = m_ * piv_div(D[q_] - bb * y, e1, r1, s_);
+    y = m_ * piv_div(D[q_] - bb * y, r1[s_]);
     D[q_] = y;
   }
   // backward
@@ -156,7 +157,7 @@ __device__ __attribute__((always_inline)) inline void k_smooth_y_body(const Smoo
   int k = 2 + by;
   int n = bz;
   if (i > d.il) return;
-  line_sweep<8>(S.dw + n * d.E, S.flags, ix(d, i, 0, k), d.sy, d.jl, S.e1, S.r1, S.e2, S.bb);
+  line_sweep<8>(S.dw + n * d.E, S.flags, ix(d, i, 0, k), d.sy, d.jl, S.r1, S.e2, S.bb);
 }
 MGE_ENTRY_T_XCD(k_smooth_y, SmoothArgs, 64, 1)
 
@@ -168,49 +169,289 @@ __device__ __attribute__((always_inline)) inline void k_smooth_z_body(const Smoo
   int j = 2 + by;
   int n = bz;
   if (i > d.il) return;
-  line_sweep<8>(S.dw + n * d.E, S.flags, ix(d, i, j, 0), d.sz, d.kl, S.e1, S.r1, S.e2, S.bb);
+  line_sweep<8>(S.dw + n * d.E, S.flags, ix(d, i, j, 0), d.sz, d.kl, S.r1, S.e2, S.bb);
 }
 MGE_ENTRY_T_XCD(k_smooth_z, SmoothArgs, 64, 1)
+
+// ---- x lines in FP32: scanned across a wave -------------------------------
+//
+// Lane l of a group of W lanes owns the CPL cells s0 .. s0 + CPL - 1 of each of
+// K lines of n cells (ok: the cell is on the line, fl: fluid).  Both recurrences
+// are composed as affine maps (forward y_i = A_i y_(i-1) + B_i, backward z_i =
+// C_i z_(i+1) + y_i), scanned over the lanes, and each lane evaluates its own
+// cells with the reference formula from the value that enters.  pr: 1/e1, pa:
+// -bb/e1, pe2: e2 of the lane's cells.  FP32 keeps this order of operations
+// where FP64 joins segments: another order rounds the entering values
+// otherwise, and where a far-field face's normal velocity is next to 0 a last
+// bit decides between inflow and outflow (3e-3 of a cell's value).
+template <int CPL, int K>
+__device__ __attribute__((always_inline)) inline void scan_lines(float (&r)[K][CPL], const bool (&fl)[K][CPL],
+                                                                 const bool (&ok)[CPL], int s0, int n, int l, int W,
+                                                                 const double (&pr)[CPL], const float (&pa)[CPL],
+                                                                 const float (&pe2)[CPL], float bb) {
+  float Al[K], Bl[K];
+#pragma unroll
+  for (int t = 0; t < K; t++) {
+    Al[t] = 1.0f;
+    Bl[t] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CPL; c++) {
+      float A, B;
+      if (!ok[c]) { A = 1.0f; B = 0.0f; }
+      else if (!fl[t][c]) { A = 0.0f; B = r[t][c]; }
+      else if (s0 + c == 0) { A = 0.0f; B = piv_div(r[t][c], pr[c]); }
+      else { A = pa[c]; B = piv_div(r[t][c], pr[c]); }
+      Bl[t] = A * Bl[t] + B;
+      Al[t] = A * Al[t];
+    }
+  }
+  for (int off = 1; off < W; off <<= 1) {
+#pragma unroll
+    for (int t = 0; t < K; t++) {
+      const float Ap = __shfl_up(Al[t], off, W), Bp = __shfl_up(Bl[t], off, W);
+      if (l >= off) {
+        Bl[t] = Al[t] * Bp + Bl[t];
+        Al[t] = Al[t] * Ap;
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < K; t++) {
+    float yp = __shfl_up(Bl[t], 1, W);
+    if (l == 0) yp = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CPL; c++) {
+      float v = r[t][c];
+      if (fl[t][c]) v = piv_div(s0 + c == 0 ? r[t][c] : r[t][c] - bb * yp, pr[c]);
+      r[t][c] = v;
+      yp = v;
+    }
+  }
+  // backward: C_i = -e2_i on fluid cells but the line's last
+#pragma unroll
+  for (int t = 0; t < K; t++) {
+    Al[t] = 1.0f;
+    Bl[t] = 0.0f;
+#pragma unroll
+    for (int c = CPL - 1; c >= 0; c--) {
+      float C, D;
+      if (!ok[c]) { C = 1.0f; D = 0.0f; }
+      else if (fl[t][c] && s0 + c < n - 1) { C = -pe2[c]; D = r[t][c]; }
+      else { C = 0.0f; D = r[t][c]; }
+      Bl[t] = C * Bl[t] + D;
+      Al[t] = C * Al[t];
+    }
+  }
+  for (int off = 1; off < W; off <<= 1) {
+#pragma unroll
+    for (int t = 0; t < K; t++) {
+      const float Cn = __shfl_down(Al[t], off, W), Dn = __shfl_down(Bl[t], off, W);
+      if (l + off < W) {
+        Bl[t] = Al[t] * Dn + Bl[t];
+        Al[t] = Al[t] * Cn;
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < K; t++) {
+    float zn = __shfl_down(Bl[t], 1, W);
+    if (l == W - 1) zn = 0.0f;
+#pragma unroll
+    for (int c = CPL - 1; c >= 0; c--) {
+      if (!ok[c]) continue;
+      if (fl[t][c] && s0 + c < n - 1) r[t][c] = r[t][c] - pe2[c] * zn;
+      zn = r[t][c];
+    }
+  }
+}
+
+// a lane moves its CPL cells as pairs when CPL is even, the line's first
+// cell (i = 2) sits on a pair boundary (so does every lane's first cell,
+// i0 - 2 being a multiple of CPL) and all its cells are inside the line
+template <int CPL>
+__device__ __attribute__((always_inline)) inline bool xscan_pairs(const float *row, int i0, int il) {
+  if constexpr (CPL % 2 != 0) return false;
+  else return ((reinterpret_cast<uintptr_t>(row + 2) & (2 * sizeof(float) - 1)) == 0) && i0 + CPL - 1 <= il;
+}
+
+// x lines of levels whose planes do not fit k_smooth_xy: a wave takes K
+// consecutive (j,k) lines of a component; the lines' loads are in flight
+// together and their shuffles interleave.  Four lines of up to 256 cells
+// share a wave, 512-cell lines take one (256^3: one, two and four lines 409,
+// 339 and 324 us with single loads; with pairs, four lines 304 us; with the
+// quotients by reciprocal pivots 250 us).
+template <int CPL>
+constexpr int xscan_lines() { return CPL >= 8 ? 1 : 4; }
+template <int CPL>
+__device__ __attribute__((always_inline)) inline void smooth_x_scan(const SmoothArgs<float> &S, int bx) {
+  constexpr int K = xscan_lines<CPL>();
+  const Dims &d = S.d;
+  const int lane = threadIdx.x & 63;
+  // the wave index is uniform: keep the line arithmetic scalar
+  const int wave = __builtin_amdgcn_readfirstlane((int)((bx * (long)blockDim.x + threadIdx.x) >> 6));
+  const int nl = d.nj * d.nk, nlines = nl * 5, l0 = wave * K;
+  if (l0 >= nlines) return;  // uniform per wave
+  const int il = d.il, i0 = 2 + lane * CPL;
+  double pr[CPL];
+  float pa[CPL], pe2[CPL];
+  bool ok[CPL];
+#pragma unroll
+  for (int c = 0; c < CPL; c++) {
+    ok[c] = i0 + c <= il;
+    const int ic = ok[c] ? i0 + c : 2;
+    pr[c] = S.r1[ic];
+    pa[c] = S.fa[ic];
+    pe2[c] = S.e2[ic];
+  }
+  float r[K][CPL];
+  bool fl[K][CPL];
+  long base[K];
+#pragma unroll
+  for (int t = 0; t < K; t++) {
+    const int lc = l0 + t < nlines ? l0 + t : l0;  // a missing line repeats the first; it is never stored
+    const int n = lc / nl, l = lc - n * nl;
+    const long f = ix(d, 0, 2 + l % d.nj, 2 + l / d.nj);
+    base[t] = (long)n * d.E + f;
+    if (xscan_pairs<CPL>(S.dw + base[t], i0, il)) {
+      const float2 *pp = reinterpret_cast<const float2 *>(S.dw + base[t] + i0);
+#pragma unroll
+      for (int h = 0; h < CPL / 2; h++) {
+        const float2 v = pp[h];
+        r[t][2 * h] = v.x;
+        r[t][2 * h + 1] = v.y;
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < CPL; c++) r[t][c] = ok[c] ? S.dw[base[t] + i0 + c] : 0.0f;
+    }
+#pragma unroll
+    for (int c = 0; c < CPL; c++) fl[t][c] = ok[c] && (S.flags[f + i0 + c] & F_FLUID);
+  }
+  scan_lines<CPL, K>(r, fl, ok, i0 - 2, d.ni, lane, 64, pr, pa, pe2, S.bb);
+#pragma unroll
+  for (int t = 0; t < K; t++) {
+    if (l0 + t >= nlines) continue;
+    if (xscan_pairs<CPL>(S.dw + base[t], i0, il)) {
+      // blank cells are written back with the value they were read with
+      float2 *pp = reinterpret_cast<float2 *>(S.dw + base[t] + i0);
+#pragma unroll
+      for (int h = 0; h < CPL / 2; h++) pp[h] = float2{r[t][2 * h], r[t][2 * h + 1]};
+    } else {
+#pragma unroll
+      for (int c = 0; c < CPL; c++)
+        if (fl[t][c]) S.dw[base[t] + i0 + c] = r[t][c];
+    }
+  }
+}
+// one pair of entry points per scan width; a batch launches each width once
+// over the cases that use it
+template <int CPL>
+__global__ void __launch_bounds__(256) k_smooth_x_scan(SmoothArgs<float> S) {
+  smooth_x_scan<CPL>(S, (int)blockIdx.x);
+}
+template <int CPL>
+__global__ void __launch_bounds__(256) k_smooth_x_scan_b(const SmoothArgs<float> *As, const int4 *cg, int nc,
+                                                         const int *act) {
+  const int b = (int)blockIdx.x;
+  const int c = batch_case(cg, nc, b);
+  const int4 g = cg[c];
+  if (!act[g.w]) return;
+  smooth_x_scan<CPL>(As[c], b - g.x);
+}
 
 // ---- lines in segments ---------------------------------------------------
 //
 // A line split into segments of L cells, one thread each, all of its cells in
-// registers and the segments joined through LDS.  Both
-// recurrences are evaluated within the segment from zero, giving the
-// segment's map from the value entering it to the value leaving it; every
+// registers; the segments are joined through LDS.
+//
+// FP64: both recurrences are evaluated within the segment from zero, giving
+// the segment's map from the value entering it to the value leaving it; every
 // thread then runs through the maps before (backward: after) it and
 // re-evaluates its cells with the reference formula from the value entering.
+// The entering values are a few ulp from the sequential ones.
+//
+// FP32: the bits of the sequential recurrence.  Every segment evaluates its
+// cells from the value its neighbour leaves, and again as long as that value
+// changes, up to the cell from which nothing changes any more.  Segment g is
+// final after g rounds at the latest; as a change shrinks by bb/e1 a cell (0.3
+// at the default coefficient, 4e-9 over 16 cells), the third round mostly ends
+// it.  Thread per line -> this -> joined by maps as FP64 (other last bits), y
+// lines: 96^3 31 -> 20 -> 15.5 us, 256^3 243 -> 199 -> 185 us.
+//
 // Branch-free: a cell's fluid bit selects its pivots or zeros (blank cells
 // hold dw = +-0, see line_sweep, and come out as 0), and the places past the
 // line's end count as blank; a branch per cell would wait for every LDS read
 // by itself (64^3 in k_smooth_xy: 25 us with branches, 13 without).
 // Called by all threads of the workgroup (barriers); sa, sb, sc, sd: LDS of
-// G x nline values each; `act` threads hold segment g of line `line`.
+// G x nline values each (FP32: sa and sc alone); `act` threads hold segment g
+// of line `line`.
 template <typename T>
 struct SegPiv {   // a line's pivots, in LDS, indexed by cell from 0
-  const T *e1, *r1, *e2;
+  const double *r1;
+  const T *e2;
 };
-// x / e1 on a fluid cell, 0 on a blank one (rm: r1 or 0).  FP64 multiplies by
-// the reciprocal pivot; FP32 corrects the product by its remainder, which
-// gives the quotient the reference's division gives
-template <typename T>
-__device__ inline T seg_div(T x, T e1, T rm) {
-  const T q = x * rm;
-  if constexpr (kDelta<T>) return __builtin_fmaf(__builtin_fmaf(-e1, q, x), rm, q);
-  else return q;
+template <int L>
+__device__ __attribute__((always_inline)) inline void seg_solve(bool act, float (&r)[L], unsigned fl, int s0, int g,
+                                                                int G, int line, int nline, const SegPiv<float> &P,
+                                                                float bb, float *sa, float *, float *sc, float *) {
+  auto rm = [&](int c) { return (fl >> c) & 1u ? P.r1[s0 + c] : 0.0; };
+  auto qm = [&](int c) { return (fl >> c) & 1u ? P.e2[s0 + c] : 0.0f; };
+  float v[L], in = 0.0f;
+  bool again;
+  // takes `in` from segment nb's place (none: zero); whether any thread's changed
+  auto join = [&](const float *s, int nb, bool none) {
+    __syncthreads();
+    const float x = act && !none ? s[nb * nline + line] : 0.0f;
+    again = __float_as_uint(x) != __float_as_uint(in);
+    in = x;
+    return __syncthreads_or(again) != 0;
+  };
+  // cell c's new value; true every fourth cell if no thread's value there changed
+  auto put = [&](float &o, float x, int c, bool first) {
+    const bool diff = __float_as_uint(x) != __float_as_uint(o);
+    o = x;
+    return !first && c % 4 == 3 && !__any(diff);
+  };
+  auto forward = [&](bool first) {
+    float y = in;
+#pragma unroll
+    for (int c = 0; c < L; c++) {
+      y = piv_div(r[c] - bb * y, rm(c));
+      if (put(v[c], y, c, first)) return;
+    }
+    if (act) sa[g * nline + line] = y;
+  };
+  forward(true);
+  for (int it = 1; it < G && join(sa, g - 1, g == 0); it++)   // uniform
+    if (again) forward(false);
+  // backward: z = y - e2 z', e2 = 0 on the line's last cell
+  in = 0.0f;
+  auto backward = [&](bool first) {
+    float z = in;
+#pragma unroll
+    for (int c = 0; c < L; c++) {
+      const int b = L - 1 - c;
+      z = v[b] - qm(b) * z;
+      if (put(r[b], z, c, first)) return;
+    }
+    if (act) sc[g * nline + line] = z;
+  };
+  backward(true);
+  for (int it = 1; it < G && join(sc, g + 1, g == G - 1); it++)
+    if (again) backward(false);
 }
-template <int L, typename T>
-__device__ __attribute__((always_inline)) inline void seg_solve(bool act, T (&r)[L], unsigned fl, int s0, int g, int G,
-                                                                int line, int nline, const SegPiv<T> &P, T bb, T *sa,
-                                                                T *sb, T *sc, T *sd) {
-  auto rm = [&](int c) { return (fl >> c) & 1u ? P.r1[s0 + c] : T(0); };
-  auto e1 = [&](int c) { if constexpr (kDelta<T>) return P.e1[s0 + c]; else return T(0); };
-  auto qm = [&](int c) { return (fl >> c) & 1u ? P.e2[s0 + c] : T(0); };
-  T A = T(1), B = T(0);
+template <int L>
+__device__ __attribute__((always_inline)) inline void seg_solve(bool act, double (&r)[L], unsigned fl, int s0, int g,
+                                                                int G, int line, int nline, const SegPiv<double> &P,
+                                                                double bb, double *sa, double *sb, double *sc,
+                                                                double *sd) {
+  auto rm = [&](int c) { return (fl >> c) & 1u ? P.r1[s0 + c] : 0.0; };
+  auto qm = [&](int c) { return (fl >> c) & 1u ? P.e2[s0 + c] : 0.0; };
+  double A = 1.0, B = 0.0;
 #pragma unroll
   for (int c = 0; c < L; c++) {
-    const T m = rm(c);
-    B = seg_div(r[c] - bb * B, e1(c), m);
+    const double m = rm(c);
+    B = piv_div(r[c] - bb * B, m);
     A = A * (-bb * m);
   }
   if (act) {
@@ -218,21 +459,21 @@ __device__ __attribute__((always_inline)) inline void seg_solve(bool act, T (&r)
     sb[g * nline + line] = B;
   }
   __syncthreads();
-  T y = T(0);
+  double y = 0.0;
   for (int q = 0; q < G - 1; q++) {   // uniform; the maps before this segment
-    const T ny = sa[q * nline + line] * y + sb[q * nline + line];
+    const double ny = sa[q * nline + line] * y + sb[q * nline + line];
     y = q < g ? ny : y;
   }
-  T C = T(1), D = T(0);
+  double C = 1.0, D = 0.0;
 #pragma unroll
   for (int c = 0; c < L; c++) {
-    y = seg_div(r[c] - bb * y, e1(c), rm(c));
+    y = piv_div(r[c] - bb * y, rm(c));
     r[c] = y;
   }
   // backward: z = y - e2 z', e2 = 0 on the line's last cell
 #pragma unroll
   for (int c = L - 1; c >= 0; c--) {
-    const T m = qm(c);
+    const double m = qm(c);
     D = r[c] - m * D;
     C = -(m * C);
   }
@@ -241,9 +482,9 @@ __device__ __attribute__((always_inline)) inline void seg_solve(bool act, T (&r)
     sd[g * nline + line] = D;
   }
   __syncthreads();
-  T z = T(0);
+  double z = 0.0;
   for (int q = G - 1; q > 0; q--) {
-    const T nz = sc[q * nline + line] * z + sd[q * nline + line];
+    const double nz = sc[q * nline + line] * z + sd[q * nline + line];
     z = q > g ? nz : z;
   }
 #pragma unroll
@@ -266,9 +507,13 @@ struct SmoothXYArgs {
   Dims d;
   T *dw;
   const uint8_t *flags;
-  const T *e1x, *e2x, *r1x, *e1y, *e2y, *r1y;
+  const T *e2x, *e2y;
+  const double *r1x, *r1y;
+  const T *fax;
   T bb;
 };
+// FP32 scans its x lines while it reads them (scan_lines; rows of up to 64
+// cells, one cell a lane): x and y of 48^3 24 us in two launches, 18 in this.
 // plane classes: cells of LDS (rows of nx | 1), mask words, pivots per
 // direction, threads, segment length.  Planes of more than 64 x 65 cells leave
 // too few workgroups a CU: 128 x 128 x 4 took 21 us in one launch, 11 in two.
@@ -277,7 +522,9 @@ struct XYClass {
 };
 constexpr XYClass kXY[2] = {{2560, 128, 264, 512, 8}, {4416, 256, 264, 512, 8}};
 // the class that holds an nx x ny plane (-1: none)
-inline int xy_class(int nx, int ny) {
+template <typename T>
+int xy_class(int nx, int ny) {
+  if (kDelta<T> && nx > 64) return -1;
   for (int c = 0; c < 2; c++) {
     const XYClass &K = kXY[c];
     const int gx = (nx + K.seg - 1) / K.seg, gy = (ny + K.seg - 1) / K.seg;
@@ -292,22 +539,22 @@ inline int xy_class(int nx, int ny) {
 template <typename T, int CLS>
 __device__ __attribute__((always_inline)) inline void k_smooth_xy_body(const SmoothXYArgs<T> &S, int bx, int by) {
   constexpr XYClass K = kXY[CLS];
-  constexpr int L = K.seg, NP = kDelta<T> ? 3 : 2;
+  constexpr int L = K.seg;
+  constexpr bool SCAN = kDelta<T>;
   __shared__ T pl[K.cells];
-  __shared__ T pv[2][NP][K.piv];   // x, y: 1/e1, e2 (and e1 in FP32)
+  __shared__ double pr[SCAN ? 1 : 2][K.piv];   // y, x: 1/e1
+  __shared__ T pe[SCAN ? 1 : 2][K.piv];        // y, x: e2
   __shared__ unsigned long long mk[K.words];
   const Dims &d = S.d;
   const int nx = d.ni, ny = d.nj, P = nx | 1, nch = (nx + 63) >> 6;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int t = tid; t < K.piv; t += K.threads) {
     const int ix2 = 2 + min(t, nx - 1), iy2 = 2 + min(t, ny - 1);
-    pv[0][0][t] = S.r1x[ix2];
-    pv[0][1][t] = S.e2x[ix2];
-    pv[1][0][t] = S.r1y[iy2];
-    pv[1][1][t] = S.e2y[iy2];
-    if constexpr (kDelta<T>) {
-      pv[0][NP - 1][t] = S.e1x[ix2];
-      pv[1][NP - 1][t] = S.e1y[iy2];
+    pr[0][t] = S.r1y[iy2];
+    pe[0][t] = S.e2y[iy2];
+    if constexpr (!SCAN) {
+      pr[1][t] = S.r1x[ix2];
+      pe[1][t] = S.e2x[ix2];
     }
   }
   // rows by groups of lp lanes (a power of two), RW rows a wave
@@ -317,6 +564,14 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xy_body(const Smo
   T *D = S.dw + by * d.E + base;
   const uint8_t *F = S.flags + base;
   constexpr int NW = K.threads / 64, U = 8;
+  double xr[1];   // FP32: the pivots of the lane's cell
+  T xa[1], xe2[1];
+  if constexpr (SCAN) {
+    const int ic = 2 + min(l, nx - 1);
+    xr[0] = S.r1x[ic];
+    xa[0] = S.fax[ic];
+    xe2[0] = S.e2x[ic];
+  }
   for (int ch = 0; ch < nch; ch++) {
     const int i = (ch << 6) + l, ic = min(i, nx - 1);
     for (int t0 = wave * RW + sub; t0 - sub < ny; t0 += NW * RW * U) {
@@ -327,6 +582,19 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xy_body(const Smo
         const long q = (long)min(t0 + u * NW * RW, ny - 1) * d.sy + ic;
         v[u] = D[q];
         f[u] = F[q];
+      }
+      if constexpr (SCAN) {
+        T x[U][1];
+        bool xf[U][1];
+        const bool ok[1] = {i < nx};
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          x[u][0] = v[u];
+          xf[u][0] = ok[0] && (f[u] & F_FLUID);
+        }
+        scan_lines<1, U>(x, xf, ok, i, nx, l, lp, xr, xa, xe2, S.bb);
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = x[u][0];
       }
 #pragma unroll
       for (int u = 0; u < U; u++) {
@@ -341,7 +609,7 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xy_body(const Smo
   }
   __syncthreads();
   T r[L];
-  {  // x lines
+  if constexpr (!SCAN) {  // x lines
     const int G = (nx + L - 1) / L, line = tid % ny, g = tid / ny;
     const bool act = g < G;
     const int i0 = act ? g * L : 0, m = act ? min(L, nx - i0) : 0;
@@ -353,7 +621,7 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xy_body(const Smo
     for (int c = 0; c < L; c++) r[c] = row[min(i0 + c, nx - 1)];
     __syncthreads();
     const int n = G * ny;
-    seg_solve<L>(act, r, fl, i0, g, G, line, ny, SegPiv<T>{pv[0][NP - 1], pv[0][0], pv[0][1]}, S.bb, pl, pl + n,
+    seg_solve<L>(act, r, fl, i0, g, G, line, ny, SegPiv<T>{pr[1], pe[1]}, S.bb, pl, pl + n,
                  pl + 2 * n, pl + 3 * n);
     __syncthreads();
 #pragma unroll
@@ -375,7 +643,7 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xy_body(const Smo
     }
     __syncthreads();
     const int n = G * nx;
-    seg_solve<L>(act, r, fl, j0, g, G, line, nx, SegPiv<T>{pv[1][NP - 1], pv[1][0], pv[1][1]}, S.bb, pl, pl + n,
+    seg_solve<L>(act, r, fl, j0, g, G, line, nx, SegPiv<T>{pr[0], pe[0]}, S.bb, pl, pl + n,
                  pl + 2 * n, pl + 3 * n);
     __syncthreads();
 #pragma unroll
@@ -411,21 +679,24 @@ __global__ void __launch_bounds__(kXY[CLS].threads)
 // cells are one segment (64 lines a wave), up to 256 cells 32 lines in 16
 // segments of 8 or 16, up to 512 cells 16 lines in 32.  Bound by the field's
 // one read and write where the level is large.  Thread per line before ->
-// this, y lines: 256^3 FP64 421 -> 296 us (4.6 TB/s), FP32 243 -> 183 us;
-// 128^3 46 -> 32 us; 512 x 512 x 4 105 -> 26 us.
+// this, FP64 y lines: 256^3 421 -> 296 us (4.6 TB/s); 128^3 46 -> 32 us; 512 x
+// 512 x 4 105 -> 26 us.  FP32 takes 16 cells beyond 16: the fewer rounds (96^3
+// 25 us with 8).
 struct SegShape {
   int sx, len;   // lines side by side, cells per segment (0: too long)
 };
-inline SegShape seg_shape(int n) {
+template <typename T>
+SegShape seg_shape(int n) {
   if (n <= 16) return SegShape{64, n <= 4 ? 4 : (n <= 8 ? 8 : 16)};
-  if (n <= 256) return SegShape{32, n <= 128 ? 8 : 16};
+  if (n <= 256) return SegShape{32, n <= 128 && !kDelta<T> ? 8 : 16};
   return n <= 512 ? SegShape{16, 16} : SegShape{0, 0};
 }
 template <typename T, int SX, int L, int DIR>
 __device__ __attribute__((always_inline)) inline void k_smooth_seg_body(const SmoothArgs<T> &S, int bx, int by,
                                                                         int bz) {
-  constexpr int NP = kDelta<T> ? 3 : 2, GM = SX == 64 ? 1 : 512 / SX;
-  __shared__ T sh[4][GM * SX], pv[NP][L * GM];
+  constexpr int GM = SX == 64 ? 1 : 512 / SX;
+  __shared__ T sh[4][GM * SX], pe[L * GM];
+  __shared__ double pr[L * GM];
   const Dims &d = S.d;
   const int n = DIR == 1 ? d.nj : d.nk, G = (n + L - 1) / L;
   const long st = DIR == 1 ? d.sy : d.sz;
@@ -446,12 +717,11 @@ __device__ __attribute__((always_inline)) inline void k_smooth_seg_body(const Sm
   }
   for (int t = threadIdx.x; t < G * L; t += blockDim.x) {
     const int s = 2 + min(t, n - 1);
-    pv[0][t] = S.r1[s];
-    pv[1][t] = S.e2[s];
-    if constexpr (kDelta<T>) pv[NP - 1][t] = S.e1[s];
+    pr[t] = S.r1[s];
+    pe[t] = S.e2[s];
   }
   __syncthreads();
-  seg_solve<L>(act, r, fl, s0, g, G, line, SX, SegPiv<T>{pv[NP - 1], pv[0], pv[1]}, S.bb, sh[0], sh[1], sh[2], sh[3]);
+  seg_solve<L>(act, r, fl, s0, g, G, line, SX, SegPiv<T>{pr, pe}, S.bb, sh[0], sh[1], sh[2], sh[3]);
 #pragma unroll
   for (int c = 0; c < L; c++)
     if (c < m) D[(long)(s0 + c) * st] = r[c];
@@ -473,32 +743,31 @@ __global__ void __launch_bounds__(SX == 64 ? 64 : 512)
   k_smooth_seg_body<T, SX, L, DIR>(As[c], l % g.y, (l / g.y) % g.z, l / (g.y * g.z));
 }
 
-// x lines in segments of 16 cells, where the planes do not fit k_smooth_xy:
+// FP64 x lines in segments of 16 cells, where the planes do not fit k_smooth_xy:
 // a workgroup stages 16 (N = 128: 32) rows of up to N cells in LDS (whole rows,
 // so loads and stores are coalesced), each thread takes a segment.  With lines
 // scanned across a wave's lanes by shuffles -> this: 256^3 FP64 399 -> 286 us
-// (4.7 TB/s), FP32 291 -> 201 us; 128^3 54 -> 48 us; 96^3 33 -> 24 us.
+// (4.7 TB/s); 128^3 54 -> 48 us; 96^3 33 -> 24 us.
 template <int N>
 constexpr int xseg_rows() { return N == 128 ? 32 : 16; }
-template <typename T, int N>
-__device__ __attribute__((always_inline)) inline void k_smooth_xseg_body(const SmoothArgs<T> &S, int bx, int by) {
-  constexpr int NP = kDelta<T> ? 3 : 2, L = 16, kXR = xseg_rows<N>(), NT = kXR * N / L, NW = NT / 64;
-  __shared__ T pl[kXR * (N + 1)], pv[NP][N];
+template <int N>
+__device__ __attribute__((always_inline)) inline void k_smooth_xseg_body(const SmoothArgs<double> &S, int bx, int by) {
+  constexpr int L = 16, kXR = xseg_rows<N>(), NT = kXR * N / L, NW = NT / 64;
+  __shared__ double pl[kXR * (N + 1)], pr[N], pe[N];
   __shared__ unsigned long long mk[kXR * N / 64];
   const Dims &d = S.d;
   const int nx = d.ni, P = nx | 1, nch = (nx + 63) >> 6, G = (nx + L - 1) / L;
   const int nl = d.nj * d.nk, l0 = bx * kXR, rows = min(kXR, nl - l0);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  T *D = S.dw + by * d.E;
+  double *D = S.dw + by * d.E;
   auto at = [&](int row) {   // the first cell of the workgroup's row
     const int l = l0 + min(row, rows - 1), k = l / d.nj;
     return ix(d, 2, 2 + l - k * d.nj, 2 + k);
   };
   for (int t = tid; t < G * L; t += NT) {
     const int s = 2 + min(t, nx - 1);
-    pv[0][t] = S.r1[s];
-    pv[1][t] = S.e2[s];
-    if constexpr (kDelta<T>) pv[NP - 1][t] = S.e1[s];
+    pr[t] = S.r1[s];
+    pe[t] = S.e2[s];
   }
   constexpr int RW = kXR / NW;                      // rows of a wave
   constexpr int U = N / 64;                         // chunks of a row
@@ -506,7 +775,7 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xseg_body(const S
   for (int u = 0; u < RW; u++) {
     const int row = wave * RW + u;
     const long q = at(row);
-    T v[U];
+    double v[U];
     uint8_t f[U];
 #pragma unroll
     for (int c = 0; c < U; c++) {
@@ -527,12 +796,12 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xseg_body(const S
   const bool act = g < G;
   const int i0 = act ? g * L : 0, m = act ? min(L, nx - i0) : 0;
   const unsigned fl = (unsigned)(mk[(i0 >> 6) * kXR + line] >> (i0 & 63)) & 0xffffu;
-  T r[L];
+  double r[L];
 #pragma unroll
   for (int c = 0; c < L; c++) r[c] = pl[line * P + min(i0 + c, nx - 1)];
   __syncthreads();
   const int n = G * kXR;
-  seg_solve<L>(act, r, fl, i0, g, G, line, kXR, SegPiv<T>{pv[NP - 1], pv[0], pv[1]}, S.bb, pl, pl + n, pl + 2 * n,
+  seg_solve<L>(act, r, fl, i0, g, G, line, kXR, SegPiv<double>{pr, pe}, S.bb, pl, pl + n, pl + 2 * n,
                pl + 3 * n);
   __syncthreads();
 #pragma unroll
@@ -547,25 +816,25 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xseg_body(const S
 #pragma unroll
     for (int c = 0; c < U; c++) {
       const int i = c * 64 + lane;
-      if (i < nx) D[q + i] = pl[row * P + i];   // blank cells: as they were read
+      if (i < nx) D[q + i] = pl[row * P + i];   // blank cells: 0
     }
   }
 }
-template <typename T, int N>
-__global__ void __launch_bounds__(xseg_rows<N>() * N / 16) k_smooth_xseg(SmoothArgs<T> S) {
+template <int N>
+__global__ void __launch_bounds__(xseg_rows<N>() * N / 16) k_smooth_xseg(SmoothArgs<double> S) {
   int bx, by, bz;
   xcd_block(bx, by, bz);
-  k_smooth_xseg_body<T, N>(S, bx, by);
+  k_smooth_xseg_body<N>(S, bx, by);
 }
-template <typename T, int N>
+template <int N>
 __global__ void __launch_bounds__(xseg_rows<N>() * N / 16)
-    k_smooth_xseg_b(const SmoothArgs<T> *As, const int4 *cg, int nc, const int *act) {
+    k_smooth_xseg_b(const SmoothArgs<double> *As, const int4 *cg, int nc, const int *act) {
   const int b = (int)blockIdx.x;
   const int c = batch_case(cg, nc, b);
   const int4 g = cg[c];
   if (!act[g.w]) return;
   const int l = b - g.x;
-  k_smooth_xseg_body<T, N>(As[c], l % g.y, l / g.y);
+  k_smooth_xseg_body<N>(As[c], l % g.y, l / g.y);
 }
 
 // ---- psmoo (psmoo.f90:1-95) with progon3's sweep (progon3.f90:1-62) ------
