@@ -47,6 +47,20 @@ inline void xfer_user(int delta) {
   }
 }
 
+// The case's device as the thread's current one for a scope: an event records
+// only on streams of the device it was made on, and a caller's current device
+// may be another.
+struct DeviceScope {
+  int prev = 0;
+  hipError_t rc;
+  explicit DeviceScope(int dev) : rc(hipGetDevice(&prev)) {
+    if (rc == hipSuccess && prev != dev) rc = hipSetDevice(dev);
+  }
+  ~DeviceScope() { if (rc == hipSuccess) hipSetDevice(prev); }
+  DeviceScope(const DeviceScope &) = delete;
+  DeviceScope &operator=(const DeviceScope &) = delete;
+};
+
 // One transfer of `bytes` bytes: up = false, device -> host: move(piece
 // offset, pinned piece, length) empties a piece the copy engine has filled;
 // up = true: it fills a piece, which is then copied to the device.  Returns
@@ -54,6 +68,8 @@ inline void xfer_user(int delta) {
 template <class Move>
 hipError_t xfer(int dev, hipStream_t stream, void *dptr, size_t bytes, bool up, Move move) {
   if (bytes == 0) return hipSuccess;
+  const DeviceScope on(dev);
+  if (on.rc != hipSuccess) return on.rc;
   hipError_t e = hipStreamSynchronize(stream);
   if (e != hipSuccess) return e;
   XferRing &R = xfer_ring();
