@@ -359,8 +359,11 @@ int check_err(mge_case *h, const double *r = nullptr) {
     h->launch_err = hipSuccess;
     return set_err(MGE_ERR_HIP, b);
   }
-  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, h->stream, r, (const int *)h->err, h->word);
-  if (hipGetLastError() != hipSuccess) return set_err(MGE_ERR_HIP, "error-flag read failed");
+  // the launch's own status: the thread's last error may be another caller's
+  const int *ep = h->err;
+  void *p[3] = {(void *)&r, (void *)&ep, (void *)&h->word};
+  if (hipLaunchKernel((const void *)&k_publish, dim3(1), dim3(64), p, 0, h->stream) != hipSuccess)
+    return set_err(MGE_ERR_HIP, "error-flag read failed");
   if (hipStreamSynchronize(h->stream) != hipSuccess) return set_err(MGE_ERR_HIP, "stream sync failed");
   const int e = h->word->err;
   if (h->timing) resolve_timers(h);
