@@ -2424,7 +2424,7 @@ int mge_download(mge_case *h, int lvl, int blk, const char *field, double *out) 
   if (!p) return set_err(MGE_ERR_ARG, "unknown field");
   if (!h->fp32) {
     HIPCHK(xfer(h->dev, h->stream, p, sizeof(double) * n, false,
-                [&](size_t o, const char *t, size_t len) { std::memcpy((char *)out + o, t, len); }));
+                [&](size_t o, const char *t, size_t len) { std::memcpy((char *)out + o, t, len); }, out));
     return check_err(h);
   }
   const int nc = state_field(field);
@@ -2451,7 +2451,7 @@ int mge_upload(mge_case *h, int lvl, int blk, const char *field, const double *i
   if (!p) return set_err(MGE_ERR_ARG, "unknown field");
   if (!h->fp32) {
     HIPCHK(xfer(h->dev, h->stream, p, sizeof(double) * n, true,
-                [&](size_t o, char *t, size_t len) { std::memcpy(t, (const char *)in + o, len); }));
+                [&](size_t o, char *t, size_t len) { std::memcpy(t, (const char *)in + o, len); }, (void *)in));
     return MGE_OK;
   }
   const int nc = state_field(field);
@@ -2689,7 +2689,7 @@ int do_upload_solut(mge_case *h, Level &L, double ptot, double *host, int nval) 
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
     e = xfer(h->dev, h->stream, dev, sizeof(double) * nval * nc, false,
-             [&](size_t o, const char *t, size_t len) { std::memcpy((char *)host + o, t, len); });
+             [&](size_t o, const char *t, size_t len) { std::memcpy((char *)host + o, t, len); }, host);
   hipError_t f = hipFreeAsync(dev, h->stream);
   if (e == hipSuccess) e = f;
   if (e != hipSuccess) return set_err(MGE_ERR_HIP, hipGetErrorString(e));

@@ -7,7 +7,9 @@
 // 0.7 GB state of a 256^3 level took 70 ms, three multigrid cycles' time.
 // Here the copy engine fills a ring of pinned pieces while several threads
 // empty (or fill) them, converting on the way; the caller's memory is first
-// touched by those threads too.
+// touched by those threads too.  A ring is one transfer's at a time; a transfer
+// that finds all of them taken, or no pinned memory, goes the runtime's way by
+// itself, so that cases never wait for each other.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -22,27 +24,34 @@
 namespace mge {
 
 constexpr size_t kPiece = 2u << 20;   // bytes of one piece
-constexpr int kPieces = 8;            // pieces of the ring
+constexpr int kPieces = 8;            // pieces of a ring
+constexpr int kRings = 4;             // rings of the process
 constexpr int kXferThreads = 8;       // threads of one transfer, the caller's among them
 
-// The process's one ring: allocated by the first large transfer, freed with
-// the last case.  A transfer holds `mu` (the copy engine and the memory bus
-// are shared anyway), after waiting for its case's stream without it.
+// The process's rings: each allocated by the first transfer that takes it, all
+// freed with the last case.  A transfer holds the mutex of a ring that it gets
+// at once, after waiting for its case's stream without it.
 struct XferRing {
   std::mutex mu;
-  int users = 0;         // live cases
   char *buf = nullptr;   // kPieces * kPiece bytes
 };
-inline XferRing &xfer_ring() {
-  static XferRing r;
-  return r;
+struct XferPool {
+  std::mutex mu;
+  int users = 0;         // live cases
+  XferRing ring[kRings];
+};
+inline XferPool &xfer_pool() {
+  static XferPool p;
+  return p;
 }
 inline void xfer_user(int delta) {
-  XferRing &r = xfer_ring();
-  std::lock_guard<std::mutex> lk(r.mu);
-  r.users += delta;
-  if (r.users == 0 && r.buf) {
-    hipHostFree(r.buf);
+  XferPool &P = xfer_pool();
+  std::lock_guard<std::mutex> lk(P.mu);
+  P.users += delta;
+  if (P.users > 0) return;
+  for (XferRing &r : P.ring) {
+    std::lock_guard<std::mutex> lr(r.mu);
+    if (r.buf) hipHostFree(r.buf);
     r.buf = nullptr;
   }
 }
@@ -61,30 +70,57 @@ struct DeviceScope {
   DeviceScope &operator=(const DeviceScope &) = delete;
 };
 
+// A transfer without the ring: the whole field straight from or to the caller's
+// memory if it crosses as it is (host), else in pieces of ordinary memory.
+template <class Move>
+hipError_t xfer_plain(hipStream_t stream, char *dptr, size_t bytes, bool up, Move move, char *host) {
+  std::unique_ptr<char[]> buf;
+  const size_t step = host ? bytes : (bytes < kPiece ? bytes : kPiece);
+  if (!host) {
+    buf.reset(new (std::nothrow) char[step]);
+    if (!buf) return hipErrorOutOfMemory;
+  }
+  for (size_t o = 0; o < bytes; o += step) {
+    const size_t len = bytes - o < step ? bytes - o : step;
+    char *t = host ? host : buf.get();
+    if (up && !host) move(o, t, len);
+    hipError_t e = up ? hipMemcpyAsync(dptr + o, t, len, hipMemcpyHostToDevice, stream)
+                      : hipMemcpyAsync(t, dptr + o, len, hipMemcpyDeviceToHost, stream);
+    const hipError_t f = hipStreamSynchronize(stream);
+    if (e == hipSuccess) e = f;
+    if (e != hipSuccess) return e;
+    if (!up && !host) move(o, t, len);
+  }
+  return hipSuccess;
+}
+
 // One transfer of `bytes` bytes: up = false, device -> host: move(piece
 // offset, pinned piece, length) empties a piece the copy engine has filled;
-// up = true: it fills a piece, which is then copied to the device.  Returns
-// the first error.  On return the transfer is complete.
+// up = true: it fills a piece, which is then copied to the device; host: the
+// caller's memory where move only copies (else null).  Returns the first error.
+// On return the transfer is complete.
 template <class Move>
-hipError_t xfer(int dev, hipStream_t stream, void *dptr, size_t bytes, bool up, Move move) {
+hipError_t xfer(int dev, hipStream_t stream, void *dptr, size_t bytes, bool up, Move move, void *host = nullptr) {
   if (bytes == 0) return hipSuccess;
   const DeviceScope on(dev);
   if (on.rc != hipSuccess) return on.rc;
   hipError_t e = hipStreamSynchronize(stream);
   if (e != hipSuccess) return e;
-  XferRing &R = xfer_ring();
-  std::lock_guard<std::mutex> lk(R.mu);
-  if (!R.buf) {
-    e = hipHostMalloc((void **)&R.buf, kPieces * kPiece, hipHostMallocPortable);
-    if (e != hipSuccess) {
-      R.buf = nullptr;
-      return e;
-    }
+  std::unique_lock<std::mutex> lk;
+  XferRing *R = nullptr;
+  for (XferRing &r : xfer_pool().ring) {
+    lk = std::unique_lock<std::mutex>(r.mu, std::try_to_lock);
+    if (!lk) continue;
+    R = &r;
+    break;
   }
+  if (R && !R->buf && hipHostMalloc((void **)&R->buf, kPieces * kPiece, hipHostMallocPortable) != hipSuccess)
+    R->buf = nullptr;
+  if (!R || !R->buf) return xfer_plain(stream, (char *)dptr, bytes, up, move, (char *)host);
   const long np = (long)((bytes + kPiece - 1) / kPiece);
   auto off = [&](long c) { return (size_t)c * kPiece; };
   auto len = [&](long c) { return bytes - off(c) < kPiece ? bytes - off(c) : kPiece; };
-  auto slot = [&](long c) { return R.buf + (size_t)(c % kPieces) * kPiece; };
+  auto slot = [&](long c) { return R->buf + (size_t)(c % kPieces) * kPiece; };
   auto dev_at = [&](long c) { return (char *)dptr + off(c); };
   if (np <= 2) {  // small: the caller's thread alone, one wait
     if (up)

@@ -60,10 +60,46 @@ static bool device() {
   return ok && d == 1;
 }
 
+// transfers of another case while `n` are stuck in their callers' memory
+static bool beside(int n) {
+  std::atomic<int> entered{0}, release{0}, done{0}, ok{0};
+  std::vector<std::thread> big;
+  for (int t = 0; t < n; t++)
+    big.emplace_back([&] {
+      StubStream st(0);
+      std::vector<char> dev(20 * kPiece);
+      xfer(0, &st, dev.data(), dev.size(), false, [&](size_t o, const char *, size_t) {
+        if (o == 0) entered++;
+        while (!release) std::this_thread::yield();
+      });
+    });
+  for (int t = 0; t < 1000 && entered < n; t++) std::this_thread::sleep_for(std::chrono::milliseconds(5));
+  std::thread other([&] {
+    StubStream st(0);
+    ok = round_trip(st, 1000, 5) && round_trip(st, 11 * kPiece + 16, 5);
+    done = 1;
+  });
+  for (int t = 0; t < 2000 && !done; t++) std::this_thread::sleep_for(std::chrono::milliseconds(5));
+  const bool in_time = done != 0;
+  release = 1;
+  for (auto &t : big) t.join();
+  other.join();
+  std::printf("finished beside %d: %d\n", n, (int)in_time);
+  return in_time && ok;
+}
+
+// no pinned memory to be had
+static bool unpinned() {
+  stub_no_pinned = 1;
+  StubStream st(0);
+  return round_trip(st, 5 * kPiece + 8, 6) && round_trip(st, 10, 6);
+}
+
 int main(int argc, char **argv) {
   const std::string t = argc > 1 ? argv[1] : "";
   xfer_user(1);
-  const bool ok = t == "sizes" ? sizes() : t == "threads" ? threads() : t == "device" ? device() : false;
+  const bool ok = t == "sizes" ? sizes() : t == "threads" ? threads() : t == "device" ? device()
+                  : t == "beside_one" ? beside(1) : t == "beside_five" ? beside(5) : t == "unpinned" ? unpinned() : false;
   xfer_user(-1);
   return ok ? 0 : 1;
 }

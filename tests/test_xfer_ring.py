@@ -1,6 +1,7 @@
 """The host side of field transfers (the pinned ring and its threads) on a
 stand-in for the HIP runtime: every size and direction, from several threads,
-and from a thread whose current device is not the case's."""
+from a thread whose current device is not the case's, beside other transfers
+that stand still, and without pinned memory."""
 import os
 import shutil
 import subprocess
@@ -21,7 +22,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["sizes", "threads", "device"])
+@pytest.mark.parametrize("name", ["sizes", "threads", "device", "beside_one", "beside_five", "unpinned"])
 def test_transfer(program, name):
     r = subprocess.run([program, name], capture_output=True, text=True, timeout=60)
     print(r.stdout)
