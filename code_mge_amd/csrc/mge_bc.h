@@ -533,7 +533,7 @@ __device__ inline double pow25(double x) {
   const double y = x * x, ey = __builtin_fma(x, x, -y);
   const double s = sqrt(x), es = __builtin_fma(-s, s, x);
   const double r = y * s, er = __builtin_fma(y, s, -r);
-  return x > 0.0 ? r + (er + __builtin_fma(ey, s, y * (0.5 * es * rcp_pos(s)))) : r;
+  return r > 0.0 && !__builtin_isinf(r) ? r + (er + __builtin_fma(ey, s, y * (0.5 * es * rcp_pos(s)))) : r;
 }
 // x^(7/5) to rounding: z = x^(2/5) from an FP32 estimate z0 and the relative
 // defect e = x^2 / z0^5 - 1 (about 1e-6), z = z0 (1 + e)^(1/5); products that
@@ -550,12 +550,6 @@ __device__ inline double pow75(double x) {
   const double w = x * z0, ew = __builtin_fma(x, z0, -w);
   return w + (ew + x * dz);
 }
-// a / b from the refined reciprocal rb of b: the quotient corrected by its
-// remainder, the rounded quotient but for rare last-bit cases
-__device__ inline double div_by(double a, double b, double rb) {
-  const double q = a * rb;
-  return __builtin_fma(__builtin_fma(-b, q, a), rb, q);
-}
 template <typename T>
 __device__ inline CellV<T> far_state(const FacesArgs<T> &A, int f, CellV<T> v, uint8_t *dec,
                                                         bool rec) {
@@ -566,18 +560,34 @@ __device__ inline CellV<T> far_state(const FacesArgs<T> &A, int f, CellV<T> v, u
   const double gamma = A.gamma, g1 = gamma - 1.0, gm = A.gm;
   const double rho = full(fi, 0, v.w[0]), m0 = full(fi, 1, v.w[1]), m1 = full(fi, 2, v.w[2]),
                m2 = full(fi, 3, v.w[3]), pe = full(fi, 5, v.p);
-  const double rr = rcp_pos(rho);
-  const double u0 = div_by(m0, rho, rr), u1 = div_by(m1, rho, rr), u2 = div_by(m2, rho, rr);
-  bool inflow = pick3(dir, u0, u1, u2) * sg <= 0.0;
+  double vn = 0.0, u0, u1, u2, c2;   // normal velocity, velocity, squared speed of sound
+  vn = vn + m0 * (dir == 0 ? sg : 0.0);
+  vn = vn + m1 * (dir == 1 ? sg : 0.0);
+  vn = vn + m2 * (dir == 2 ? sg : 0.0);
+  if (fabs(rho) > 1e-290 && fabs(rho) < 1e290) {
+    const double rr = rcp_pos(rho);
+    vn = quot(vn, rho, rr);
+    u0 = quot(m0, rho, rr);
+    u1 = quot(m1, rho, rr);
+    u2 = quot(m2, rho, rr);
+    c2 = quot(gamma * pe, rho, rr);
+  } else {   // no reciprocal
+    vn = vn / rho;
+    u0 = m0 / rho;
+    u1 = m1 / rho;
+    u2 = m2 / rho;
+    c2 = gamma * pe / rho;
+  }
+  bool inflow = vn <= 0.0;
   if (dec) {
     if (*A.frozen) inflow = *dec == 0;
     else if (rec) *dec = inflow ? 0 : 1;
   }
-  const double rpo = pick3(dir, u0, u1, u2) * sg + div_by(2.0 * sqrt(div_by(gamma * pe, rho, rr)), g1, gm);
+  const double rpo = pick3(dir, u0, u1, u2) * sg + quot(2.0 * sqrt(c2), g1, gm);
   const double rmi = pick3(dir, A.u0, A.v0, A.w0) * sg - A.rinf;
   const double un = 0.5 * (rpo + rmi) * sg;
   const double ci = 0.25 * g1 * (rpo - rmi);
-  const double cc = div_by(ci * ci, gamma, A.rgamma);
+  const double cc = quot(ci * ci, gamma, A.rgamma);
   double si = A.s0;
   if (!inflow) si = (A.air ? pow75(rho) : pow(rho, gamma)) / pe;
   const double x = si * cc;
@@ -1131,7 +1141,8 @@ struct XferArgs {
   const T *wsc;
   T *wr;
   uint8_t *marker;
-  T volc, volf;
+  T volc, volf, rvolf;   // cell volumes, 1/volf
+  int div;               // the restriction divides: per-cell volumes, or 1/volf overflows
   int fmg;               // mgl-1 == mlvl: interpolate the solution itself
   const uint8_t *flagsf;
   T *wfo;                // fine state (prolongation, in place)
@@ -1155,6 +1166,13 @@ struct XferArgs {
   T gamma;
   Inf<T> inf;
   int gx, gy, gz0;
+  // the fine cells' volume, or their array
+  void fine_volume(T v, const T *per_cell) {
+    volf = v;
+    vf = per_cell;
+    rvolf = T(1) / v;
+    div = per_cell || std::isinf(rvolf);
+  }
 };
 
 // the EOS of ghost-shell cell t of a level
@@ -1233,7 +1251,6 @@ __device__ __attribute__((always_inline)) inline void k_restrict_body(const Xfer
   // every load before the first use; one volume for the level: its
   // reciprocal, and the product corrected by its remainder, in place of 40
   // divisions (9.5 -> 8.2 us on the levels of a 128^3 FP32 hierarchy)
-  const T rvol = T(1) / X.volf;
   T dv[5][8], wv[5][8];
 #pragma unroll
   for (int n = 0; n < 5; n++)
@@ -1247,7 +1264,7 @@ __device__ __attribute__((always_inline)) inline void k_restrict_body(const Xfer
     T acc = T(0);
 #pragma unroll
     for (int c8 = 0; c8 < 8; c8++) {
-      const T val = X.vf ? dv[n][c8] / X.vf[qf[c8]] : quot(dv[n][c8], X.volf, rvol);
+      const T val = X.div ? dv[n][c8] / (X.vf ? X.vf[qf[c8]] : X.volf) : quot(dv[n][c8], X.volf, X.rvolf);
       acc = acc + val * fac[c8];
     }
     X.wr[n * c.E + qc] = acc * (X.vc ? X.vc[qc] : X.volc);

@@ -132,7 +132,7 @@ int comp_movco(mge_comp *C, int mgl) {
       X.wr = tp<T>(Cb.wr);
       X.marker = Cb.marker;
       X.volc = (T)Cb.cellvolume;
-      X.volf = (T)F.cellvolume;
+      X.fine_volume((T)F.cellvolume, nullptr);
       X.flagsf = F.flags;
       for (int d = 0; d < 3; d++) X.off[d] = C->b[f].g0[d] / 2 - C->b[c].g0[d];
       X.nrc[0] = F.d.ni / 2; X.nrc[1] = F.d.nj / 2; X.nrc[2] = F.d.nk / 2;
@@ -173,7 +173,7 @@ int comp_movfin(mge_comp *C, int mgl, int mlvl) {
     X.wc = tp<T>(P.S[P.cur]);
     X.wsc = tp<T>(P.ws);
     X.volc = (T)P.cellvolume;
-    X.volf = (T)F.cellvolume;
+    X.fine_volume((T)F.cellvolume, nullptr);
     X.fmg = fmg;
     X.flagsf = F.flags;
     X.wfo = tp<T>(F.S[F.cur]);

@@ -1074,9 +1074,8 @@ int do_movco(mge_case *h, int mgl) {
   X.wr = tp<T>(c.wr);
   X.marker = c.marker;
   X.volc = (T)c.cellvolume;
-  X.volf = (T)f.cellvolume;
   X.vc = c.vol ? tp<T>(c.vol) : nullptr;
-  X.vf = f.vol ? tp<T>(f.vol) : nullptr;
+  X.fine_volume((T)f.cellvolume, f.vol ? tp<T>(f.vol) : nullptr);
   for (int a = 0; a < 3; a++) X.rw[a] = f.rw[a] ? tp<T>(f.rw[a]) : nullptr;
   if ((X.vc != nullptr) != (X.vf != nullptr) || (X.vf && !X.rw[0]))
     return set_err(MGE_ERR_ARG, "a stretched level and a uniform level do not nest");
@@ -1106,7 +1105,6 @@ int do_movfin(mge_case *h, int mgl, int mlvl) {
   X.wr = nullptr;
   X.marker = nullptr;
   X.volc = (T)c.cellvolume;
-  X.volf = (T)f.cellvolume;
   for (int a = 0; a < 3; a++) X.pw[a] = f.pw[a] ? tp<T>(f.pw[a]) : nullptr;
   if ((c.vol != nullptr) != (f.vol != nullptr) || (f.vol && !X.pw[0]))
     return set_err(MGE_ERR_ARG, "a stretched level and a uniform level do not nest");
