@@ -169,6 +169,7 @@ def lib():
     L.mge_batch_run.argtypes = [P, I, C.POINTER(I)]
     L.mge_batch_status.argtypes = [P, I, C.POINTER(I), C.POINTER(I), dp, dp]
     L.mge_batch_log.argtypes = [P, I, dp, I]
+    L.mge_batch_stage_tile.argtypes = [P, I, I, C.POINTER(I), C.POINTER(I)]
     _lib = L
     return L
 
@@ -188,7 +189,7 @@ EXPORTED = [
     "mge_upload", "mge_get_cuts", "mge_get_dtim", "mge_wall_force", "mge_synchronize",
     "mge_kernel_timing", "mge_last_error", "mge_cycles",
     "mge_batch_create", "mge_batch_destroy", "mge_batch_add", "mge_batch_remove", "mge_batch_run",
-    "mge_batch_status", "mge_batch_log", "mge_case_bytes", "mge_autotune", "mge_set_kc", "mge_geom_level_tri",
+    "mge_batch_status", "mge_batch_log", "mge_batch_stage_tile", "mge_case_bytes", "mge_autotune", "mge_set_kc", "mge_geom_level_tri",
     "mge_stage_tile", "mge_set_tile", "mge_set_freeze", "mge_comp_create", "mge_comp_solve", "mge_comp_destroy",
     "mge_read_job", "mge_job_params", "mge_job_level", "mge_read_pin", "mge_read_p3d", "mge_input_error",
     "mge_write_solut", "mge_read_solut", "mge_solve_step", "mge_shift_time_levels",

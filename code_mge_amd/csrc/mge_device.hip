@@ -1762,6 +1762,7 @@ struct mge_batch {
   std::vector<Step> prog;
   std::vector<int> prog_slots;         // slots the program was built for
   std::vector<std::vector<int>> cur1;  // per program case: level buffers after cycle 1
+  std::vector<std::vector<TileShape>> shape;  // per program case and level: the stage launches' shape
   char *d_arena = nullptr;
   size_t arena_cap = 0;
   hipGraph_t graph = nullptr;
@@ -1831,6 +1832,7 @@ int batch_build(mge_batch *b) {
   b->prog.clear();
   b->prog_slots.clear();
   b->cur1.clear();
+  b->shape.clear();
   for (int c = 0; c < (int)b->cs.size(); c++)
     if (b->cs[c] && b->hact[c]) b->prog_slots.push_back(c);
   b->dirty = false;
@@ -1838,6 +1840,7 @@ int batch_build(mge_batch *b) {
   if (nc == 0) return MGE_OK;
   std::vector<std::vector<Rec>> R(nc);
   b->cur1.resize(nc);
+  b->shape.resize(nc);
   // one stage launch shape per level for all cases: they run in one launch,
   // whose workgroups fill the chip together, so the shape that is fastest for
   // each case alone (many small chunks, and other tile rows for some, hence a
@@ -1868,7 +1871,10 @@ int batch_build(mge_batch *b) {
     int rc = MGE_OK;
     // the program replays these two cycles from the buffers they start in
     std::vector<int> cur0;
-    for (int l = 1; l <= h->nlevel; l++) cur0.push_back(h->lv[l].cur);
+    for (int l = 1; l <= h->nlevel; l++) {
+      cur0.push_back(h->lv[l].cur);
+      b->shape[i].push_back(stage_shape(h, h->lv[l]));
+    }
     for (int cyc = 1; cyc <= 2 && rc >= 0; cyc++) {
       rc = by_type(h, [&](auto z) { return do_cycle<decltype(z)>(h, b->nlevel, cyc, &cs); });
       Rec m;
@@ -2903,6 +2909,17 @@ int mge_batch_log(mge_batch *b, int slot, double *out, int cap) {
     HIPCHK(hipStreamSynchronize(b->stream));
   }
   return n;
+}
+
+int mge_batch_stage_tile(mge_batch *b, int slot, int lvl, int *tj, int *kc) {
+  if (!b || !tj || !kc || lvl < 1 || lvl > b->nlevel) return set_err(MGE_ERR_ARG, "bad batch, level or output pointer");
+  const auto it = std::find(b->prog_slots.begin(), b->prog_slots.end(), slot);
+  const size_t i = it - b->prog_slots.begin();
+  if (i >= b->shape.size()) return set_err(MGE_ERR_ARG, "the slot is not in the batch's program");
+  const TileShape &sh = b->shape[i][lvl - 1];
+  *tj = sh.tj;
+  *kc = sh.kc;
+  return MGE_OK;
 }
 
 long long mge_case_bytes(mge_case *h) {

@@ -301,6 +301,12 @@ class Batch:
                    "mge_batch_status")
         return dict(status=st.value, ncyc=nc.value, ini=ini.value, last=last.value)
 
+    def stage_tile(self, slot: int, lvl: int):
+        """(tile rows, k-chunk length) of the slot's stage launches on level lvl"""
+        tj, kc = C.c_int(0), C.c_int(0)
+        _ffi.check(self.lib.mge_batch_stage_tile(self.h, slot, lvl, C.byref(tj), C.byref(kc)), "mge_batch_stage_tile")
+        return tj.value, kc.value
+
     def log(self, slot: int, cap: int = 100000):
         out = np.zeros(cap)
         n = _ffi.check(self.lib.mge_batch_log(self.h, slot, out.ctypes.data_as(_dp), cap), "mge_batch_log")

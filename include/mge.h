@@ -384,6 +384,9 @@ int mge_batch_run(mge_batch *b, int periods, int *nactive);
 int mge_batch_status(mge_batch *b, int slot, int *status, int *ncyc, double *ini, double *last);
 /* residual history of a slot (one value per cycle); returns the count */
 int mge_batch_log(mge_batch *b, int slot, double *out, int cap);
+/* the tile rows and k-chunk length the stage launches of level lvl take for
+ * a slot in the batch's present program (the cases active when it was built) */
+int mge_batch_stage_tile(mge_batch *b, int slot, int lvl, int *tj, int *kc);
 
 #ifdef __cplusplus
 }

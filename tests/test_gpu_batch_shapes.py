@@ -1,0 +1,50 @@
+"""The stage launch shapes a batch's program takes: one per level for the cases
+whose shape the library picks, tuned or not, and its own for a case whose
+caller forced one."""
+import pytest
+
+from code_mge_amd import _ffi, configs
+from code_mge_amd.solver import Batch, Case
+
+pytestmark = pytest.mark.gpu
+
+
+def make(n, mode, distype, precision):
+    prm, levels, bdy, _ = configs.ellipsoid3d(n=n, nlevel=3, semi=(0.9, 0.6, 0.5), box=4.0, mach=0.4, alpha=3.0,
+                                              distype=distype, precision=precision)
+    c = Case(prm, levels, body=bdy, mxcyc=8)
+    c.init_flow()
+    for lvl in (1, 2, 3):
+        if mode == "forced":
+            c.set_tile(lvl, 8, 3)
+        elif mode == "forced chunk":
+            c.set_kc(lvl, 5)
+    if mode == "tuned":
+        c.autotune()
+    return c
+
+
+def run_batch(modes, distype, precision):
+    """the modes' cases in one batch: their shapes by level, alone and in it"""
+    cases = [make(24 + 8 * k, m, distype, precision) for k, m in enumerate(modes)]
+    alone = [[c.stage_tile(lvl) for lvl in (1, 2, 3)] for c in cases]
+    with Batch(log_cap=8) as b:
+        slots = [b.add(c, 1e30, 4) for c in cases]
+        with pytest.raises(_ffi.MgeError):   # no program yet
+            b.stage_tile(slots[0], 1)
+        b.run(1)
+        got = [[b.stage_tile(s, lvl) for lvl in (1, 2, 3)] for s in slots]
+        with pytest.raises(_ffi.MgeError):
+            b.stage_tile(slots[-1] + 1, 1)
+    for c in cases:
+        c.close()
+    return got, alone
+
+
+@pytest.mark.parametrize("distype,precision", [("c", 64), ("r2", 32)])
+def test_common_and_forced_shapes(require_gpu, distype, precision):
+    got, alone = run_batch(["tuned", "forced", "plain", "forced chunk"], distype, precision)
+    print(got, alone)
+    assert got[0] == got[2]
+    assert got[1] == alone[1] and all(s == (8, 3) for s in got[1])
+    assert got[3] == alone[3] and all(kc == min(5, n) for (_, kc), n in zip(got[3], (12, 24, 48)))
