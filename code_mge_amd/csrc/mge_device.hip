@@ -113,9 +113,8 @@ struct Level {
   double *dtim = nullptr;
   double *rtrms = nullptr;
   double *force = nullptr;
-  int kc = 0;                   // tuned or forced k planes per stage workgroup (0: tile_pick's)
-  int tj = 0;                   // tuned or forced tile rows of the stage kernels (0: tile_pick's)
-  bool tuned = false;           // kc and tj come from the autotuner (a batch picks its own)
+  int kc = 0, tj = 0;           // stage kernels' k planes per workgroup and tile rows: the caller's (0: none)
+  int tkc = 0, ttj = 0;         // the autotuner's (0: none), taken where the caller forces none
   int btj = 0, bkc = 0;         // the batch's common choice while the case is recorded into it (0: none)
   int *vtile = nullptr;         // Navier-Stokes: wall records by tile of the viscous kernel
   ViscRec *vrec = nullptr;
@@ -765,12 +764,13 @@ TileShape tile_pick(const std::vector<const Dims *> &ds, bool fp32, bool roe, in
 }
 
 // the stage launch shape of a level: the batch's choice while it is recorded
-// into one (unless the caller forced a shape), else the tuned or forced
-// values, the rest by tile_pick
+// into one (unless the caller forced a shape), else the forced values, then the
+// tuned ones, the rest by tile_pick
 TileShape stage_shape(const mge_case *h, const Level &L) {
   if (h->rec && L.btj > 0) return TileShape{L.btj, std::min(L.bkc, L.d.nk)};
-  if (L.tj > 0 && L.kc > 0) return TileShape{L.tj, std::min(L.kc, L.d.nk)};
-  return tile_pick({&L.d}, h->fp32, h->prm.distype != 0, L.tj, L.kc);
+  const int tj = L.tj > 0 ? L.tj : L.ttj, kc = L.kc > 0 ? L.kc : L.tkc;
+  if (tj > 0 && kc > 0) return TileShape{tj, std::min(kc, L.d.nk)};
+  return tile_pick({&L.d}, h->fp32, h->prm.distype != 0, tj, kc);
 }
 
 // single-case and batch entry points of the LDS-tiled stage kernel of a
@@ -1343,8 +1343,7 @@ int do_autotune(mge_case *h, Level &L, int *kc_out, double *us_out) {
   const Dims &d = L.d;
   if (h->rec) return set_err(MGE_ERR_STATE, "autotune while a batch is being recorded");
   if (P.distype == 0 && P.dissip != 0) {  // matrix dissipation: one thread per cell, nothing to tune
-    L.kc = 0;
-    L.tj = 0;
+    L.kc = L.tj = L.tkc = L.ttj = 0;
     if (kc_out) *kc_out = 0;
     if (us_out) *us_out = 0.0;
     return MGE_OK;
@@ -1354,10 +1353,10 @@ int do_autotune(mge_case *h, Level &L, int *kc_out, double *us_out) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune.find(key);
     if (it != g_tune.end()) {
-      L.kc = it->second.kc;
-      L.tj = it->second.tj;
-      L.tuned = true;
-      if (kc_out) *kc_out = L.kc;
+      L.kc = L.tj = 0;
+      L.tkc = it->second.kc;
+      L.ttj = it->second.tj;
+      if (kc_out) *kc_out = L.tkc;
       if (us_out) *us_out = it->second.us;
       return MGE_OK;
     }
@@ -1418,9 +1417,9 @@ int do_autotune(mge_case *h, Level &L, int *kc_out, double *us_out) {
     best_tj = tj_def == 4 ? 8 : 4;
   }
   CHKRC(check_err(h));
-  L.kc = best;
-  L.tj = best_tj;
-  L.tuned = true;
+  L.kc = L.tj = 0;
+  L.tkc = best;
+  L.ttj = best_tj;
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune[key] = {best_tj, best, best_us};
@@ -1858,7 +1857,7 @@ int batch_build(mge_batch *b) {
     const TileShape sh = tile_pick(ds, b->fp32 == 1, b->distype != 0, 0, 0);
     for (int s : b->prog_slots) {
       Level &L = b->cs[s]->lv[l];
-      if (L.tuned || (L.tj == 0 && L.kc == 0)) {
+      if (L.tj == 0 && L.kc == 0) {
         L.btj = sh.tj;
         L.bkc = sh.kc;
       }
@@ -2944,7 +2943,7 @@ int mge_set_kc(mge_case *h, int lvl, int kc) {
   Level *L = get_level(h, lvl);
   if (!L || kc < 0) return set_err(MGE_ERR_ARG, "bad level or kc");
   L->kc = kc;
-  L->tuned = false;
+  L->tkc = 0;   // tuned rows stay
   return MGE_OK;
 }
 
@@ -2972,7 +2971,7 @@ int mge_set_tile(mge_case *h, int lvl, int tj, int kc) {
   if (!L || !(tj == 0 || tj == 4 || tj == 8) || kc < 0) return set_err(MGE_ERR_ARG, "bad level, tile rows or kc");
   L->tj = tj;
   L->kc = kc;
-  L->tuned = false;
+  L->ttj = L->tkc = 0;
   return MGE_OK;
 }
 

@@ -19,8 +19,12 @@ def make(n, mode, distype, precision):
             c.set_tile(lvl, 8, 3)
         elif mode == "forced chunk":
             c.set_kc(lvl, 5)
-    if mode == "tuned":
+    if mode in ("tuned", "tuned, chunk given back"):
         c.autotune()
+    if mode == "tuned, chunk given back":
+        for lvl in (1, 2, 3):
+            c.set_kc(lvl, 5)
+            c.set_kc(lvl, 0)
     return c
 
 
@@ -48,3 +52,11 @@ def test_common_and_forced_shapes(require_gpu, distype, precision):
     assert got[0] == got[2]
     assert got[1] == alone[1] and all(s == (8, 3) for s in got[1])
     assert got[3] == alone[3] and all(kc == min(5, n) for (_, kc), n in zip(got[3], (12, 24, 48)))
+
+
+def test_given_back_chunk_is_not_forced(require_gpu):
+    """a chunk length forced and given back (0) leaves the level to the library,
+    tuned rows or not: the batch's common shape"""
+    got, _ = run_batch(["plain", "tuned, chunk given back", "plain"], "r2", 32)
+    print(got)
+    assert got[0] == got[1] == got[2]
