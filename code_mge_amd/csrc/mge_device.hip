@@ -1843,7 +1843,7 @@ int batch_build(mge_batch *b) {
   // one stage launch shape per level for all cases: they run in one launch,
   // whose workgroups fill the chip together, so the shape that is fastest for
   // each case alone (many small chunks, and other tile rows for some, hence a
-  // second launch) is not the batch's
+  // second launch) is not the batch's.  A single case keeps its own.
   struct ShapeTag {
     mge_batch *b;
     ~ShapeTag() {
@@ -1851,7 +1851,7 @@ int batch_build(mge_batch *b) {
         for (Level &L : b->cs[s]->lv) L.btj = L.bkc = 0;
     }
   } stag{b};
-  for (int l = 1; l <= b->nlevel; l++) {
+  for (int l = 1; l <= b->nlevel && nc > 1; l++) {
     std::vector<const Dims *> ds;
     for (int s : b->prog_slots) ds.push_back(&b->cs[s]->lv[l].d);
     const TileShape sh = tile_pick(ds, b->fp32 == 1, b->distype != 0, 0, 0);

@@ -307,8 +307,8 @@ int mge_kernel_timing(mge_case *h, int enable, const char *name, double *ms, lon
  * 4, ... nk, and keeps the fastest pair for the level; results are cached
  * per (shape, precision, scheme) for the process.  The launch shape changes
  * no arithmetic.  An untuned level takes the shape a cost model picks, and a
- * batch picks one shape per level for all its cases whether tuned or not
- * (a shape forced with mge_set_tile or mge_set_kc stays).  Overwrites only scratch state (a non-current state
+ * batch of several cases picks one shape per level for all of them whether
+ * tuned or not (a shape forced with mge_set_tile or mge_set_kc stays).  Overwrites only scratch state (a non-current state
  * buffer, dw, fw, the time-step arrays); call it between solves, not while
  * a batch is recording.  *kc (0 for the matrix-dissipation kernel, which has
  * no chunks) and *us (best launch time, microseconds) may be NULL; the

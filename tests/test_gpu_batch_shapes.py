@@ -28,9 +28,9 @@ def make(n, mode, distype, precision):
     return c
 
 
-def run_batch(modes, distype, precision):
+def run_batch(modes, distype, precision, n=24):
     """the modes' cases in one batch: their shapes by level, alone and in it"""
-    cases = [make(24 + 8 * k, m, distype, precision) for k, m in enumerate(modes)]
+    cases = [make(n + 8 * k, m, distype, precision) for k, m in enumerate(modes)]
     alone = [[c.stage_tile(lvl) for lvl in (1, 2, 3)] for c in cases]
     with Batch(log_cap=8) as b:
         slots = [b.add(c, 1e30, 4) for c in cases]
@@ -60,3 +60,13 @@ def test_given_back_chunk_is_not_forced(require_gpu):
     got, _ = run_batch(["plain", "tuned, chunk given back", "plain"], "r2", 32)
     print(got)
     assert got[0] == got[1] == got[2]
+
+
+@pytest.mark.parametrize("distype,precision", [("c", 64), ("r2", 64), ("c", 32), ("r2", 32)])
+def test_single_case_keeps_its_shape(require_gpu, distype, precision):
+    """what was timed for the case, where that is not the library's pick either"""
+    for n in (24, 32, 40, 64):
+        plain, _ = run_batch(["plain"], distype, precision, n)
+        got, alone = run_batch(["tuned"], distype, precision, n)
+        print(n, "plain", plain, "tuned", alone)
+        assert got == alone
