@@ -9,7 +9,7 @@ each batch by a few periods (two multigrid cycles each, all cases in one
 launch per operation); a case leaves the batch at the cycle its residual
 has dropped by `drop` (or at maxcyc), its Cd/Cl are read, its memory is
 freed and waiting requests are admitted in its place.  Admission (geometry,
-device state, init_flow, autotune) runs on its own thread while the GPU
+device state, init_flow) runs on its own thread while the GPU
 works, and the batches of different classes (Euler and Navier-Stokes, say)
 advance concurrently on their own streams.  A case computes exactly what
 it computes alone.
@@ -123,8 +123,11 @@ class Server:
         return total
 
     def _prepare(self, req: Request):
-        """host geometry, device state, init_flow and autotune of one
-        request: the admission work, done off the tick thread"""
+        """host geometry, device state and init_flow of one request: the
+        admission work, done off the tick thread.  The launch shapes are timed
+        for a request admitted alone: a batch of several cases takes one shape
+        for all of them, tuned or not, and the timing's launches would run
+        beside theirs."""
         geoms = [level_geometry(s, req.body) for s in req.levels]
         need = self.estimate(req, geoms)
         with self._cv:
@@ -135,13 +138,14 @@ class Server:
                 return None
             self.used += need
             self._resident += 1
+            alone = self._resident == 1
             self.peak_used = max(self.peak_used, self.used)
         prm = dataclasses.replace(req.params, precision=self.precision)
         if self.ffreeze is not None:
             prm = dataclasses.replace(prm, ffreeze=self.ffreeze)
         case = Case(prm, req.levels, geoms=geoms, mxcyc=4)
         case.init_flow()
-        if self.autotune:
+        if self.autotune and alone:
             case.autotune()   # cached per level shape after the first request
         got = case.device_bytes()
         with self._cv:
