@@ -560,25 +560,21 @@ __device__ inline CellV<T> far_state(const FacesArgs<T> &A, int f, CellV<T> v, u
   const double gamma = A.gamma, g1 = gamma - 1.0, gm = A.gm;
   const double rho = full(fi, 0, v.w[0]), m0 = full(fi, 1, v.w[1]), m1 = full(fi, 2, v.w[2]),
                m2 = full(fi, 3, v.w[3]), pe = full(fi, 5, v.p);
-  double vn = 0.0, u0, u1, u2, c2;   // normal velocity, velocity, squared speed of sound
-  vn = vn + m0 * (dir == 0 ? sg : 0.0);
-  vn = vn + m1 * (dir == 1 ? sg : 0.0);
-  vn = vn + m2 * (dir == 2 ? sg : 0.0);
-  if (fabs(rho) > 1e-290 && fabs(rho) < 1e290) {
-    const double rr = rcp_pos(rho);
-    vn = quot(vn, rho, rr);
-    u0 = quot(m0, rho, rr);
-    u1 = quot(m1, rho, rr);
-    u2 = quot(m2, rho, rr);
-    c2 = quot(gamma * pe, rho, rr);
-  } else {   // no reciprocal
-    vn = vn / rho;
-    u0 = m0 / rho;
-    u1 = m1 / rho;
-    u2 = m2 / rho;
-    c2 = gamma * pe / rho;
+  const double rr = rcp_pos(rho);
+  double u0 = quot(m0, rho, rr), u1 = quot(m1, rho, rr), u2 = quot(m2, rho, rr), c2 = quot(gamma * pe, rho, rr);
+  bool inflow = pick3(dir, u0, u1, u2) * sg <= 0.0;
+  if (!((fabs(m0) + fabs(m1)) + (fabs(m2) + fabs(rr)) < __builtin_inf())) {
+    // a density without a reciprocal (its own infinity or zero then), or an
+    // infinite momentum: the reference's normal velocity, a sum over all
+    // components, is NaN beside an infinite tangential one
+    const double r = fabs(rr) < __builtin_inf() ? rr : __builtin_amdgcn_rcp(rho);
+    u0 = m0 * r;
+    u1 = m1 * r;
+    u2 = m2 * r;
+    c2 = gamma * pe * r;
+    const double mn = m0 * (dir == 0 ? sg : 0.0) + m1 * (dir == 1 ? sg : 0.0) + m2 * (dir == 2 ? sg : 0.0);
+    inflow = mn * r <= 0.0;
   }
-  bool inflow = vn <= 0.0;
   if (dec) {
     if (*A.frozen) inflow = *dec == 0;
     else if (rec) *dec = inflow ? 0 : 1;

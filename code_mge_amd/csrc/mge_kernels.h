@@ -305,16 +305,17 @@ __device__ inline void xcd_block(int &bx, int &by, int &bz) {
     NAME##_body(As[c], l % g.y, (l / g.y) % g.z, l / (g.y * g.z));                                     \
   }
 
-// x / h from r = 1/h, both normal: the product corrected by its remainder, which
-// is the rounded quotient but for rare last-bit cases; an infinite product is
-// the quotient itself (its remainder would be NaN)
+// x / h from r = 1/h: the product corrected by its remainder, which is the
+// rounded quotient but for rare last-bit cases.  An infinite product is the
+// quotient itself: its remainder is NaN, which the minimum replaces by a finite
+// number (one instruction; a select takes three).
 __device__ inline float quot(float x, float h, float r) {
   const float q = x * r;
-  return __builtin_isinf(q) ? q : __builtin_fmaf(__builtin_fmaf(-h, q, x), r, q);
+  return __builtin_fmaf(__builtin_fminf(__builtin_fmaf(-h, q, x), 0x1p127f), r, q);
 }
 __device__ inline double quot(double x, double h, double r) {
   const double q = x * r;
-  return __builtin_isinf(q) ? q : __builtin_fma(__builtin_fma(-h, q, x), r, q);
+  return __builtin_fma(__builtin_fmin(__builtin_fma(-h, q, x), 0x1p1023), r, q);
 }
 
 template <typename T>
