@@ -350,6 +350,18 @@ Level *get_level(mge_case *h, int lvl) {
   return L->defined ? L : nullptr;
 }
 
+// one kernel outside the cycle's launches; returns the launch's own status (the
+// thread's last error may be another caller's)
+template <class U>
+struct Same {
+  using type = U;
+};
+template <class... A>
+hipError_t launch_on(hipStream_t s, void (*k)(A...), dim3 g, dim3 b, typename Same<A>::type... a) {
+  void *p[] = {(void *)&a...};
+  return hipLaunchKernel((const void *)k, g, b, p, 0, s);
+}
+
 // waits for the case's work; its error flag, and with r the value *r in h->word
 int check_err(mge_case *h, const double *r = nullptr) {
   if (h->launch_err != hipSuccess) {
@@ -358,10 +370,7 @@ int check_err(mge_case *h, const double *r = nullptr) {
     h->launch_err = hipSuccess;
     return set_err(MGE_ERR_HIP, b);
   }
-  // the launch's own status: the thread's last error may be another caller's
-  const int *ep = h->err;
-  void *p[3] = {(void *)&r, (void *)&ep, (void *)&h->word};
-  if (hipLaunchKernel((const void *)&k_publish, dim3(1), dim3(64), p, 0, h->stream) != hipSuccess)
+  if (launch_on(h->stream, k_publish, dim3(1), dim3(64), r, h->err, h->word) != hipSuccess)
     return set_err(MGE_ERR_HIP, "error-flag read failed");
   if (hipStreamSynchronize(h->stream) != hipSuccess) return set_err(MGE_ERR_HIP, "stream sync failed");
   const int e = h->word->err;
@@ -1256,9 +1265,8 @@ int ffreeze_test(mge_case *h, int mlvl, int ncyc) {
   if (!(h->prm.ffreeze > 0.0 || h->prm.lfreeze > 0.0) || mlvl != h->nlevel || h->rec) return MGE_OK;
   Level &B = h->lv[mlvl];
   const int c = ncyc >= 1 && ncyc <= B.mxcyc ? ncyc : 0;
-  hipLaunchKernelGGL(k_ffreeze, dim3(1), dim3(64), 0, h->stream, (const double *)(B.rtrms + c), h->ffini, ncyc,
-                     h->prm.ffreeze, h->prm.lfreeze, h->ffrozen);
-  HIPCHK(hipGetLastError());
+  HIPCHK(launch_on(h->stream, k_ffreeze, dim3(1), dim3(64), B.rtrms + c, h->ffini, ncyc, h->prm.ffreeze,
+                   h->prm.lfreeze, h->ffrozen));
   return MGE_OK;
 }
 
@@ -2688,8 +2696,7 @@ int do_upload_solut(mge_case *h, Level &L, double ptot, double *host, int nval) 
   HIPCHK(hipMallocAsync((void **)&dev, sizeof(double) * nval * nc, h->stream));
   SolutArgs<T> A{L.d, stc<T>(L, L.cur), make_inf<T>(h->prm), h->prm.gamma, h->prm.p0,
                  freestream_mach(h->prm), ptot, nval == 11, nc, dev};
-  hipLaunchKernelGGL(k_upload_solut<T>, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, h->stream, A);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_on(h->stream, k_upload_solut<T>, dim3((unsigned)((nc + 255) / 256)), dim3(256), A);
   if (e == hipSuccess)
     e = xfer(h->dev, h->stream, dev, sizeof(double) * nval * nc, false,
              [&](size_t o, const char *t, size_t len) { std::memcpy((char *)host + o, t, len); }, host);
@@ -2714,8 +2721,7 @@ int do_upload_solut_noalloc(mge_case *h, Level &L, double ptot, double *host, in
                    freestream_mach(h->prm), ptot, nval == 11, ncc, h->scratch};
     A.c0 = c0;
     A.ostride = ncc;
-    hipLaunchKernelGGL(k_upload_solut<T>, dim3((unsigned)((ncc + 255) / 256)), dim3(256), 0, h->stream, A);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_on(h->stream, k_upload_solut<T>, dim3((unsigned)((ncc + 255) / 256)), dim3(256), A);
     for (int f = 0; f < nval && e == hipSuccess; f++)
       e = hipMemcpyAsync(host + (long)f * nc + c0, h->scratch + (long)f * ncc, sizeof(double) * ncc,
                          hipMemcpyDeviceToHost, h->stream);
