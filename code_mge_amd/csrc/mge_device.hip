@@ -1902,8 +1902,8 @@ int batch_build(mge_batch *b) {
   const size_t np = R[0].size();
   for (int i = 1; i < nc; i++)
     if (R[i].size() != np) return set_err(MGE_ERR_STATE, "cases of a batch must follow the same cycle");
-  // per position, the cases grouped by entry point (cases whose line
-  // lengths pick different scan widths launch different kernels there)
+  // per position, the cases grouped by entry point and block (cases whose
+  // line lengths or forced shapes pick other kernels launch them there)
   struct Group {
     size_t p;
     std::vector<int> cases;
