@@ -585,7 +585,7 @@ __device__ __attribute__((always_inline)) inline void k_smooth_xy_body(const Smo
       }
       if constexpr (SCAN) {
         const bool ok[1] = {i < nx};
-        constexpr int KR = 2;   // rows scanned together (24^3 .. 48^3 in a batch 25 us; all eight 35 us)
+        constexpr int KR = 2;   // rows scanned together (planes of 12^2 to 48^2 in a batch: 25 us; all eight 35 us)
 #pragma unroll
         for (int g = 0; g < U; g += KR) {
           if (t0 - sub + g * NW * RW >= ny) break;   // rows past the plane (uniform in the wave)
